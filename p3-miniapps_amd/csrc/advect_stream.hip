@@ -22,6 +22,12 @@
 // beyond one cell, or y offset different from the workgroup's) is interpolated
 // by the direct 4^4 gather from C4 in global memory at the step it is opened
 // and takes no streamed contribution.
+//
+// The vy = 0 slab has feet of both y offsets (they follow the sign of Ey), so
+// it is streamed by two workgroups per vx tile, one for each offset; each
+// writes its own feet.  With one workgroup, half of the slab took the gather,
+// whose 64 dependent row loads per step made these few workgroups the tail of
+// the launch: 140 us of a 16^4 advection, 1.01 ms at 64^4 (FP64).
 #include "advect_common.hpp"
 
 #include <cstdlib>
@@ -96,6 +102,10 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
   long S1, S2, S3;
   int F0;
   int wave, nwave, lane;
+  // this slab is shared by two workgroups, one per y offset: 0 no, 1 this one
+  // has offset 0 and also the feet outside both patterns, 2 offset -1
+  int pair;
+  int keep;  // pair: bit c set when this workgroup writes the cell in slot c
   int force;  // bit 0: every lane reads rows per cell; bit 1: every foot by direct gather
   int cbase;  // C4 element of (x -2, y -3, vx tile-2, vy ivy-2)
   double cx[3];          // x Lagrange weights of the half-step foot
@@ -190,6 +200,7 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
     OpenCell<A> &c = cell[R];
     c.acc = 0;
     c.kbit = 0;
+    if (pair) keep &= ~(1 << R);
     if (q >= N1) {
       // no cell: zero x-weights make its share of a common pass zero
 #pragma unroll
@@ -251,8 +262,20 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
       bspline_eta<A>((A)(fj - fl), c.w[j]);
     }
     const int ox = ip[0] - ix, oy = ip[1] - q, ovx = ip[2] - ivx, ovy = ip[3] - ivy;
-    const bool fast = ok & ((unsigned)(ox + 1) < 2u) & (oy == oyw) & ((unsigned)(ovx + 1) < 2u) &
-                      ((unsigned)(ovy + 1) < 2u) & !(force & 2);
+    const bool near = ok & ((unsigned)(ox + 1) < 2u) & ((unsigned)(ovx + 1) < 2u) & ((unsigned)(ovy + 1) < 2u) &
+                      !(force & 2);
+    const bool fast = near & (oy == oyw);
+    if (pair) {
+      // the other workgroup's foot: nothing to do here
+      const bool own = pair == 2 ? fast : !(near & (oy == -1));
+      keep |= own ? 1 << R : 0;
+      if (!own) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) c.w[0][k] = 0;
+        bad |= pair == 1 && !ok;
+        return;
+      }
+    }
     c.kbit = fast ? 1 << ((ox + 1) | ((ovx + 1) << 1) | ((ovy + 1) << 2)) : 0;
     // out of domain: the reference stops with "Time step is too large"
     bad |= !ok;
@@ -356,6 +379,7 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
     // the distinct keys of the open cells as bits: one key (or none) when
     // at most one bit is set
     const int m = cell[0].kbit | cell[1].kbit | cell[2].kbit | cell[3].kbit;
+    if (pair && __builtin_amdgcn_ballot_w64(m != 0) == 0) return;  // nothing of this offset here
     const bool same = ((m & (m - 1)) == 0) & !(force & 1);
     A t[4];
     if (__builtin_amdgcn_ballot_w64(!same) == 0) {
@@ -403,6 +427,7 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
     const int y = q - 3;
     if (y < 0 || y >= N1) return;
     const A v = cell[(R + 1) & 3].acc;
+    if (pair && !((keep >> ((R + 1) & 3)) & 1)) return;
     fbase[(long)N0 * y] = (T)v;
   }
 
@@ -427,7 +452,8 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
     if (NB == 3) {
       if (q + 2 < nsteps) n = fetch(q + 2, b == 0 ? 2 : b - 1);
     } else {
-      n = (wave_has_cells && q >= 3 && q - 3 < N1) ? 1 : 0;
+      // (a shared slab's store may have been skipped: wait for everything)
+      n = (wave_has_cells && !pair && q >= 3 && q - 3 < N1) ? 1 : 0;
     }
     wait_vm(n);
     __builtin_amdgcn_s_barrier();
@@ -441,12 +467,11 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
 // vx tiles [x ntile/8, (x+1) ntile/8) for every vy, vy slower and tile
 // faster, so that the workgroups resident on one XCD at a time cover a
 // compact block of (tile, vy) and share their rows through its L2, while
-// every XCD gets its share of each vy (the vy = 0 row, whose feet mostly take
-// the direct gather, is the slowest).  Without remap (or when the tiles do
+// every XCD gets its share of each vy.  Without remap (or when the tiles do
 // not split over the XCDs) block b is (b mod ntile, b / ntile).
-__device__ __forceinline__ void ys_block_tile(int b, int grid, int ntile, int N3, int remap, int &tile, int &ivy) {
+__device__ __forceinline__ void ys_block_tile(int b, int ntile, int remap, int &tile, int &ivy) {
   constexpr int NX = 8;
-  if (remap && ntile % NX == 0 && grid == ntile * N3) {
+  if (remap && ntile % NX == 0) {
     const int x = b % NX, k = b / NX;
     const int tx = ntile / NX;  // tiles per XCD
     ivy = k / tx;
@@ -463,7 +488,7 @@ template <typename T, typename A, int TVX, int NB, int RXC>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(A) == 4 ? 3 : 1)))
 void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geom g,
                                                      FeetConsts fc, double dt, T *__restrict__ fout,
-                                                     int *__restrict__ err, int force, int remap) {
+                                                     int *__restrict__ err, int force, int remap, int iv0) {
   extern __shared__ __align__(16) unsigned char ys_smem[];
   YStream<T, A, TVX, NB, RXC> s;
   s.force = force;
@@ -503,7 +528,18 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
   s.nsteps = s.N1 + 3;
   const int ntile = s.N2 / TVX;
   int tile, ivy;
-  ys_block_tile(blockIdx.x, gridDim.x, ntile, s.N3, remap, tile, ivy);
+  ys_block_tile(blockIdx.x, ntile, remap, tile, ivy);
+  // slab N3 (launched when iv0 >= 0): the second workgroups of slab iv0
+  s.pair = 0;
+  if (iv0 >= 0) {
+    if (ivy == s.N3) {
+      ivy = iv0;
+      s.pair = 2;
+    } else if (ivy == iv0) {
+      s.pair = 1;
+    }
+  }
+  s.keep = 0;
   s.ivy = ivy;
   {  // the y part of computeFeet for every cell y of this vy (VMO/Advection.hpp:174-196)
     const double vyw = g.minPhy[3] + ivy * g.dx[3];
@@ -529,7 +565,7 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
   s.x = g.minPhy[0] + s.ix * g.dx[0];
   s.vx = g.minPhy[2] + s.ivx * g.dx[2];
   s.vy = g.minPhy[3] + s.ivy * g.dx[3];
-  s.oyw = s.vy > 0. ? -1 : 0;
+  s.oyw = s.pair ? s.pair == 2 ? -1 : 0 : s.vy > 0. ? -1 : 0;
   s.fbase = fout + s.ix + (long)s.N0 * s.N1 * (s.ivx + (long)s.N2 * s.ivy);
   {
     const C4Pitch cp = c4_pitch(s.N0, s.N1, s.N2);
@@ -657,13 +693,25 @@ void launch_ys_t(const Geom &g, const YsPlan &p, const T *c4, const double *exy,
                  hipStream_t s) {
   const void *fn = (const void *)k_advect4d_ys<T, A, TVX, NB, RXC>;
   if (p.lds > 64 * 1024) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds);
-  const unsigned grid = (unsigned)((g.n[2] / TVX) * g.n[3]);
+  // the slab whose velocity vanishes (to rounding), if there is one: its
+  // drift dt vy / dy is below that of any field.  It is shared by two sets
+  // of workgroups as long as the launch is short enough for its tail to show:
+  // 48^4 gradient 29.2 -> 26.3 ms, 64^4 two-stream 30.8 -> 27.4 ms for 20
+  // steps, but 96^4 float storage (4608 workgroups) 187.8 -> 191.0 ms and
+  // 128^4 (8192) 215.1 -> 216.6 ms, the gathering workgroups being hidden
+  // there by the others.
+  int iv0 = -1;
+  if ((long)(g.n[2] / TVX) * g.n[3] < 4096) {
+    const double r = -g.minPhy[3] * g.inv_dx[3];
+    if (r > -0.5 && r < g.n[3] - 0.5 && std::fabs(r - std::nearbyint(r)) < 1e-6) iv0 = (int)std::nearbyint(r);
+  }
+  const unsigned grid = (unsigned)((g.n[2] / TVX) * (g.n[3] + (iv0 >= 0)));
   int force = 0;  // test switch: VLP4D_YS_FORCE=1 rows per cell, 2 direct gather, 3 both
   if (const char *e = getenv("VLP4D_YS_FORCE")) force = atoi(e) & 3;
   int remap = 1;  // VLP4D_YS_REMAP=0: block b -> (b mod ntile, b / ntile)
   if (const char *e = getenv("VLP4D_YS_REMAP")) remap = atoi(e) != 0;
   hipLaunchKernelGGL((k_advect4d_ys<T, A, TVX, NB, RXC>), dim3(grid), dim3(p.block), p.lds, s, c4, exy, g,
-                     feet_consts(g), dt, fout, err, force, remap);
+                     feet_consts(g), dt, fout, err, force, remap, iv0);
 }
 
 template <typename T, typename A, int TVX>

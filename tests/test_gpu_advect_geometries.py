@@ -1,0 +1,49 @@
+"""The 4-D advection over the geometries its dispatch distinguishes, against
+the oracle.
+
+The tolerance is that of the whole-step parity tests: a step sums 256 products
+of weights (positive, sum 1) per cell and solves four lines, so two steps
+differ from the oracle by some hundred roundings of the result's magnitude,
+1e-14; 1e-12 is asserted, as elsewhere.
+"""
+import math
+
+import numpy as np
+import pytest
+
+from conftest import relmax, sld_box
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(vlp, orc, n, steps=2, vmax=6.0, alpha=0.4):
+    """Steps of a strongly perturbed f (both signs of Ex and Ey everywhere)
+    from the library and the oracle."""
+    lx = 4 * math.pi
+    dt = 0.5 * (lx / max(n[0], n[1])) / vmax
+    args = sld_box(n, vmax=vmax, dt=dt, nbiter=steps, idcase=10, lx=lx)
+    cfg = vlp.VlpConfig.make(*args)
+    x = np.arange(n[0]) * cfg.dx[0]
+    y = np.arange(n[1]) * cfg.dx[1]
+    vx = cfg.minPhy[2] + np.arange(n[2]) * cfg.dx[2]
+    vy = cfg.minPhy[3] + np.arange(n[3]) * cfg.dx[3]
+    sp = 1 + alpha * np.cos(0.5 * x + 0.3)[None, :] + alpha * np.sin(0.5 * y + 0.2)[:, None]
+    f0 = (np.exp(-0.5 * (vx[None, :] ** 2 + vy[:, None] ** 2)) / (2 * math.pi))[:, :, None, None] * sp[None, None]
+    st = orc.State(orc.make_config(*args))
+    st.set_f(f0)
+    st.step(steps)
+    ref, nrj = st.f_interior(), st.diags()["nrj"][1:]
+    st.close()
+    with vlp.Vlp4d(cfg) as sim:
+        sim.set_f(f0)
+        sim.step(steps)
+        return relmax(sim.get_f(), ref), relmax(sim.diags()["nrj"][1:], nrj)
+
+
+# A vy = 0 slab (even Nvy), whose feet have both y offsets and which two
+# workgroups share: one and two vx tiles per wave, 8 tiles (XCD order), the
+# smallest grid; odd Nvy has no such slab.
+@pytest.mark.parametrize("n", [(16, 10, 10, 10), (16, 16, 16, 16), (32, 21, 16, 12), (64, 13, 12, 14), (32, 12, 14, 11)])
+def test_slab_of_both_y_offsets(vlp, orc, n):
+    ef, en = _run(vlp, orc, n)
+    assert ef < 1e-12 and en < 1e-12
