@@ -37,18 +37,15 @@ namespace vlp {
 namespace {
 
 // One open cell: B-spline weights along x, y, vx, vy ([dim][k]), running
-// sum, and the packed stencil offsets (ox+1) | (ovx+1) << 1 | (ovy+1) << 2,
-// or -1 when the cell takes no streamed contribution (with the same key as
-// a bit, so that the four cells' keys compare by two bit operations).  (Keeping the four y
-// weights rather than re-evaluating the one a plane needs from the
-// fractional y position measured 1 % faster with double arithmetic, at 246
-// registers.)
+// sum, and the LDS element of its first stencil row in a plane's slab.  A
+// cell without a streamed contribution has zero x-weights and the row of the
+// cell opened before it.  (Keeping the four y weights rather than
+// re-evaluating the one a plane needs from the fractional y position measured
+// 1 % faster with double arithmetic.)
 template <typename A> struct OpenCell {
   A w[4][4];
   A acc;
-  // 1 << key (key = (ox + 1) | (ovx + 1) << 1 | (ovy + 1) << 2, the stencil
-  // offsets of a streamed foot), or 0 without a streamed contribution
-  int kbit;
+  int row;
 };
 
 typedef __attribute__((address_space(3))) void lds_void;
@@ -67,13 +64,13 @@ typedef __attribute__((address_space(3))) void lds_void;
 // computeFeet's 3x3 Lagrange interpolation of E at the half-step position
 // (x - dt/2 vx, y - dt/2 vy) separates: the x part (base column ip0 and
 // weights cx) depends on the lane's (x, vx) only, the y part (row ip1 and
-// weights cy) on (y, vy), which is uniform in the workgroup at a step.  A lane
-// therefore keeps G[k1] = sum_k0 cx[k0] E(ip0+k0, ip1+k1) for the three rows
-// and, as ip1 advances by one per step, computes only the new row.
+// weights cy) on (y, vy), which is uniform in the workgroup at a step.  As ip1
+// advances by one per step, a lane reads one new row per step,
+// g = sum_k0 cx[k0] E(ip0+k0, ip1+2), and adds it to the sums of the three
+// cells it belongs to: it completes cell q's, is the second term of cell
+// q+1's and the first of cell q+2's.
 template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
   static constexpr int VPL = 16 / (int)sizeof(T);  // slab values per lane load
-  // double arithmetic reads the foot constants from LDS (see open())
-  static constexpr bool KLDS = sizeof(A) == sizeof(double);
   static constexpr int MS = 8;  // slab DMA instructions per wave per plane, at most
   const T *__restrict__ c4;
   const double *__restrict__ exy;  // (Ex, Ey) pairs, [N1][N0]
@@ -81,24 +78,23 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
   T *slab;         // NB buffers of slab_bytes
   double *eb;      // [NB][3][EPR][2]
   double *kconst;  // LDS: domain constants of the foot computation (KC_* layout)
-  // LDS: per y-step values uniform in the workgroup, [q][QT]: the y of cell
-  // q, computeFeet's E row ip1 (as a double) and its three y Lagrange weights
+  // LDS: per y-step values uniform in the workgroup, rows q = -2 .. N1-1 of
+  // QT: computeFeet's E row ip1 of cell q (as a double), and the y Lagrange
+  // weights of the row that is new at step q: cy[2] of cell q, cy[1] of cell
+  // q+1, cy[0] of cell q+2
   double *qtab;
-  static constexpr int QT = 5;
+  static constexpr int QT = 4;
   T *fbase;  // f^{n+1} at (x, y = 0, vx, vy) of this lane
-  static constexpr int KC_MIN = 0, KC_INV = 4, KC_LMIN = 8, KC_LMAX = 12, KC_VHI = 16, KC_N = 18;
+  static constexpr int KC_MIN = 0, KC_INV = 4, KC_LMIN = 8, KC_LMAX = 12, KC_VHI = 16, KC_DX = 18, KC_DT = 22, KC_N = 24;
   int slab_bytes;  // whole 1 KB blocks
   int EPR, cpr;    // E points per LDS row (whole 64-point chunks), chunks per row
   unsigned voff[MS];  // C4 byte offset of this lane's chunk in the wave's k-th slab DMA
   int nslot;       // slab DMA instructions of this wave (wave-uniform)
-  Geom g;
-  FeetConsts fc;
-  double dt;
   int N0, N1, N2, N3, RX, nsteps, oyw;
   int ix, tv, ivx, ivy;
+  int row0;  // LDS element of the stencil row of a foot with offset 0 along x, vx, vy
   bool active;
   bool wave_has_cells;  // some lane of this wave owns cells (wave-uniform)
-  double x, vx, vy;
   long S1, S2, S3;
   int F0;
   int wave, nwave, lane;
@@ -110,7 +106,14 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
   int cbase;  // C4 element of (x -2, y -3, vx tile-2, vy ivy-2)
   double cx[3];          // x Lagrange weights of the half-step foot
   int jx[3];             // wrapped E columns ip0 .. ip0+2
-  double gx[3], gy[3];   // x-interpolated E of rows ip1 .. ip1+2
+  double s1x, s1y, s2x, s2y;  // partial E of cells q+1 (two rows) and q+2 (one row)
+  // The foot in cells from the node: d = -dt (v - dt/2 E) / dx along x and y,
+  // -dt E / dv along vx and vy.  ax, ay1: its part without E (along y less
+  // the workgroup's offset, so that a streamed foot has 0 <= w < 1, except in
+  // a shared slab)
+  double ax, ay1;
+  double bex, bey, bvx, bvy;  // factors of E in the four directions
+  double lo2, lo3;            // lower bounds of the vx and vy displacement (the clamp at v_min)
   int ip1p;              // ip1 of the previous step (wave-uniform)
   OpenCell<A> cell[4];
   int bad;
@@ -118,7 +121,7 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
   // E row ip1 of the cell y (computeFeet: round of the half-step y) - 1;
   // uniform in the workgroup.
   __device__ __forceinline__ int erow0(int y) const {
-    return __builtin_amdgcn_readfirstlane((int)qtab[QT * y + 1]);
+    return __builtin_amdgcn_readfirstlane((int)qtab[QT * y]);
   }
 
   // Start moving step q's slab and E rows into LDS buffer b by LDS-DMA.
@@ -163,43 +166,48 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
     return n;
   }
 
-  // Per step, uniform in the workgroup: the y part of computeFeet for cell
-  // y = q, and the update of the lane's x-interpolated E rows (buffer b).
-  __device__ __forceinline__ void field_rows(int q, int b, double cy[3], double &yq) {
+  // E at the half-step foot of cell q (computeFeet, VMO/Advection.hpp:
+  // 174-206) from the E rows in buffer b.
+  __device__ __forceinline__ void field_at(int q, int b, double &efx, double &efy) {
     const double *t = qtab + QT * q;
-    yq = t[0];
-    const int ip1 = __builtin_amdgcn_readfirstlane((int)t[1]);
-    cy[0] = t[2];
-    cy[1] = t[3];
-    cy[2] = t[4];
+    const int ip1 = __builtin_amdgcn_readfirstlane((int)t[0]);
     const double2 *er = (const double2 *)(eb + b * 6 * EPR);
-    if (ip1 == ip1p + 1) {
-      gx[0] = gx[1];
-      gy[0] = gy[1];
-      gx[1] = gx[2];
-      gy[1] = gy[2];
-      const double2 e0 = er[2 * EPR + jx[0]], e1 = er[2 * EPR + jx[1]], e2 = er[2 * EPR + jx[2]];
-      gx[2] = cx[0] * e0.x + cx[1] * e1.x + cx[2] * e2.x;
-      gy[2] = cx[0] * e0.y + cx[1] * e1.y + cx[2] * e2.y;
-    } else {
+    if (ip1 != ip1p + 1) {  // the first cell (or a rounding tie of the row): its rows 0 and 1
+      const double c0 = t[3 - 2 * QT], c1 = t[2 - QT], d0 = t[3 - QT];
+      double gx[2], gy[2];
 #pragma unroll
-      for (int k1 = 0; k1 < 3; k1++) {
+      for (int k1 = 0; k1 < 2; k1++) {
         const double2 e0 = er[k1 * EPR + jx[0]], e1 = er[k1 * EPR + jx[1]], e2 = er[k1 * EPR + jx[2]];
         gx[k1] = cx[0] * e0.x + cx[1] * e1.x + cx[2] * e2.x;
         gy[k1] = cx[0] * e0.y + cx[1] * e1.y + cx[2] * e2.y;
       }
+      s1x = c0 * gx[0] + c1 * gx[1];
+      s1y = c0 * gy[0] + c1 * gy[1];
+      s2x = d0 * gx[1];
+      s2y = d0 * gy[1];
     }
     ip1p = ip1;
+    const double2 e0 = er[2 * EPR + jx[0]], e1 = er[2 * EPR + jx[1]], e2 = er[2 * EPR + jx[2]];
+    const double gx = cx[0] * e0.x + cx[1] * e1.x + cx[2] * e2.x;
+    const double gy = cx[0] * e0.y + cx[1] * e1.y + cx[2] * e2.y;
+    efx = s1x + t[1] * gx;
+    efy = s1y + t[1] * gy;
+    s1x = s2x + t[2] * gx;
+    s1y = s2y + t[2] * gy;
+    s2x = t[3] * gx;
+    s2y = t[3] * gy;
   }
 
-  // Open cell y = q in slot R: the rest of computeFeet (VMO/Advection.hpp:
-  // 166-218), the bound check, B-spline weights and stencil offsets.  A cell
-  // that takes no streamed contribution gets no key bit and zero x-weights,
-  // so that a common pass adds nothing to it.
-  template <int R> __device__ __forceinline__ void open(int q, double yq, const double cy[3]) {
+  // Open cell y = q in slot R with the field at its half-step foot: the
+  // displacement, B-spline weights and stencil row.  The displacement is
+  // formed in cells from the node, which needs no position, division or
+  // floor: the fraction is that of the displacement and the stencil offset its
+  // sign, for |displacement| < 1 (other feet take open_direct, the reference's
+  // sequence).
+  template <int R> __device__ __forceinline__ void open(int q, double efx, double efy) {
     OpenCell<A> &c = cell[R];
     c.acc = 0;
-    c.kbit = 0;
+    c.row = cell[(R + 3) & 3].row;
     if (pair) keep &= ~(1 << R);
     if (q >= N1) {
       // no cell: zero x-weights make its share of a common pass zero
@@ -207,102 +215,92 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
       for (int k = 0; k < 4; k++) c.w[0][k] = 0;
       return;
     }
-    // with double arithmetic the domain constants come from LDS (ds_read,
-    // wave-uniform address) at each open rather than living in scalar
-    // registers for the whole loop, where they would be spilled; float
-    // arithmetic (vector registers held to three waves per SIMD) keeps them
-    // in scalar registers
-    double minp[4], invd[4], lmin[4], lmax[4], vhi[2];
-    if constexpr (KLDS) {
-      const double *kc = kconst;
-      asm volatile("" : "+s"(kc));
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        minp[j] = kc[KC_MIN + j];
-        invd[j] = kc[KC_INV + j];
-        lmin[j] = kc[KC_LMIN + j];
-        lmax[j] = kc[KC_LMAX + j];
+    const double d0 = ax + bex * efx;
+    double w1 = ay1 + bey * efy;
+    // the velocity clamp at v_min binds for the first plane only (a foot
+    // beyond v_max is one cell or more away and not taken here)
+    const double d2 = fmax(bvx * efx, lo2), d3 = fmax(bvy * efy, lo3);
+    // all comparisons fail for a NaN (of Ex in d0, of Ey in w1)
+    const bool near = (fabs(d0) < 1.) & (fabs(d2) < 1.) & (fabs(d3) < 1.) & !(force & 2);
+    bool in = (w1 >= 0.) & (w1 < 1.);
+    bool other = false;  // in a shared slab: the other workgroup's foot
+    if (pair) {          // there w1 is the displacement itself, so that the two workgroups split the feet exactly
+      const bool neg = (w1 >= -1.) & (w1 < 0.);
+      if (pair == 2) {
+        in = neg;
+        w1 += 1.;
+        other = true;
+      } else {
+        other = near & neg;
       }
-      vhi[0] = kc[KC_VHI];
-      vhi[1] = kc[KC_VHI + 1];
+    }
+    const bool fast = near & in;
+    bspline_eta<A>((A)__builtin_amdgcn_fract(d0), c.w[0]);
+    bspline_eta<A>((A)w1, c.w[1]);
+    bspline_eta<A>((A)__builtin_amdgcn_fract(d2), c.w[2]);
+    bspline_eta<A>((A)__builtin_amdgcn_fract(d3), c.w[3]);
+    const int rx = RXC ? RXC : RX;
+    const int row = row0 + (d0 < 0. ? -1 : 0) + (d2 < 0. ? -rx : 0) + (d3 < 0. ? -(TVX + 4) * rx : 0);
+    if (pair) keep |= fast ? 1 << R : 0;
+    if (__builtin_amdgcn_ballot_w64(!fast) == 0) {
+      c.row = row;
     } else {
+      if (fast) {
+        c.row = row;
+      } else {
+        if (!other) open_direct(q, efx, efy, c);
+        if (pair) keep |= other ? 0 : 1 << R;
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        minp[j] = g.minPhy[j];
-        invd[j] = g.inv_dx[j];
-        lmin[j] = fc.locmin[j];
-        lmax[j] = fc.locmax[j];
-      }
-      vhi[0] = g.minPhy[2] + fc.rxwidth[2];
-      vhi[1] = g.minPhy[3] + fc.rxwidth[3];
-    }
-    const double ftmp1 = cy[0] * gx[0] + cy[1] * gx[1] + cy[2] * gx[2];
-    const double ftmp2 = cy[0] * gy[0] + cy[1] * gy[1] + cy[2] * gy[2];
-    const double xt2 = vx - 0.5 * dt * ftmp1;
-    const double xt3 = vy - 0.5 * dt * ftmp2;
-    double xs[4];
-    xs[0] = x - dt * xt2;
-    xs[1] = yq - dt * xt3;
-    // the velocity clamp max(min(v*, vmax), vmin) as v_min / v_max: they
-    // differ from the comparisons only for a NaN v*, which makes x* NaN
-    // too, so the bound check below still fails
-    xs[2] = fmax(fmin(vx - dt * ftmp1, vhi[0]), minp[2]);
-    xs[3] = fmax(fmin(vy - dt * ftmp2, vhi[1]), minp[3]);
-    // all eight comparisons, no short cut (NaN fails them)
-    bool ok = true;
-#pragma unroll
-    for (int j = 0; j < 4; j++) ok = ok & (xs[j] >= lmin[j]) & (xs[j] <= lmax[j]);
-    int ip[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const double fj = invd[j] * (xs[j] - minp[j]);
-      const double fl = floor(fj);
-      ip[j] = ok ? (int)fl : 0;
-      // fj - floor(fj) is fj - ip exactly wherever the foot is valid
-      bspline_eta<A>((A)(fj - fl), c.w[j]);
-    }
-    const int ox = ip[0] - ix, oy = ip[1] - q, ovx = ip[2] - ivx, ovy = ip[3] - ivy;
-    const bool near = ok & ((unsigned)(ox + 1) < 2u) & ((unsigned)(ovx + 1) < 2u) & ((unsigned)(ovy + 1) < 2u) &
-                      !(force & 2);
-    const bool fast = near & (oy == oyw);
-    if (pair) {
-      // the other workgroup's foot: nothing to do here
-      const bool own = pair == 2 ? fast : !(near & (oy == -1));
-      keep |= own ? 1 << R : 0;
-      if (!own) {
-#pragma unroll
-        for (int k = 0; k < 4; k++) c.w[0][k] = 0;
-        bad |= pair == 1 && !ok;
-        return;
+        for (int k = 0; k < 4; k++) c.w[0][k] = 0;  // no share of a common pass
       }
     }
-    c.kbit = fast ? 1 << ((ox + 1) | ((ovx + 1) << 1) | ((ovy + 1) << 2)) : 0;
-    // out of domain: the reference stops with "Time step is too large"
-    bad |= !ok;
-    if (ok & !fast) {
-      // a foot outside the streamed pattern: direct gather.  A copy keeps the
-      // slot's weights out of the callee's reach (the per-lane state then
-      // stays in registers).
-      A e[4][4];
+    if (q == 0) {  // the slots still empty agree with the first cell
 #pragma unroll
-      for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int k = 0; k < 4; k++) e[j][k] = c.w[j][k];
-      // the C4 strides are rebuilt here, on this rare path, rather than
-      // kept in scalar registers across the loop
-      int n0 = N0, n1 = N1, n2 = N2;
-      asm volatile("" : "+s"(n0), "+s"(n1), "+s"(n2));
-      const C4Pitch cp = c4_pitch(n0, n1, n2);
-      c.acc = gather4d<T, A>(c4, cp.s1, cp.s2, cp.s3, ip, e);
-#pragma unroll
-      for (int k = 0; k < 4; k++) c.w[0][k] = 0;  // no share of a common pass
+      for (int k = 1; k < 4; k++) cell[(R + k) & 3].row = c.row;
     }
   }
 
-  // LDS element of the first value of row (kvx = 0, kvy = 0) for a key.
-  __device__ __forceinline__ int row_base(int key) const {
-    const int ox = (key & 1) - 1, ovx = ((key >> 1) & 1) - 1, ovy = ((key >> 2) & 1) - 1;
-    return (tv + 1 + ovx) * RX + (1 + ovy) * (TVX + 4) * RX + ix + 1 + ox;
+  // A foot outside the streamed pattern: computeFeet's own sequence
+  // (VMO/Advection.hpp:208-217), the bound check and the direct 4^4 gather.
+  // Its constants come from LDS and the C4 strides are rebuilt here, so that
+  // this rare path keeps nothing in scalar registers across the loop.
+  __device__ __forceinline__ void open_direct(int q, double ftmp1, double ftmp2, OpenCell<A> &c) {
+    const double *kc = kconst;
+    asm volatile("" : "+s"(kc));
+    const double x = kc[KC_MIN] + ix * kc[KC_DX], yq = kc[KC_MIN + 1] + q * kc[KC_DX + 1];
+    const double vx = kc[KC_MIN + 2] + ivx * kc[KC_DX + 2], vy = kc[KC_MIN + 3] + ivy * kc[KC_DX + 3];
+    const double dtl = kc[KC_DT];
+    const double xt2 = vx - 0.5 * dtl * ftmp1;
+    const double xt3 = vy - 0.5 * dtl * ftmp2;
+    double xs[4];
+    xs[0] = x - dtl * xt2;
+    xs[1] = yq - dtl * xt3;
+    // the velocity clamp max(min(v*, vmax), vmin) as v_min / v_max: they
+    // differ from the comparisons only for a NaN v*, which makes x* NaN
+    // too, so the bound check below still fails
+    xs[2] = fmax(fmin(vx - dtl * ftmp1, kc[KC_VHI]), kc[KC_MIN + 2]);
+    xs[3] = fmax(fmin(vy - dtl * ftmp2, kc[KC_VHI + 1]), kc[KC_MIN + 3]);
+    // all eight comparisons, no short cut (NaN fails them)
+    bool ok = true;
+#pragma unroll
+    for (int j = 0; j < 4; j++) ok = ok & (xs[j] >= kc[KC_LMIN + j]) & (xs[j] <= kc[KC_LMAX + j]);
+    // out of domain: the reference stops with "Time step is too large"
+    bad |= !ok;
+    if (!ok) return;
+    int ip[4];
+    // (the weights go to the cell's registers: other lanes of the wave keep
+    // theirs there, so this path adds none)
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const double fj = kc[KC_INV + j] * (xs[j] - kc[KC_MIN + j]);
+      const double fl = floor(fj);
+      ip[j] = (int)fl;
+      bspline_eta<A>((A)(fj - fl), c.w[j]);
+    }
+    int n0 = N0, n1 = N1, n2 = N2;
+    asm volatile("" : "+s"(n0), "+s"(n1), "+s"(n2));
+    const C4Pitch cp = c4_pitch(n0, n1, n2);
+    c.acc = gather4d<T, A>(c4, cp.s1, cp.s2, cp.s3, ip, c.w);
   }
 
   // The plane's contribution t[c] to each of the four open cells from the 16
@@ -367,44 +365,38 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
 
   // Add plane q (LDS buffer b) to the four open cells; the cell opened at
   // step q - j sits in slot (R - j) & 3 and takes y-weight j.  When every
-  // lane's streamed cells agree on their stencil key (the usual case), one
-  // pass over the 16 rows of that key serves all four cells; cells without a
-  // streamed contribution have zero x-weights, so their share is zero.
-  // Otherwise one pass reads the rows of one key per lane (the first key
-  // among its cells still to do) and adds to the cells with that key; the
-  // wave repeats until no lane has cells left.  force & 1 takes the second
+  // lane's cells agree on their first stencil row (the usual case), one pass
+  // over the 16 rows serves all four cells; cells without a streamed
+  // contribution have zero x-weights, so their share is zero.  Otherwise one
+  // pass reads the rows of one cell per lane (the first still to do) and adds
+  // to the cells with the same rows; the wave repeats until no lane has cells
+  // left.  force & 1 takes the second
   // form with one cell per pass.
   template <int R> __device__ __forceinline__ void accumulate(int b) {
     const T *s = (const T *)((const char *)slab + b * slab_bytes);
-    // the distinct keys of the open cells as bits: one key (or none) when
-    // at most one bit is set
-    const int m = cell[0].kbit | cell[1].kbit | cell[2].kbit | cell[3].kbit;
-    if (pair && __builtin_amdgcn_ballot_w64(m != 0) == 0) return;  // nothing of this offset here
-    const bool same = ((m & (m - 1)) == 0) & !(force & 1);
+    const int r0 = cell[0].row;
+    const bool same = (r0 == cell[1].row) & (r0 == cell[2].row) & (r0 == cell[3].row) & !(force & 1);
     A t[4];
     if (__builtin_amdgcn_ballot_w64(!same) == 0) {
-      const int k0 = m ? __builtin_ctz(m) : 0;
-      pass_rows(s + row_base(k0), t);
+      pass_rows(s + r0, t);
       close_plane<R, 0>(t, 15u);
       close_plane<R, 1>(t, 15u);
       close_plane<R, 2>(t, 15u);
       close_plane<R, 3>(t, 15u);
       return;
     }
-    unsigned todo = 0;
-#pragma unroll
-    for (int c = 0; c < 4; c++) todo |= (cell[c].kbit ? 1u : 0u) << c;
+    unsigned todo = 15u;
     while (__builtin_amdgcn_ballot_w64(todo != 0)) {
-      int kp = 0;
+      int rp = r0;
 #pragma unroll
       for (int c = 3; c >= 0; c--)
-        if ((todo >> c) & 1) kp = cell[c].kbit;
+        if ((todo >> c) & 1) rp = cell[c].row;
       unsigned sel = 0;
 #pragma unroll
       for (int c = 0; c < 4; c++)
-        if (((todo >> c) & 1) && cell[c].kbit == kp && !((force & 1) && sel)) sel |= 1u << c;
+        if (((todo >> c) & 1) && cell[c].row == rp && !((force & 1) && sel)) sel |= 1u << c;
       todo &= ~sel;
-      pass_rows(s + row_base(kp ? __builtin_ctz(kp) : 0), t);
+      pass_rows(s + rp, t);
       close_plane<R, 0>(t, sel);
       close_plane<R, 1>(t, sel);
       close_plane<R, 2>(t, sel);
@@ -442,9 +434,9 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
   template <int R> __device__ __forceinline__ void step(int q, int b) {
     if (NB == 2 && q + 1 < nsteps) fetch(q + 1, b ^ 1);
     if (active) {
-      double cy[3] = {0., 0., 0.}, yq = 0.;
-      if (q < N1) field_rows(q, b, cy, yq);  // no cell opens beyond the last y
-      open<R>(q, yq, cy);
+      double efx = 0., efy = 0.;
+      if (q < N1) field_at(q, b, efx, efy);  // no cell opens beyond the last y
+      open<R>(q, efx, efy);
       accumulate<R>(b);
       close<R>(q);
     }
@@ -495,9 +487,6 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
   s.c4 = c4;
   s.exy = exy;
   s.fout = fout;
-  s.g = g;
-  s.fc = fc;
-  s.dt = dt;
   s.N0 = g.n[0];
   s.N1 = g.n[1];
   s.N2 = g.n[2];
@@ -512,7 +501,7 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
   s.slab = (T *)ys_smem;
   s.eb = (double *)(ys_smem + NB * (size_t)s.slab_bytes);
   s.kconst = s.eb + NB * 6 * s.EPR;
-  s.qtab = s.kconst + s.KC_N;
+  s.qtab = s.kconst + s.KC_N + 2 * s.QT;
   if (threadIdx.x == 0) {
     double *k = s.kconst;
 #pragma unroll
@@ -521,7 +510,9 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
       k[s.KC_INV + j] = g.inv_dx[j];
       k[s.KC_LMIN + j] = fc.locmin[j];
       k[s.KC_LMAX + j] = fc.locmax[j];
+      k[s.KC_DX + j] = g.dx[j];
     }
+    k[s.KC_DT] = dt;
     k[s.KC_VHI] = g.minPhy[2] + fc.rxwidth[2];
     k[s.KC_VHI + 1] = g.minPhy[3] + fc.rxwidth[3];
   }
@@ -549,11 +540,15 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
       const int ip1 = (int)(round(xt1) - 1);
       const double py = xt1 - ip1;
       double *t = s.qtab + s.QT * q;
-      t[0] = yq;
-      t[1] = (double)ip1;
-      t[2] = .5 * (py - 1.) * (py - 2.);
-      t[3] = -1. * (py) * (py - 2.);
-      t[4] = .5 * (py) * (py - 1.);
+      t[0] = (double)ip1;
+      t[1] = .5 * (py) * (py - 1.);
+      t[2 - s.QT] = -1. * (py) * (py - 2.);
+      t[3 - 2 * s.QT] = .5 * (py - 1.) * (py - 2.);
+    }
+    // past the last cell: weights of cells that do not exist
+    if (threadIdx.x == 0) {
+      double *t = s.qtab + s.QT * s.N1;
+      t[2 - s.QT] = t[3 - s.QT] = t[3 - 2 * s.QT] = 0.;
     }
   }
   __syncthreads();  // both tables are written before the first fetch reads them
@@ -562,10 +557,19 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
   s.ix = s.active ? tid % s.N0 : 0;
   s.tv = s.active ? tid / s.N0 : 0;
   s.ivx = tile * TVX + s.tv;
-  s.x = g.minPhy[0] + s.ix * g.dx[0];
-  s.vx = g.minPhy[2] + s.ivx * g.dx[2];
-  s.vy = g.minPhy[3] + s.ivy * g.dx[3];
-  s.oyw = s.pair ? s.pair == 2 ? -1 : 0 : s.vy > 0. ? -1 : 0;
+  const double x = g.minPhy[0] + s.ix * g.dx[0];
+  const double vx = g.minPhy[2] + s.ivx * g.dx[2];
+  const double vy = g.minPhy[3] + s.ivy * g.dx[3];
+  s.oyw = s.pair ? s.pair == 2 ? -1 : 0 : vy > 0. ? -1 : 0;
+  s.ax = -(dt * vx) * g.inv_dx[0];
+  s.ay1 = -(dt * vy) * g.inv_dx[1] - (s.pair ? 0 : s.oyw);
+  s.bex = 0.5 * dt * dt * g.inv_dx[0];
+  s.bey = 0.5 * dt * dt * g.inv_dx[1];
+  s.bvx = -dt * g.inv_dx[2];
+  s.bvy = -dt * g.inv_dx[3];
+  s.lo2 = s.ivx == 0 ? 0. : -2.;
+  s.lo3 = s.ivy == 0 ? 0. : -2.;
+  s.row0 = s.ix + 1 + (RXC ? RXC : s.RX) * (s.tv + 1 + (TVX + 4));
   s.fbase = fout + s.ix + (long)s.N0 * s.N1 * (s.ivx + (long)s.N2 * s.ivy);
   {
     const C4Pitch cp = c4_pitch(s.N0, s.N1, s.N2);
@@ -589,7 +593,7 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
     }
   }
   {  // x part of computeFeet's E interpolation (VMO/Advection.hpp:174-196)
-    double xt0 = s.x - 0.5 * dt * s.vx;
+    double xt0 = x - 0.5 * dt * vx;
     xt0 = g.inv_dx[0] * (xt0 - g.minPhy[0]);
     const int ip0 = (int)(round(xt0) - 1);
     const double px = xt0 - ip0;
@@ -604,7 +608,7 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
   s.cbase = (int)(1 + s.S2 * (tile * TVX + 1) + s.S3 * (s.ivy + 1));
 #pragma unroll
   for (int c = 0; c < 4; c++) {
-    s.cell[c].kbit = 0;
+    s.cell[c].row = s.row0;
     s.cell[c].acc = 0;
 #pragma unroll
     for (int j = 0; j < 4; j++)
@@ -677,7 +681,7 @@ YsPlan ys_plan(const Geom &g, size_t tsz, int want_tvx = 0, int want_nb = 0) {
     const long ninstr = ys_slab_instr(N0, tvx, tsz);
     if ((ninstr + block / 64 - 1) / (block / 64) > 8) continue;  // DMA slots per wave
     const size_t lds = nb * (size_t)ninstr * 1024 + nb * 3 * (size_t)ys_epr(N0) * 2 * sizeof(double) +
-                       (18 + 5 * (size_t)N1) * sizeof(double);  // domain constants, per-step table
+                       (24 + 4 * (size_t)(N1 + 2)) * sizeof(double);  // domain constants, per-step table
     if (lds > 160 * 1024) continue;
     p.tvx = tvx;
     p.nb = nb;

@@ -47,3 +47,12 @@ def _run(vlp, orc, n, steps=2, vmax=6.0, alpha=0.4):
 def test_slab_of_both_y_offsets(vlp, orc, n):
     ef, en = _run(vlp, orc, n)
     assert ef < 1e-12 and en < 1e-12
+
+
+# Velocity displacements dt E / dv on both sides of one cell: below it a foot
+# is streamed (with the clamp at the first velocity plane), beyond it the foot
+# takes the direct gather (with the clamp at both ends).
+@pytest.mark.parametrize("n,vmax", [((16, 10, 64, 64), 3.0), ((16, 16, 48, 20), 4.0), ((32, 12, 16, 90), 3.0)])
+def test_velocity_displacement_beyond_a_cell(vlp, orc, n, vmax):
+    ef, en = _run(vlp, orc, n, vmax=vmax)
+    assert ef < 1e-12 and en < 1e-12
