@@ -58,7 +58,12 @@ typedef __attribute__((address_space(3))) void lds_void;
 // fills LDS bytes [1024 j, 1024 j + 1024) of the buffer, lane l taking chunk
 // 64 j + l wherever it sits in C4; instructions are dealt to the waves in
 // turn, and each lane keeps the C4 byte offset (from the plane's first row)
-// of its chunk in every instruction of its wave.  E rows sit in LDS as
+// of its chunk in every instruction of its wave.  When the C4 rows are not
+// whole 16-byte chunks (N0 + 4 odd, or for float not a multiple of 4), a
+// plane's rows start shift(q) elements past a chunk boundary, the same for all
+// rows of the plane (the pitches past y are multiples of 16 elements): the
+// chunks are taken from the boundary and the slab pitch RX holds the
+// remainder.  E rows sit in LDS as
 // (Ex, Ey) pairs: [buffer][row k1 = 0..2][EPR], moved 64 points per instruction.
 //
 // computeFeet's 3x3 Lagrange interpolation of E at the half-step position
@@ -124,11 +129,15 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
     return __builtin_amdgcn_readfirstlane((int)qtab[QT * y]);
   }
 
+  // Elements by which plane q's rows sit past a 16-byte boundary (C4's base
+  // puts the rows of y = -2 on one).
+  __device__ __forceinline__ int shift(int q) const { return RXC ? 0 : (F0 * (q + oyw + 1)) & (VPL - 1); }
+
   // Start moving step q's slab and E rows into LDS buffer b by LDS-DMA.
   // Returns the number of DMA instructions this wave issued (wave-uniform).
   __device__ __forceinline__ int fetch(int q, int b) {
     const int p = q + oyw - 1;  // y-position of the plane
-    const char *src = (const char *)c4 + ((long)cbase + (long)F0 * (p + 3)) * (long)sizeof(T);
+    const char *src = (const char *)c4 + ((long)cbase + (long)F0 * (p + 3) - shift(q)) * (long)sizeof(T);
     // the slot bookkeeping is recomputed each step from these (a few scalar
     // operations) rather than kept live across the loop, where it would be
     // spilled from the scalar registers
@@ -372,8 +381,8 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
   // to the cells with the same rows; the wave repeats until no lane has cells
   // left.  force & 1 takes the second
   // form with one cell per pass.
-  template <int R> __device__ __forceinline__ void accumulate(int b) {
-    const T *s = (const T *)((const char *)slab + b * slab_bytes);
+  template <int R> __device__ __forceinline__ void accumulate(int q, int b) {
+    const T *s = (const T *)((const char *)slab + b * slab_bytes) + shift(q);
     const int r0 = cell[0].row;
     const bool same = (r0 == cell[1].row) & (r0 == cell[2].row) & (r0 == cell[3].row) & !(force & 1);
     A t[4];
@@ -437,7 +446,7 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
       double efx = 0., efy = 0.;
       if (q < N1) field_at(q, b, efx, efy);  // no cell opens beyond the last y
       open<R>(q, efx, efy);
-      accumulate<R>(b);
+      accumulate<R>(q, b);
       close<R>(q);
     }
     int n = 0;
@@ -451,6 +460,13 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
     __builtin_amdgcn_s_barrier();
   }
 };
+
+// 16-byte chunks of a slab row: the row's N0 + 4 values and, when they are not
+// whole chunks, the up to vpl - 1 values before them (see YStream).
+__host__ __device__ inline int ys_row_chunks(int N0, int vpl) {
+  const int n = N0 + 4;
+  return n % vpl ? (n + vpl - 1 + vpl - 1) / vpl : n / vpl;
+}
 
 // Workgroup -> (vx tile, vy).  Workgroups go to the 8 XCDs (each with its
 // own L2) round-robin: block b runs on XCD b mod 8, as the (b / 8)-th of
@@ -491,8 +507,8 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
   s.N1 = g.n[1];
   s.N2 = g.n[2];
   s.N3 = g.n[3];
-  s.RX = s.N0 + 4;
-  const int per_row = s.RX / s.VPL;                 // 16-byte chunks per slab row
+  const int per_row = ys_row_chunks(s.N0, s.VPL);  // 16-byte chunks per slab row
+  s.RX = per_row * s.VPL;
   const int nchunk = 5 * (TVX + 4) * per_row;
   const int ninstr = (nchunk + 63) >> 6;
   s.slab_bytes = ninstr * 1024;
@@ -517,7 +533,7 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
     k[s.KC_VHI + 1] = g.minPhy[3] + fc.rxwidth[3];
   }
   s.nsteps = s.N1 + 3;
-  const int ntile = s.N2 / TVX;
+  const int ntile = (s.N2 + TVX - 1) / TVX;
   int tile, ivy;
   ys_block_tile(blockIdx.x, ntile, remap, tile, ivy);
   // slab N3 (launched when iv0 >= 0): the second workgroups of slab iv0
@@ -553,7 +569,8 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
   }
   __syncthreads();  // both tables are written before the first fetch reads them
   const int tid = threadIdx.x;
-  s.active = tid < s.N0 * TVX;
+  // (the last tile may reach past N2)
+  s.active = tid < s.N0 * TVX && tile * TVX + tid / s.N0 < s.N2;
   s.ix = s.active ? tid % s.N0 : 0;
   s.tv = s.active ? tid / s.N0 : 0;
   s.ivx = tile * TVX + s.tv;
@@ -588,7 +605,8 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
       // chunks past the slab repeat its last chunk into the buffer's padding
       const int c = min(64 * (s.wave + k * s.nwave) + s.lane, nchunk - 1);
       const int row = c / per_row, col = c - row * per_row;
-      const int kvx = row % (TVX + 4), kvy = row / (TVX + 4);
+      // (rows past the last plane of C4 belong to no cell: repeat it)
+      const int kvx = min(row % (TVX + 4), s.N2 + 4 - tile * TVX), kvy = row / (TVX + 4);
       s.voff[k] = (unsigned)((s.S2 * kvx + s.S3 * kvy + (long)s.VPL * col) * (long)sizeof(T));
     }
   }
@@ -616,7 +634,7 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
       for (int k = 0; k < 4; k++) s.cell[c].w[j][k] = 0;
   }
   s.bad = 0;
-  s.wave_has_cells = s.wave * 64 < s.N0 * TVX;
+  s.wave_has_cells = __builtin_amdgcn_ballot_w64(s.active) != 0;
   if (NB == 3) {  // planes 0 and 1 in flight; wait for plane 0
     s.fetch(0, 0);
     wait_vm(s.fetch(1, 1));
@@ -650,7 +668,9 @@ struct YsPlan {
 
 // Slab DMA instructions per plane and E points per LDS row of the streaming
 // kernel (the same arithmetic as its set-up).
-long ys_slab_instr(long N0, long tvx, size_t tsz) { return (5 * (tvx + 4) * ((N0 + 4) * (long)tsz / 16) + 63) / 64; }
+long ys_slab_instr(long N0, long tvx, size_t tsz) {
+  return (5 * (tvx + 4) * ys_row_chunks((int)N0, 16 / (int)tsz) + 63) / 64;
+}
 long ys_epr(long N0) { return (N0 + 63) / 64 * 64; }
 
 // want_tvx / want_nb: a chosen vx tile and buffer count (0: free); the
@@ -659,7 +679,7 @@ YsPlan ys_plan(const Geom &g, size_t tsz, int want_tvx = 0, int want_nb = 0) {
   YsPlan p;
   const long N0 = g.n[0], N1 = g.n[1], N2 = g.n[2], N3 = g.n[3];
   const long c4n = c4_elems(N0, N1, N2, N3);
-  if (N0 % 2 || c4n >= (1L << 31)) return p;
+  if (c4n >= (1L << 31)) return p;
   int force = want_tvx, force_nb = want_nb;
   if (const char *e = getenv("VLP4D_YS_TVX")) force = atoi(e);
   if (const char *e = getenv("VLP4D_YS_NBUF")) force_nb = atoi(e);
@@ -667,28 +687,41 @@ YsPlan ys_plan(const Geom &g, size_t tsz, int want_tvx = 0, int want_nb = 0) {
   // (vx tile 2, two buffers), whose barriers are independent, run best for
   // both slab types (double: 8.0 ms against 8.7 at tile 4; float storage 7.5
   // against 8.1; float arithmetic, three waves per SIMD, 5.2 against 6.2).
+  // Lanes past N0 TVX (to whole waves) and past N2 (last tile) do nothing: a
+  // tile is passed over when another keeps over 1/0.9 times as many busy.
+  // Any extents are taken; the vx-blocked kernel, which ragged grids used to
+  // run, is bound by L1 latency: 90 x 77 x 84 x 75 4.23 -> 1.51 ms (double) and
+  // 2.95 -> 0.78 (float), 61 x 50 x 45 x 58 0.78 -> 0.33, 20 x 21 x 22 x 23
+  // 0.30 -> 0.07.  It keeps the grids whose C4 has 2^31 elements or whose
+  // slab does not fit LDS.
   static const int pref_f[][2] = {{2, 2}, {4, 2}, {8, 2}, {4, 3}, {2, 3}, {8, 3}};
   static const int pref_d[][2] = {{2, 2}, {4, 2}, {8, 2}, {4, 3}, {8, 3}, {2, 3}};
-  for (const auto &c : (tsz == sizeof(float) ? pref_f : pref_d)) {
-    const int tvx = c[0], nb = c[1];
-    if (force && tvx != force) continue;
-    if (force_nb && nb != force_nb) continue;
-    if (N2 % tvx) continue;
-    const long lanes = N0 * tvx;
-    if (lanes > 512) continue;
-    const int block = (int)((lanes + 63) / 64 * 64);
-    if ((N0 + 4) % (16 / (long)tsz) || N0 % 16) continue;  // whole 16-byte slab chunks per row
-    const long ninstr = ys_slab_instr(N0, tvx, tsz);
-    if ((ninstr + block / 64 - 1) / (block / 64) > 8) continue;  // DMA slots per wave
-    const size_t lds = nb * (size_t)ninstr * 1024 + nb * 3 * (size_t)ys_epr(N0) * 2 * sizeof(double) +
-                       (24 + 4 * (size_t)(N1 + 2)) * sizeof(double);  // domain constants, per-step table
-    if (lds > 160 * 1024) continue;
-    p.tvx = tvx;
-    p.nb = nb;
-    p.block = block;
-    p.lds = lds;
-    return p;
-  }
+  double best = 0.;
+  for (int pass = 0; pass < 2; pass++)
+    for (const auto &c : (tsz == sizeof(float) ? pref_f : pref_d)) {
+      const int tvx = c[0], nb = c[1];
+      if (force && tvx != force) continue;
+      if (force_nb && nb != force_nb) continue;
+      const long lanes = N0 * tvx;
+      if (lanes > 512) continue;
+      const int block = (int)((lanes + 63) / 64 * 64);
+      const long ninstr = ys_slab_instr(N0, tvx, tsz);
+      if ((ninstr + block / 64 - 1) / (block / 64) > 8) continue;  // DMA slots per wave
+      const size_t lds = nb * (size_t)ninstr * 1024 + nb * 3 * (size_t)ys_epr(N0) * 2 * sizeof(double) +
+                         (24 + 4 * (size_t)(N1 + 2)) * sizeof(double);  // domain constants, per-step table
+      if (lds > 160 * 1024) continue;
+      const double busy = (double)(N0 * N2) / (double)(block * ((N2 + tvx - 1) / tvx));
+      if (pass == 0) {
+        if (busy > best) best = busy;
+        continue;
+      }
+      if (busy < 0.9 * best) continue;
+      p.tvx = tvx;
+      p.nb = nb;
+      p.block = block;
+      p.lds = lds;
+      return p;
+    }
   return p;
 }
 
@@ -705,11 +738,12 @@ void launch_ys_t(const Geom &g, const YsPlan &p, const T *c4, const double *exy,
   // 128^4 (8192) 215.1 -> 216.6 ms, the gathering workgroups being hidden
   // there by the others.
   int iv0 = -1;
-  if ((long)(g.n[2] / TVX) * g.n[3] < 4096) {
+  const int ntile = (g.n[2] + TVX - 1) / TVX;
+  if ((long)ntile * g.n[3] < 4096) {
     const double r = -g.minPhy[3] * g.inv_dx[3];
     if (r > -0.5 && r < g.n[3] - 0.5 && std::fabs(r - std::nearbyint(r)) < 1e-6) iv0 = (int)std::nearbyint(r);
   }
-  const unsigned grid = (unsigned)((g.n[2] / TVX) * (g.n[3] + (iv0 >= 0)));
+  const unsigned grid = (unsigned)(ntile * (g.n[3] + (iv0 >= 0)));
   int force = 0;  // test switch: VLP4D_YS_FORCE=1 rows per cell, 2 direct gather, 3 both
   if (const char *e = getenv("VLP4D_YS_FORCE")) force = atoi(e) & 3;
   int remap = 1;  // VLP4D_YS_REMAP=0: block b -> (b mod ntile, b / ntile)

@@ -16,7 +16,7 @@ from conftest import relmax, sld_box
 pytestmark = pytest.mark.gpu
 
 
-def _run(vlp, orc, n, steps=2, vmax=6.0, alpha=0.4):
+def _run(vlp, orc, n, steps=2, vmax=6.0, alpha=0.4, precision=64):
     """Steps of a strongly perturbed f (both signs of Ex and Ey everywhere)
     from the library and the oracle."""
     lx = 4 * math.pi
@@ -34,7 +34,7 @@ def _run(vlp, orc, n, steps=2, vmax=6.0, alpha=0.4):
     st.step(steps)
     ref, nrj = st.f_interior(), st.diags()["nrj"][1:]
     st.close()
-    with vlp.Vlp4d(cfg) as sim:
+    with vlp.Vlp4d(cfg, precision=precision) as sim:
         sim.set_f(f0)
         sim.step(steps)
         return relmax(sim.get_f(), ref), relmax(sim.diags()["nrj"][1:], nrj)
@@ -56,3 +56,19 @@ def test_slab_of_both_y_offsets(vlp, orc, n):
 def test_velocity_displacement_beyond_a_cell(vlp, orc, n, vmax):
     ef, en = _run(vlp, orc, n, vmax=vmax)
     assert ef < 1e-12 and en < 1e-12
+
+
+# Grids whose rows, tiles and planes do not divide evenly: rows of 4 k + 1, 2,
+# 3 values (so that a plane's rows start 1 to 3 floats past a 16-byte
+# boundary), a last vx tile reaching past Nvx, a last wave with few lanes,
+# the longest rows.  In float a coefficient is stored to 2^-24 relative and is
+# up to sqrt(3)^4 = 9 times f, so two steps differ by about 2 * 9 * 6e-8, and
+# float interpolation adds some 10 roundings per step: 4e-6 is asserted.
+RAGGED = [(61, 13, 11, 12), (17, 12, 13, 10), (90, 11, 21, 10), (51, 12, 19, 13), (251, 10, 11, 10), (10, 77, 10, 15)]
+
+
+@pytest.mark.parametrize("n", RAGGED)
+@pytest.mark.parametrize("precision,tol", [(64, 1e-12), (32, 4e-6), (33, 4e-6)])
+def test_ragged_grids(vlp, orc, n, precision, tol):
+    ef, en = _run(vlp, orc, n, precision=precision)
+    assert ef < tol and en < tol
