@@ -430,6 +430,35 @@ template <typename T> void launch_moments(const Geom &g, const T *f, double *rho
     hipLaunchKernelGGL((k_moments<T, 1>), dim3((unsigned)l2_partials(g)), dim3(256), 0, s, f, g, rho_part, l2_part);
 }
 
+// Conversions between float storage and the interface's doubles, four values
+// per lane (12 bytes per value at HBM rate, 5 times that of the PCIe copy they
+// feed).  Both sides start 16-byte aligned.
+__global__ __launch_bounds__(256) void k_widen(const float *__restrict__ in, double *__restrict__ out, long n) {
+  const long i = 4 * ((long)blockIdx.x * 256 + threadIdx.x);
+  if (i + 4 <= n) {
+    const float4 v = *(const float4 *)(in + i);
+    *(double2 *)(out + i) = make_double2(v.x, v.y);
+    *(double2 *)(out + i + 2) = make_double2(v.z, v.w);
+  } else {
+    for (long k = i; k < n; k++) out[k] = in[k];
+  }
+}
+__global__ __launch_bounds__(256) void k_narrow(const double *__restrict__ in, float *__restrict__ out, long n) {
+  const long i = 4 * ((long)blockIdx.x * 256 + threadIdx.x);
+  if (i + 4 <= n) {
+    const double2 a = *(const double2 *)(in + i), b = *(const double2 *)(in + i + 2);
+    *(float4 *)(out + i) = make_float4((float)a.x, (float)a.y, (float)b.x, (float)b.y);
+  } else {
+    for (long k = i; k < n; k++) out[k] = (float)in[k];
+  }
+}
+void launch_widen(const float *in, double *out, long n, hipStream_t s) {
+  hipLaunchKernelGGL(k_widen, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, s, in, out, n);
+}
+void launch_narrow(const double *in, float *out, long n, hipStream_t s) {
+  hipLaunchKernelGGL(k_narrow, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, s, in, out, n);
+}
+
 // ---------------------------------------------------------------------------
 // Initial conditions, VMO/Init.cpp:126-277 (f must be zero on entry).
 // ---------------------------------------------------------------------------

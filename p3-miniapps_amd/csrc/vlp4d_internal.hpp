@@ -129,6 +129,10 @@ int ystream_tvx(const Geom &g, bool fp32_storage, bool arith32);
 template <typename T>
 void launch_moments(const Geom &g, const T *f, double *rho_part, double *l2_part, hipStream_t s);
 
+// float <-> double copies of n device values (both pointers 16-byte aligned).
+void launch_widen(const float *in, double *out, long n, hipStream_t s);
+void launch_narrow(const double *in, float *out, long n, hipStream_t s);
+
 // Number of l2 partial sums written by launch_advect4d / launch_moments.
 long l2_partials(const Geom &g);
 
