@@ -169,167 +169,248 @@ __global__ __launch_bounds__(256) void k_lag_v(const double *__restrict__ in, do
   }
 }
 
-// x/2 then y/2 through one LDS-resident (x, y) plane (the first and last
-// pair of VO/timestep.hpp:11-55 in one pass over f).  Workgroup of 1024 lanes
-// per (vy, run of G vx planes).  Per plane: stage it in LDS from registers
-// (its loads were issued before the previous plane's y pass); x pass -- wave w
-// owns rows w, w + 16, ...: it reads the stencils of a whole row, then writes
-// the row back in place (no other wave touches it, and one wave's LDS
-// operations execute in order); y pass from LDS to HBM.  The weights come
-// from the context's tables (k_lag_tables): the x ones (x, vx) into registers
-// once per plane -- a lane's x positions are fixed -- and the y ones (y, vy)
-// as wave-uniform reads when a wave's points lie in one row; the LDS holds
-// only the plane.  The plane's loads, its LDS copy and the y pass work on
-// pairs of points (16 bytes per lane).  Each cell's arithmetic is that of
-// k_lag_x followed by k_lag_y.
-constexpr int LAG_XY_THREADS = 1024;
-constexpr int LAG_XY_MAXM = 16;  // plane points per lane: planes up to 16384 points
-
-struct LagTab {  // stencil of one point: six weights and the wrapped first index
+// x/2 then y/2 through one LDS-resident (x, y) plane (the first or last pair of
+// VO/timestep.hpp:11-55 in one pass over f), or, TWICE, the last pair of a step
+// and the first pair of the next; RHO also sums the result over the
+// workgroup's vx planes (field_rho).  Workgroup per (vy, run of G vx planes).
+// A plane goes from registers (loaded during the previous plane's passes)
+// to LDS; each pass gives a wave 64 lines across the lanes and S consecutive
+// points along them.  The displacement is that of the line's velocity, the same
+// for all its points, so a lane has one set of weights and slides a six-value
+// window along its points: (S + 5) / S LDS reads per point, at addresses
+// uniform in the wave up to the lane's line.  A pass in place reads, waits for
+// the workgroup and writes; the last y pass goes from LDS to HBM, and its
+// points are the same in every plane, so their density sums stay in
+// registers.  The LDS row pitch is odd, so neither direction has bank conflicts.
+//
+// Bound: HBM (16 bytes per cell; 0.91 ms per pass at 128^4 at the 4.7 TB/s of a
+// large copy), with one 132 KB plane per CU there: a TWICE pass takes 1.21 ms,
+// and its LDS work (about 0.35 ms) and barriers are not all hidden behind the
+// loads.  128^4 step in a run of steps 4.14 -> 2.97 ms: before, the pair read
+// six stencil values per point and pass from LDS (1.01 ms), the density was a
+// pass of its own (0.41 ms) and neighbouring steps each had their pair.
+struct LagTab {  // stencil of a line: six weights and the wrapped first index of point 0
   double w[6];
   int b;
 };
-static_assert(sizeof(LagTab) == 7 * sizeof(double), "LagTab is copied as 7 doubles");
 
-__device__ __forceinline__ void lag_tab(const Geom &g, int d, double h, double dep, LagTab &t) {
+// The stencils of the x/2 and y/2 passes, fixed for a context: x lines for
+// every vx, then y lines for every vy.
+__global__ __launch_bounds__(256) void k_lag_tables(LagTab *__restrict__ tab, Geom g, double dt) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= g.n[2] + g.n[3]) return;
+  const int d = i < g.n[2] ? 0 : 1, iv = d ? i - g.n[2] : i;
   int j[6];
-  lag_stencil(g, d, h, dep, j, t.w);
-  t.b = j[0];
+  lag_stencil(g, d, g.minPhy[d], dt * (g.minPhy[2 + d] + iv * g.dx[2 + d]), j, tab[i].w);
+  tab[i].b = j[0];
 }
 
-// The stencils of the x/2 and y/2 passes, fixed for a context: x for every
-// (vx, x) -- N2 x N0 entries -- then y for every (vy, y) -- N3 x N1.
-__global__ __launch_bounds__(256) void k_lag_tables(LagTab *__restrict__ tab, Geom g, double dt) {
-  const int N0 = g.n[0], N1 = g.n[1], N2 = g.n[2], N3 = g.n[3];
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < N2 * N0) {
-    const int ivx = i / N0, ix = i % N0;
-    lag_tab(g, 0, g.minPhy[0] + ix * g.dx[0], dt * (g.minPhy[2] + ivx * g.dx[2]), tab[i]);
-  } else if (i < N2 * N0 + N3 * N1) {
-    const int k = i - N2 * N0, ivy = k / N1, iy = k % N1;
-    lag_tab(g, 1, g.minPhy[1] + iy * g.dx[1], dt * (g.minPhy[3] + ivy * g.dx[3]), tab[i]);
+// Results of the line at `line` (LDS, stride st between its N points) at the S
+// points from p0 on (periodic), each handed to out(i, value).  Everything but
+// `line` is uniform in the wave.  (The empty asm keeps the positions from being
+// hoisted out of the loop over planes, where they would be spilled.)
+template <int S, typename F>
+__device__ __forceinline__ void lag_slide(const double *line, int st, int N, int p0, const LagTab &t, F out) {
+  int q = t.b + p0;
+  q = q >= N ? q - N : q;
+  asm volatile("" : "+s"(q));
+  const double *p = line + q * st;
+  const int wrap = st - N * st;
+  double w[6];
+#pragma unroll
+  for (int k = 0; k < 5; k++) {
+    w[k] = *p;
+    q++;
+    p += q == N ? wrap : st;
+    q = q == N ? 0 : q;
+  }
+#pragma unroll
+  for (int i = 0; i < S; i++) {
+    w[(5 + i) % 6] = *p;
+    q++;
+    p += q == N ? wrap : st;
+    q = q == N ? 0 : q;
+    double s = 0.;
+#pragma unroll
+    for (int k = 0; k < 6; k++) s += t.w[k] * w[(i + k) % 6];
+    out(i, s);
+    // at most four points' reads in flight (registers)
+    if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-template <int NC>
-__global__ __launch_bounds__(LAG_XY_THREADS) void k_lag_xy(const double *__restrict__ in, double *__restrict__ out,
-                                                           Geom g, const LagTab *__restrict__ tab, int G,
-                                                           int nchunk) {
-  extern __shared__ double pl[];  // the (x, y) plane, N0 * N1 doubles
-  const int N0 = g.n[0], N1 = g.n[1], N2 = g.n[2];
-  const int P = N0 * N1;
+template <int S, int NT, bool TWICE, bool RHO>
+__global__ __launch_bounds__(NT) void k_lag_plane(const double *__restrict__ in, double *__restrict__ out, Geom g,
+                                                    const LagTab *__restrict__ tab, int G, int nchunk,
+                                                    double *__restrict__ rho_part) {
+  extern __shared__ double pl[];  // the (x, y) plane, rows of `pitch`
+  const int N0 = g.n[0], N1 = g.n[1], N2 = g.n[2], N3 = g.n[3];
+  const int P = N0 * N1, pitch = N0 | 1;
   const int ivy = blockIdx.x / nchunk, chunk = blockIdx.x % nchunk;
   const int v0 = chunk * G, v1 = min(N2, v0 + G);
-  const int l = threadIdx.x, wave = l >> 6, lane = l & 63;
-  constexpr int NW = LAG_XY_THREADS / 64;
-  const LagTab *ytab = tab + (size_t)N2 * N0 + (size_t)ivy * N1;
-  // points go in pairs (x, x+1), 16 bytes per lane for the plane's loads,
-  // its LDS copy, the y pass's reads and its stores (N0 even, checked by the
-  // launcher); with N0 a multiple of 128 a wave's 128 points of the y pass
-  // lie in one row, whose weights are then wave-uniform
-  constexpr int MH = LAG_XY_MAXM / 2;
-  const bool row_waves2 = (N0 & 127) == 0;
-  const int dix = (2 * LAG_XY_THREADS) % N0, diy = (2 * LAG_XY_THREADS) / N0;
-  typedef double d2v __attribute__((ext_vector_type(2)));
-  // the plane in flight: loaded during the previous plane's y pass
-  d2v r[MH];
-  {
-    const double *src = in + ((size_t)ivy * N2 + v0) * (size_t)P;
+  const int l = threadIdx.x, nl = blockDim.x, lane = l & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(l >> 6);
+  const LagTab &ty = tab[N2 + ivy];
+  // x pass: rows 64 rg + lane, points xs .. xs + xn - 1
+  const int nsx = (N0 + S - 1) / S, nsy = (N1 + S - 1) / S;
+  const int xrow = 64 * (wave / nsx) + lane, xs = S * (wave % nsx), xn = min(S, N0 - xs);
+  const bool xact = xrow < N1;
+  double *const xl = pl + (xact ? xrow : 0) * pitch;
+  // y pass: columns 64 cg + lane, points ys .. ys + yn - 1
+  const int ycol = 64 * (wave / nsy) + lane, ys = S * (wave % nsy), yn = min(S, N1 - ys);
+  const bool yact = ycol < N0;
+  double *const yl = pl + (yact ? ycol : 0);
+  // this lane's plane points l, l + nl, ..., at most S of them
+  const int dcol = nl % N0, drow = nl / N0, col0 = l % N0, row0 = l / N0;
+  constexpr bool AHEAD = NT <= 512;  // a plane's loads go out a pass ahead of its use (registers permitting)
+  double r[AHEAD ? S : 1], o[S], rho[RHO ? S : 1];
+  if constexpr (RHO)
 #pragma unroll
-    for (int m = 0; m < MH; m++) {
-      const int p = 2 * (l + LAG_XY_THREADS * m);
-      r[m] = p < P ? *(const d2v *)(src + p) : d2v{0., 0.};
+    for (int i = 0; i < S; i++) rho[i] = 0.;
+  // (opaque copies of the lane index keep the addresses and conditions of the
+  // plane's points from being held across the loop over planes)
+  auto load = [&](const double *src) {
+    int p = l;
+    asm volatile("" : "+v"(p));
+#pragma unroll
+    for (int m = 0; m < S; m++) {
+      // (lanes past the plane repeat its last point; a 32-bit byte offset)
+      r[m] = *(const double *)((const char *)src + 8u * (unsigned)min(p, P - 1));
+      p += nl;
+      if (m % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
-  }
+  };
+  auto keep = [&](int i, double v) { o[i] = v; };
+  if constexpr (AHEAD) load(in + ((size_t)ivy * N2 + v0) * P);
   for (int ivx = v0; ivx < v1; ivx++) {
-    const size_t off = ((size_t)ivy * N2 + ivx) * (size_t)P;
-    // this lane's x stencils (x = lane + 64 c) for this vx
-    LagTab xr[NC];
+    const size_t off = ((size_t)ivy * N2 + ivx) * P;
+    const LagTab &tx = tab[ivx];
+    __syncthreads();  // the previous plane's last pass has read pl
+    {
+      int p = l, col = col0, o = row0 * pitch + col0;
+      asm volatile("" : "+v"(p), "+v"(col), "+v"(o));
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
-      const int ix = lane + 64 * c;
-      if (ix < N0) xr[c] = tab[(size_t)ivx * N0 + ix];
-    }
-    __syncthreads();  // the previous plane's y pass has read pl
-#pragma unroll
-    for (int m = 0; m < MH; m++) {
-      const int p = 2 * (l + LAG_XY_THREADS * m);
-      if (p < P) *(d2v *)(pl + p) = r[m];
-    }
-    __syncthreads();
-    for (int row = wave; row < N1; row += NW) {
-      double *pr = pl + row * N0;
-      double xv[NC];
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        const int ix = lane + 64 * c;
-        xv[c] = 0.;
-        if (ix < N0) {
-          double s = 0.;
-#pragma unroll
-          for (int k = 0; k < 6; k++) {
-            int q = xr[c].b + k;
-            q = q >= N0 ? q - N0 : q;
-            s += xr[c].w[k] * pr[q];
-          }
-          xv[c] = s;
+      for (int m = 0; m < S; m++) {
+        // (lanes past the plane write to a slot behind it)
+        const int at = p < P ? o : pitch * N1;
+        if constexpr (AHEAD) pl[at] = r[m];
+        else pl[at] = *(const double *)((const char *)(in + off) + 8u * (unsigned)min(p, P - 1));
+        p += nl;
+        col += dcol;
+        o += drow * pitch + dcol;
+        if (col >= N0) {
+          col -= N0;
+          o += pitch - N0;
         }
       }
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        const int ix = lane + 64 * c;
-        if (ix < N0) pr[ix] = xv[c];
-      }
     }
     __syncthreads();
-    if (ivx + 1 < v1) {  // next plane's loads, in flight during the y pass
-      const double *nx = in + off + (size_t)P;
+    if constexpr (AHEAD)
+      if (ivx + 1 < v1) load(in + off + P);  // in flight during the passes
 #pragma unroll
-      for (int m = 0; m < MH; m++) {
-        const int p = 2 * (l + LAG_XY_THREADS * m);
-        if (p < P) r[m] = *(const d2v *)(nx + p);
+    for (int half = 0; half < (TWICE ? 2 : 1); half++) {
+      if (xact) lag_slide<S>(xl, 1, N0, xs, tx, keep);
+      __syncthreads();
+      if (xact) {
+        int n = xn;
+        asm volatile("" : "+s"(n));
+#pragma unroll
+        for (int i = 0; i < S; i++)
+          if (i < n) xl[xs + i] = o[i];
+      }
+      __syncthreads();
+      if (TWICE && half == 0) {
+          if (yact) lag_slide<S>(yl, pitch, N1, ys, ty, keep);
+        __syncthreads();
+        if (yact) {
+          int n = yn, row = pitch;
+          asm volatile("" : "+s"(n), "+s"(row));
+#pragma unroll
+          for (int i = 0; i < S; i++)
+            if (i < n) yl[(ys + i) * row] = o[i];
+        }
+        __syncthreads();
       }
     }
-    double *dst = out + off;
-    int ix = (2 * l) % N0, iy = (2 * l) / N0;
-#pragma unroll 4
-    for (int p = 2 * l; p < P; p += 2 * LAG_XY_THREADS) {
-      const int ty = row_waves2 ? __builtin_amdgcn_readfirstlane(iy) : iy;
-      const LagTab &t = ytab[ty];
-      d2v s = {0., 0.};
-#pragma unroll
-      for (int k = 0; k < 6; k++) {
-        int q = t.b + k;
-        q = q >= N1 ? q - N1 : q;
-        const d2v v = *(const d2v *)(pl + q * N0 + ix);
-        s.x += t.w[k] * v.x;
-        s.y += t.w[k] * v.y;
-      }
-      *(d2v *)(dst + p) = s;
-      ix += dix;
-      iy += diy;
-      if (ix >= N0) {
-        ix -= N0;
-        iy++;
+    if (yact) {
+      // a scalar row address and the lane's column
+      char *dst = (char *)(out + off + (size_t)ys * N0);
+      unsigned at = 8u * (unsigned)ycol;
+      int n = yn, row = 8 * N0;
+      asm volatile("" : "+v"(at), "+s"(n), "+s"(row));
+      if (n == S) {  // (no branch between the points)
+        lag_slide<S>(yl, pitch, N1, ys, ty, [&](int i, double v) {
+          *(double *)(dst + at) = v;
+          dst += row;
+          if constexpr (RHO) rho[i] += v;
+        });
+      } else {
+        lag_slide<S>(yl, pitch, N1, ys, ty, [&](int i, double v) {
+          if (i < n) *(double *)(dst + at) = v;
+          dst += row;
+          if constexpr (RHO) rho[i] += v;
+        });
       }
     }
   }
+  if constexpr (RHO)
+    if (yact) {
+      double *dst = rho_part + ((size_t)chunk * N3 + ivy) * P + (size_t)ys * N0 + ycol;
+#pragma unroll
+      for (int i = 0; i < S; i++)
+        if (i < yn) dst[(size_t)i * N0] = rho[i];
+    }
 }
 
-static size_t lag_xy_lds(const Geom &g) { return (size_t)g.n[0] * g.n[1] * sizeof(double); }
+// Waves of a workgroup for S points per lane and pass: every pass has a wave
+// for each of its 64-line groups and S-point segments.
+static int lag_waves(const Geom &g, int S) {
+  const int N0 = g.n[0], N1 = g.n[1];
+  const int x = (N1 + 63) / 64 * ((N0 + S - 1) / S), y = (N0 + 63) / 64 * ((N1 + S - 1) / S);
+  return x > y ? x : y;
+}
 
-// vx runs per vy of the fused x/y pass (0: the plane does not fit; separate
-// kernels).  About 1024 workgroups; VLP4D_LAG_FUSED=0 disables the fusion.
-int lag_xy_chunks(const Geom &g) {
+static size_t lag_xy_lds(const Geom &g) { return ((size_t)(g.n[0] | 1) * g.n[1] + 1) * sizeof(double); }
+
+// 16 or 32 points per lane where that takes at most 8 waves (the plane's loads
+// run a pass ahead and the density is summed along), else 32 and up to 16
+// waves (longest planes: neither, registers); 0: the plane does not fit,
+// separate kernels.  VLP4D_LAG_FUSED=0 disables the fusion.
+static int lag_points(const Geom &g) {
   if (const char *e = getenv("VLP4D_LAG_FUSED"))
     if (atoi(e) == 0) return 0;
-  // rows of up to 128 points (two 64-lane chunks of x weights in registers)
-  if (g.n[0] > 128 || (g.n[0] & 1) || (long)g.n[0] * g.n[1] > (long)LAG_XY_THREADS * LAG_XY_MAXM ||
-      lag_xy_lds(g) > 160 * 1024)
-    return 0;
-  const int want = (1024 + g.n[3] - 1) / g.n[3];
-  const int G = (g.n[2] + want - 1) / want;  // vx planes per workgroup
-  return (g.n[2] + G - 1) / G;
+  if (lag_xy_lds(g) > 160 * 1024) return 0;
+  return lag_waves(g, 16) <= 8 ? 16 : lag_waves(g, 32) <= 16 ? 32 : 0;
+}
+
+// vx runs per vy of the fused pass (0: separate kernels): the fewest rounds of
+// workgroups over the CUs, counting one plane time for a run's start, with
+// runs of at least four planes (their density sums are stored per run).
+int lag_xy_chunks(const Geom &g) {
+  const int S = lag_points(g);
+  if (!S) return 0;
+  int per_cu = (int)(160 * 1024 / lag_xy_lds(g));
+  if (per_cu > 32 / lag_waves(g, S)) per_cu = 32 / lag_waves(g, S);
+  if (per_cu > 8) per_cu = 8;
+  const long cap = 256L * (per_cu < 1 ? 1 : per_cu);
+  int best = 1;
+  long cost = -1;
+  for (int n = 1; n <= g.n[2]; n++) {
+    const int G = (g.n[2] + n - 1) / n;
+    if (n > 1 && G < 4) break;
+    if ((g.n[2] + G - 1) / G != n) continue;  // the same runs in fewer workgroups
+    const long c = ((long)g.n[3] * n + cap - 1) / cap * (G + 1);
+    if (cost < 0 || c < cost) {
+      cost = c;
+      best = n;
+    }
+  }
+  return best;
+}
+
+bool lag_xy_sums(const Geom &g) {
+  const int S = lag_points(g);
+  return S && lag_waves(g, S) <= 8;
 }
 
 // Initial conditions of VO/init.cpp:144-285 (TSI20 differs from the spline
@@ -377,31 +458,42 @@ void launch_lag_x(const Geom &g, const double *in, double *out, double dt, hipSt
   hipLaunchKernelGGL(k_lag_x, dim3(blocks(n)), dim3(256), 0, s, in, out, g, dt);
 }
 
-size_t lag_tables_bytes(const Geom &g) {
-  return ((size_t)g.n[2] * g.n[0] + (size_t)g.n[3] * g.n[1]) * sizeof(LagTab);
-}
+size_t lag_tables_bytes(const Geom &g) { return (size_t)(g.n[2] + g.n[3]) * sizeof(LagTab); }
 
 void launch_lag_tables(const Geom &g, void *tab, double dt, hipStream_t s) {
-  const int n = g.n[2] * g.n[0] + g.n[3] * g.n[1];
-  hipLaunchKernelGGL(k_lag_tables, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (LagTab *)tab, g, dt);
+  hipLaunchKernelGGL(k_lag_tables, dim3(blocks(g.n[2] + g.n[3])), dim3(256), 0, s, (LagTab *)tab, g, dt);
 }
 
-bool launch_lag_xy(const Geom &g, const double *in, double *out, const void *tab, int nchunk, hipStream_t s) {
-  if (nchunk <= 0 || !tab) return false;
+template <int S, int NT, bool TWICE, bool RHO>
+static void launch_plane(const Geom &g, const double *in, double *out, const void *tab, int nchunk, double *rho_part,
+                         hipStream_t s) {
   const int G = (g.n[2] + nchunk - 1) / nchunk;
-  static bool attr = false;
-  if (!attr) {
-    (void)hipFuncSetAttribute((const void *)k_lag_xy<1>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    (void)hipFuncSetAttribute((const void *)k_lag_xy<2>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    attr = true;
+  const void *fn = (const void *)k_lag_plane<S, NT, TWICE, RHO>;
+  if (lag_xy_lds(g) > 64 * 1024)
+    (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lag_xy_lds(g));
+  hipLaunchKernelGGL((k_lag_plane<S, NT, TWICE, RHO>), dim3((unsigned)(g.n[3] * nchunk)), dim3(64 * lag_waves(g, S)),
+                     lag_xy_lds(g), s, in, out, g, (const LagTab *)tab, G, nchunk, rho_part);
+}
+
+template <int S>
+static void launch_plane_sums(const Geom &g, const double *in, double *out, const void *tab, int nchunk, bool twice,
+                              double *rho_part, hipStream_t s) {
+  if (twice) launch_plane<S, 512, true, true>(g, in, out, tab, nchunk, rho_part, s);
+  else if (rho_part) launch_plane<S, 512, false, true>(g, in, out, tab, nchunk, rho_part, s);
+  else launch_plane<S, 512, false, false>(g, in, out, tab, nchunk, nullptr, s);
+}
+
+bool launch_lag_xy(const Geom &g, const double *in, double *out, const void *tab, int nchunk, bool twice,
+                   double *rho_part, hipStream_t s) {
+  if (nchunk <= 0 || !tab) return false;
+  if (!lag_xy_sums(g)) {
+    if (twice) launch_plane<32, 1024, true, false>(g, in, out, tab, nchunk, nullptr, s);
+    else launch_plane<32, 1024, false, false>(g, in, out, tab, nchunk, nullptr, s);
+  } else if (lag_points(g) == 16) {
+    launch_plane_sums<16>(g, in, out, tab, nchunk, twice, rho_part, s);
+  } else {
+    launch_plane_sums<32>(g, in, out, tab, nchunk, twice, rho_part, s);
   }
-  const dim3 grid((unsigned)(g.n[3] * nchunk)), block(LAG_XY_THREADS);
-  const size_t lds = lag_xy_lds(g);
-  const LagTab *t = (const LagTab *)tab;
-  if (g.n[0] <= 64)  // 64-point chunks of an x row
-    hipLaunchKernelGGL(k_lag_xy<1>, grid, block, lds, s, in, out, g, t, G, nchunk);
-  else
-    hipLaunchKernelGGL(k_lag_xy<2>, grid, block, lds, s, in, out, g, t, G, nchunk);
   return true;
 }
 

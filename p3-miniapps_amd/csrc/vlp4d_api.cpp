@@ -341,58 +341,84 @@ int enqueue_step(vlp_ctx *c, int *iter_dev, hipEvent_t *evs = nullptr) {
   return VLP_OK;
 }
 
-// onetimestep of the Lagrange split-step solver (VO/timestep.hpp:11-55):
+// Steps of the Lagrange split-step solver (onetimestep, VO/timestep.hpp:11-55):
 // x/2, y/2 (+ density), field solve with the step's diagnostics, vx, vy, x/2,
-// y/2; the result ends in f.  Timers: the x/y passes count as advec2D, the
+// y/2; the result ends in f.  Within a call the last x/2, y/2 of a step and the
+// first of the next are one pass through the LDS-resident plane (two where
+// the plane does not fit), and the host waits for a step's events only when
+// the next step is queued.  Timers: the x/y passes count as advec2D, the
 // velocity passes as advec4D.
-int lag_step_once(vlp_ctx *c) {
-  hipEvent_t *ev = c->ev;
+int lag_steps(vlp_ctx *c, int nsteps) {
+  if (nsteps == 0) return VLP_OK;
   const Geom &g = c->g;
   const double dt = c->cfg.dt;
-  double *f = (double *)c->f, *t = (double *)c->fnext;
   hipStream_t s = c->stream;
-  HIP_TRY(c, hipEventRecord(ev[0], s));
-  // x/2 + y/2: one pass through an LDS plane and the density from a
-  // streaming pass over its output, or two kernels with the density fused
   const int nch = vlp::lag_xy_chunks(g);
-  const bool fused = vlp::launch_lag_xy(g, f, t, c->lag_tab, nch, s);
-  if (fused) {
-    std::swap(f, t);
-  } else {
-    vlp::launch_lag_x(g, f, t, 0.5 * dt, s);
-    vlp::launch_lag_y(g, t, f, 0.5 * dt, c->rho_part, s);
+  const bool fused = nch > 0, sums = fused && vlp::lag_xy_sums(g);
+  // the x/2, y/2 pair from f into f, `twice` over; rho: with its density
+  auto xy = [&](bool twice, bool rho) {
+    double *f = (double *)c->f, *t = (double *)c->fnext;
+    if (fused) {
+      vlp::launch_lag_xy(g, f, t, c->lag_tab, nch, twice, rho && sums ? c->rho_part : nullptr, s);
+      std::swap(c->f, c->fnext);
+      if (rho && !sums) vlp::launch_moments<double>(g, t, c->rho_part, c->l2_part, s);
+    } else {
+      for (int k = 0; k < (twice ? 2 : 1); k++) {
+        vlp::launch_lag_x(g, f, t, 0.5 * dt, s);
+        vlp::launch_lag_y(g, t, f, 0.5 * dt, rho && k == (twice ? 1 : 0) ? c->rho_part : nullptr, s);
+      }
+    }
+    c->rho_outer = (long)(sums ? nch : 1) * g.n[3];
+  };
+  // ev[4], ev[5] of the first set: around the first pass
+  hipEvent_t *sets[2] = {c->ev, c->evb};
+  auto t_last = std::chrono::steady_clock::now();
+  auto account = [&](int k, bool first) {  // the step of event set k is complete
+    hipEvent_t *ev = sets[k];
+    HIP_TRY(c, hipEventSynchronize(ev[3]));
+    if (first) c->tsec[VLP_T_ADVEC2D] += 1e-3 * ev_ms(c->ev[4], c->ev[5]);
+    c->tsec[VLP_T_FIELD] += 1e-3 * ev_ms(ev[0], ev[1]);
+    c->tsec[VLP_T_ADVEC4D] += 1e-3 * ev_ms(ev[1], ev[2]);
+    c->tsec[VLP_T_ADVEC2D] += 1e-3 * ev_ms(ev[2], ev[3]);
+    c->tcalls[VLP_T_ADVEC2D] += 2;
+    c->tcalls[VLP_T_ADVEC4D]++;
+    c->tcalls[VLP_T_FIELD]++;
+    c->tcalls[VLP_T_FOURIER]++;
+    c->tcalls[VLP_T_DIAG]++;
+    const auto now = std::chrono::steady_clock::now();
+    const double sec = std::chrono::duration<double>(now - t_last).count();
+    t_last = now;
+    c->tsec[VLP_T_MAINLOOP] += sec;
+    c->tcalls[VLP_T_MAINLOOP]++;
+    c->tsec[VLP_T_TOTAL] += sec;
+    return (int)VLP_OK;
+  };
+  HIP_TRY(c, hipEventRecord(c->ev[4], s));
+  xy(false, true);
+  HIP_TRY(c, hipEventRecord(c->ev[5], s));
+  for (int n = 0; n < nsteps; n++) {
+    hipEvent_t *ev = sets[n & 1];
+    HIP_TRY(c, hipEventRecord(ev[0], s));
+    int rc = field(c, c->iter + 1, true, false);
+    if (rc) return rc;
+    HIP_TRY(c, hipEventRecord(ev[1], s));
+    vlp::launch_lag_v(g, 2, (double *)c->f, (double *)c->fnext, c->fb.ex, dt, s);
+    vlp::launch_lag_v(g, 3, (double *)c->fnext, (double *)c->f, c->fb.ey, dt, s);
+    HIP_TRY(c, hipEventRecord(ev[2], s));
+    const bool last = n + 1 == nsteps;
+    xy(!last, !last);
+    HIP_TRY(c, hipEventRecord(ev[3], s));
+    rc = check_launch(c, "step");
+    if (rc) return rc;
+    c->iter++;
+    if (n > 0) {
+      rc = account((n - 1) & 1, n == 1);
+      if (rc) return rc;
+    }
   }
-  HIP_TRY(c, hipEventRecord(ev[1], s));
-  if (fused) vlp::launch_moments<double>(g, f, c->rho_part, c->l2_part, s);
-  c->rho_outer = g.n[3];
-  int rc = field(c, c->iter + 1, true, false);
+  int rc = account((nsteps - 1) & 1, nsteps == 1);
   if (rc) return rc;
-  HIP_TRY(c, hipEventRecord(ev[2], s));
-  vlp::launch_lag_v(g, 2, f, t, c->fb.ex, dt, s);
-  vlp::launch_lag_v(g, 3, t, f, c->fb.ey, dt, s);
-  HIP_TRY(c, hipEventRecord(ev[3], s));
-  if (vlp::launch_lag_xy(g, f, t, c->lag_tab, nch, s)) {
-    std::swap(f, t);
-  } else {
-    vlp::launch_lag_x(g, f, t, 0.5 * dt, s);
-    vlp::launch_lag_y(g, t, f, 0.5 * dt, nullptr, s);
-  }
-  HIP_TRY(c, hipEventRecord(ev[4], s));
-  if (f != (double *)c->f) std::swap(c->f, c->fnext);  // the result is in f
-  rc = check_launch(c, "step");
-  if (rc) return rc;
-  c->iter++;
-  rc = sync_and_check(c);
-  if (rc) return rc;
-  c->tsec[VLP_T_ADVEC2D] += 1e-3 * (ev_ms(ev[0], ev[1]) + ev_ms(ev[3], ev[4]));
-  c->tsec[VLP_T_FIELD] += 1e-3 * ev_ms(ev[1], ev[2]);
-  c->tsec[VLP_T_ADVEC4D] += 1e-3 * ev_ms(ev[2], ev[3]);
-  c->tcalls[VLP_T_ADVEC2D] += 2;
-  c->tcalls[VLP_T_ADVEC4D]++;
-  c->tcalls[VLP_T_FIELD]++;
-  c->tcalls[VLP_T_FOURIER]++;
-  c->tcalls[VLP_T_DIAG]++;
-  return VLP_OK;
+  return sync_and_check(c);
 }
 
 // One onetimestep + swap, events between phases.
@@ -417,7 +443,6 @@ void add_step_timers(vlp_ctx *c, hipEvent_t *ev) {
 }
 
 int step_once(vlp_ctx *c) {
-  if (c->scheme == VLP_SCHEME_LAGRANGE) return lag_step_once(c);
   int rc = enqueue_step(c, nullptr);
   if (rc) return rc;
   c->iter++;
@@ -678,7 +703,8 @@ static int create_ctx(const vlp_config *cfg_in, int precision, int device, int s
     ALLOC(c->c4_alloc, (c->n_c4s + 16) * c->esz);
     c->c4 = (char *)c->c4_alloc + c4_shift(c->g) * c->esz;
   }
-  ALLOC(c->rho_part, N0 * N1 * N3 * (c->xy_groups > 1 ? (size_t)c->xy_groups : 1) * sizeof(double));
+  const int rho_runs = lag ? vlp::lag_xy_chunks(c->g) : c->xy_groups;
+  ALLOC(c->rho_part, N0 * N1 * N3 * (size_t)std::max(rho_runs, 1) * sizeof(double));
   ALLOC(c->l2_part, (size_t)c->n_l2 * sizeof(double));
   ALLOC(c->fb.rho, N0 * N1 * sizeof(double));
   ALLOC(c->fb.ex, N0 * N1 * sizeof(double));
@@ -759,7 +785,12 @@ int vlp_step(vlp_ctx *c, int nsteps) {
   if (rc) return rc;
   if (nsteps < 0 || c->iter + nsteps > c->cfg.nbiter)
     return set_err(c, VLP_E_ARG, "step count exceeds nbiter of the configuration");
-  if (c->scheme == VLP_SCHEME_SPLINE && nsteps > 1) return steps_pipelined(c, nsteps);
+  if (c->scheme == VLP_SCHEME_LAGRANGE) {
+    rc = lag_steps(c, nsteps);
+    if (rc == VLP_E_HIP) c->broken = true;  // queued steps of unknown outcome
+    return rc;
+  }
+  if (nsteps > 1) return steps_pipelined(c, nsteps);
   for (int s = 0; s < nsteps; s++) {
     const auto t0 = std::chrono::steady_clock::now();
     rc = step_once(c);

@@ -156,13 +156,18 @@ void launch_lag_y(const Geom &g, const double *in, double *out, double dt, doubl
 void launch_lag_v(const Geom &g, int d, const double *in, double *out, const double *e, double dt, hipStream_t s);
 // Fused x/2 + y/2 (one pass over f) when the (x, y) plane fits in LDS:
 // lag_xy_chunks gives the vx runs per vy, 0 when not eligible;
-// launch_lag_xy returns false for nchunk 0.
+// launch_lag_xy returns false for nchunk 0.  twice: the pair two times over
+// (the end of one step and the start of the next).  With lag_xy_sums(g), a
+// non-null rho_part (always for twice) receives the density of the result,
+// nchunk * N3 partial planes; without, the caller takes it from the result.
 // The stencil tables of the x/2, y/2 passes (lag_tables_bytes) are built once
 // per context for the half step dt.
 int lag_xy_chunks(const Geom &g);
+bool lag_xy_sums(const Geom &g);
 size_t lag_tables_bytes(const Geom &g);
 void launch_lag_tables(const Geom &g, void *tab, double dt, hipStream_t s);
-bool launch_lag_xy(const Geom &g, const double *in, double *out, const void *tab, int nchunk, hipStream_t s);
+bool launch_lag_xy(const Geom &g, const double *in, double *out, const void *tab, int nchunk, bool twice,
+                   double *rho_part, hipStream_t s);
 
 // Work buffers of the reproducible adjoint scatter: scl (4 doubles: the
 // fixed-point scale S, 1/S, and the max|g| bits), axy (2 per cell), part
