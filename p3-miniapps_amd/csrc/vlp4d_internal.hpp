@@ -212,8 +212,8 @@ struct FieldBufs {
   int nbiter;
 };
 // rho_outer: number of N0*N1 density-partial planes in rho_part (N3, or
-// G*N3 after the fused xy kernel).  Beyond 64 planes they are first summed in
-// RHO_SLICES slices by a wide kernel.
+// G*N3 after the fused xy kernel).  For the analytic fields, more than 64
+// planes are first summed in RHO_SLICES slices by a wide kernel.
 constexpr int RHO_SLICES = 16;
 // iter_dev (optional): device-side iteration counter for graph replays; the
 // diagnostics then go to index *iter_dev + 1, which is stored back.
