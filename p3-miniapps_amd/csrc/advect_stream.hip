@@ -5,7 +5,8 @@
 // work is organised so that every C4 coefficient a workgroup needs crosses
 // from L2 into the CU once, through LDS.
 //
-// Workgroup = (all x) x (TVX consecutive vx) at one vy.  It walks y: at step q
+// Workgroup = (all x) x (TVX consecutive vx) at one vy.  It walks y (all of it, or
+// a segment when there are few workgroups): at step q
 // it holds one y-plane of C4 in LDS -- positions x -2..N0+1, vx tile-2 ..
 // tile+TVX+1, vy ivy-2..ivy+2 (a slab) -- with the next two in flight.
 // Lane (x, vx) keeps the four cells (x, y, vx, vy) whose y-stencil contains
@@ -30,6 +31,7 @@
 // the launch: 140 us of a 16^4 advection, 1.01 ms at 64^4 (FP64).
 #include "advect_common.hpp"
 
+#include <algorithm>
 #include <cstdlib>
 
 namespace vlp {
@@ -95,7 +97,8 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
   int EPR, cpr;    // E points per LDS row (whole 64-point chunks), chunks per row
   unsigned voff[MS];  // C4 byte offset of this lane's chunk in the wave's k-th slab DMA
   int nslot;       // slab DMA instructions of this wave (wave-uniform)
-  int N0, N1, N2, N3, RX, nsteps, oyw;
+  int N0, N1, N2, N3, RX, oyw;
+  int y0, y1;  // the cells y0 <= y < y1 of this workgroup: steps y0 .. y1 + 2
   int ix, tv, ivx, ivy;
   int row0;  // LDS element of the stencil row of a foot with offset 0 along x, vx, vy
   bool active;
@@ -156,7 +159,7 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
         __builtin_amdgcn_global_load_lds((const void *)(src + o), (lds_void *)(sb + k * ls), 16, 0, 0);
         n++;
       }
-    if (q < N1) {
+    if (q < y1) {
       const int ip1 = erow0(q);
       char *el = (char *)(eb + b * 6 * EPR);
       for (int e = wave; e < 3 * cpr; e += nwave, n++) {
@@ -218,7 +221,7 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
     c.acc = 0;
     c.row = cell[(R + 3) & 3].row;
     if (pair) keep &= ~(1 << R);
-    if (q >= N1) {
+    if (q >= y1) {
       // no cell: zero x-weights make its share of a common pass zero
 #pragma unroll
       for (int k = 0; k < 4; k++) c.w[0][k] = 0;
@@ -263,7 +266,7 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
         for (int k = 0; k < 4; k++) c.w[0][k] = 0;  // no share of a common pass
       }
     }
-    if (q == 0) {  // the slots still empty agree with the first cell
+    if (q == y0) {  // the slots still empty agree with the first cell
 #pragma unroll
       for (int k = 1; k < 4; k++) cell[(R + k) & 3].row = c.row;
     }
@@ -426,7 +429,7 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
   // Write cell y = q - 3 (slot (R + 1) & 3).
   template <int R> __device__ __forceinline__ void close(int q) {
     const int y = q - 3;
-    if (y < 0 || y >= N1) return;
+    if (y < y0 || y >= y1) return;
     const A v = cell[(R + 1) & 3].acc;
     if (pair && !((keep >> ((R + 1) & 3)) & 1)) return;
     fbase[(long)N0 * y] = (T)v;
@@ -441,20 +444,20 @@ template <typename T, typename A, int TVX, int NB, int RXC> struct YStream {
   //  NB = 2: the loads of plane q+1 are issued first and overlap the step;
   //   the wait leaves only this step's store of f in flight.
   template <int R> __device__ __forceinline__ void step(int q, int b) {
-    if (NB == 2 && q + 1 < nsteps) fetch(q + 1, b ^ 1);
+    if (NB == 2 && q + 1 < y1 + 3) fetch(q + 1, b ^ 1);
     if (active) {
       double efx = 0., efy = 0.;
-      if (q < N1) field_at(q, b, efx, efy);  // no cell opens beyond the last y
+      if (q < y1) field_at(q, b, efx, efy);  // no cell opens beyond the last y
       open<R>(q, efx, efy);
       accumulate<R>(q, b);
       close<R>(q);
     }
     int n = 0;
     if (NB == 3) {
-      if (q + 2 < nsteps) n = fetch(q + 2, b == 0 ? 2 : b - 1);
+      if (q + 2 < y1 + 3) n = fetch(q + 2, b == 0 ? 2 : b - 1);
     } else {
       // (a shared slab's store may have been skipped: wait for everything)
-      n = (wave_has_cells && !pair && q >= 3 && q - 3 < N1) ? 1 : 0;
+      n = (wave_has_cells && !pair && q >= y0 + 3 && q - 3 < y1) ? 1 : 0;
     }
     wait_vm(n);
     __builtin_amdgcn_s_barrier();
@@ -496,7 +499,7 @@ template <typename T, typename A, int TVX, int NB, int RXC>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(A) == 4 ? 3 : 1)))
 void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geom g,
                                                      FeetConsts fc, double dt, T *__restrict__ fout,
-                                                     int *__restrict__ err, int force, int remap, int iv0) {
+                                                     int *__restrict__ err, int force, int remap, int iv0, int nslab, int ylen) {
   extern __shared__ __align__(16) unsigned char ys_smem[];
   YStream<T, A, TVX, NB, RXC> s;
   s.force = force;
@@ -532,10 +535,13 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
     k[s.KC_VHI] = g.minPhy[2] + fc.rxwidth[2];
     k[s.KC_VHI + 1] = g.minPhy[3] + fc.rxwidth[3];
   }
-  s.nsteps = s.N1 + 3;
   const int ntile = (s.N2 + TVX - 1) / TVX;
   int tile, ivy;
-  ys_block_tile(blockIdx.x, ntile, remap, tile, ivy);
+  // y segments of the whole (tile, slab) grid one after another
+  const int seg = blockIdx.x / (ntile * nslab);
+  s.y0 = seg * ylen;
+  s.y1 = min(s.N1, s.y0 + ylen);
+  ys_block_tile(blockIdx.x - seg * ntile * nslab, ntile, remap, tile, ivy);
   // slab N3 (launched when iv0 >= 0): the second workgroups of slab iv0
   s.pair = 0;
   if (iv0 >= 0) {
@@ -636,22 +642,22 @@ void k_advect4d_ys(const T *__restrict__ c4, const double *__restrict__ exy, Geo
   s.bad = 0;
   s.wave_has_cells = __builtin_amdgcn_ballot_w64(s.active) != 0;
   if (NB == 3) {  // planes 0 and 1 in flight; wait for plane 0
-    s.fetch(0, 0);
-    wait_vm(s.fetch(1, 1));
+    s.fetch(s.y0, 0);
+    wait_vm(s.fetch(s.y0 + 1, 1));
   } else {
-    s.fetch(0, 0);
+    s.fetch(s.y0, 0);
     wait_vm(0);
   }
   __builtin_amdgcn_s_barrier();
-  int b = 0;  // q mod NB
-  for (int q0 = 0; q0 < s.nsteps; q0 += 4) {
+  int b = 0;  // (q - y0) mod NB
+  for (int q0 = s.y0; q0 < s.y1 + 3; q0 += 4) {
     s.template step<0>(q0, b);
     b = b == NB - 1 ? 0 : b + 1;
-    if (q0 + 1 < s.nsteps) s.template step<1>(q0 + 1, b);
+    if (q0 + 1 < s.y1 + 3) s.template step<1>(q0 + 1, b);
     b = b == NB - 1 ? 0 : b + 1;
-    if (q0 + 2 < s.nsteps) s.template step<2>(q0 + 2, b);
+    if (q0 + 2 < s.y1 + 3) s.template step<2>(q0 + 2, b);
     b = b == NB - 1 ? 0 : b + 1;
-    if (q0 + 3 < s.nsteps) s.template step<3>(q0 + 3, b);
+    if (q0 + 3 < s.y1 + 3) s.template step<3>(q0 + 3, b);
     b = b == NB - 1 ? 0 : b + 1;
   }
   if (s.bad) atomicOr(err, 2);
@@ -743,13 +749,36 @@ void launch_ys_t(const Geom &g, const YsPlan &p, const T *c4, const double *exy,
     const double r = -g.minPhy[3] * g.inv_dx[3];
     if (r > -0.5 && r < g.n[3] - 0.5 && std::fabs(r - std::nearbyint(r)) < 1e-6) iv0 = (int)std::nearbyint(r);
   }
-  const unsigned grid = (unsigned)(ntile * (g.n[3] + (iv0 >= 0)));
+  const int nslab = g.n[3] + (iv0 >= 0);
+  // y segments, when the workgroups would not fill the chip: the fewest
+  // rounds of workgroups times steps (three beyond the cells, two steps' time
+  // for the set-up).  Workgroups per CU by LDS and by waves per SIMD (two
+  // with double arithmetic, three with float).  Advection of 16^4 FP64 58 ->
+  // 23 us, 32^4 float 97 -> 43, 48^4 FP64 355 -> 195; from four rounds on one
+  // segment is taken.
+  int ylen = g.n[1];
+  {
+    const int waves = p.block / 64, per_simd = sizeof(A) == 4 ? 3 : 2;
+    const long per_cu = std::max(1L, std::min((long)(160 * 1024 / p.lds), 4L * per_simd / waves));
+    const long cap = 256 * per_cu, w = (long)ntile * nslab;
+    long best = -1;
+    for (int n = 1; n <= (w < 4 * cap ? g.n[1] / 4 : 1); n++) {
+      const int len = (g.n[1] + n - 1) / n;
+      const long cost = (w * n + cap - 1) / cap * (len + 5);
+      if (best < 0 || cost < best) {
+        best = cost;
+        ylen = len;
+      }
+    }
+  }
+  const int nseg = (g.n[1] + ylen - 1) / ylen;
+  const unsigned grid = (unsigned)(ntile * nslab * nseg);
   int force = 0;  // test switch: VLP4D_YS_FORCE=1 rows per cell, 2 direct gather, 3 both
   if (const char *e = getenv("VLP4D_YS_FORCE")) force = atoi(e) & 3;
   int remap = 1;  // VLP4D_YS_REMAP=0: block b -> (b mod ntile, b / ntile)
   if (const char *e = getenv("VLP4D_YS_REMAP")) remap = atoi(e) != 0;
   hipLaunchKernelGGL((k_advect4d_ys<T, A, TVX, NB, RXC>), dim3(grid), dim3(p.block), p.lds, s, c4, exy, g,
-                     feet_consts(g), dt, fout, err, force, remap, iv0);
+                     feet_consts(g), dt, fout, err, force, remap, iv0, nslab, ylen);
 }
 
 template <typename T, typename A, int TVX>

@@ -72,3 +72,12 @@ RAGGED = [(61, 13, 11, 12), (17, 12, 13, 10), (90, 11, 21, 10), (51, 12, 19, 13)
 def test_ragged_grids(vlp, orc, n, precision, tol):
     ef, en = _run(vlp, orc, n, precision=precision)
     assert ef < tol and en < tol
+
+
+# Few workgroups: y goes in segments of one cell more than a quarter of the
+# extent down to four cells, the last one shorter; many: one segment.
+@pytest.mark.parametrize("n", [(16, 16, 10, 10), (16, 17, 10, 10), (16, 19, 12, 11), (10, 31, 10, 10), (32, 64, 10, 12),
+                               (16, 13, 64, 66)])
+def test_y_segments(vlp, orc, n):
+    ef, en = _run(vlp, orc, n)
+    assert ef < 1e-12 and en < 1e-12
