@@ -693,8 +693,11 @@ YsPlan ys_plan(const Geom &g, size_t tsz, int want_tvx = 0, int want_nb = 0) {
   // (vx tile 2, two buffers), whose barriers are independent, run best for
   // both slab types (double: 8.0 ms against 8.7 at tile 4; float storage 7.5
   // against 8.1; float arithmetic, three waves per SIMD, 5.2 against 6.2).
-  // Lanes past N0 TVX (to whole waves) and past N2 (last tile) do nothing: a
-  // tile is passed over when another keeps over 1/0.9 times as many busy.
+  // A tile is passed over when another has over 1/0.9 times as many lanes with
+  // cells on a CU: lanes past N0 TVX (to whole waves) and past N2 (last tile)
+  // do nothing, and the workgroups of a CU are bounded by LDS and waves (three
+  // per SIMD for float storage, else two).  (By the share of such lanes alone,
+  // 80 x 96 x 96 x 80 in float took tile 4: 1.76 ms, tile 2 takes 1.09.)
   // Any extents are taken; the vx-blocked kernel, which ragged grids used to
   // run, is bound by L1 latency: 90 x 77 x 84 x 75 4.23 -> 1.51 ms (double) and
   // 2.95 -> 0.78 (float), 61 x 50 x 45 x 58 0.78 -> 0.33, 20 x 21 x 22 x 23
@@ -716,7 +719,9 @@ YsPlan ys_plan(const Geom &g, size_t tsz, int want_tvx = 0, int want_nb = 0) {
       const size_t lds = nb * (size_t)ninstr * 1024 + nb * 3 * (size_t)ys_epr(N0) * 2 * sizeof(double) +
                          (24 + 4 * (size_t)(N1 + 2)) * sizeof(double);  // domain constants, per-step table
       if (lds > 160 * 1024) continue;
-      const double busy = (double)(N0 * N2) / (double)(block * ((N2 + tvx - 1) / tvx));
+      const long per_cu = std::max(1L, std::min((long)(160 * 1024 / lds),
+                                                4L * (tsz == sizeof(float) ? 3 : 2) / (block / 64)));
+      const double busy = (double)per_cu * N0 * N2 / ((N2 + tvx - 1) / tvx);
       if (pass == 0) {
         if (busy > best) best = busy;
         continue;
