@@ -276,14 +276,20 @@ typedef double d2a __attribute__((ext_vector_type(2)));
 typedef float f4e __attribute__((ext_vector_type(4), aligned(4)));
 typedef double d2e __attribute__((ext_vector_type(2), aligned(8)));
 
-template <typename T, int C, int XT>
+// RAG: lines of any length (the RAG form of the recursion).
+// Against the line kernels, 62 x 66 planes, both passes: 58 points 0.106 ->
+// 0.099 ms (double), 84 points 0.27 -> 0.21, 124 points 0.59 -> 0.48 (float
+// 0.32 -> 0.25); lengths the line kernels have no split for (113 x 118 x 101 x
+// 126 in float) 1.21 -> 0.66.
+template <typename T, int C, int XT, bool RAG>
 __global__ __launch_bounds__(XT == 256 ? 1024 : 512) void k_spline_tile(const T *__restrict__ in, T *__restrict__ out, LineMap m, int P,
                                                      SplineConsts sc, double aC, double aN3) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *tile = reinterpret_cast<T *>(smem_raw);  // [N+4][XT]
   constexpr int VPL = 16 / (int)sizeof(T), CPR = XT / VPL;  // 16-byte chunks per row
   static_assert(CPR <= 64, "a tile row must fit one 64-lane DMA instruction");
-  const int N = P * C;
+  const int N = RAG ? m.N : P * C;
+  const int nl = RAG ? (N + C - 1) / C : P, skip = RAG ? nl * C - N : 0;
   const bool comb = m.is1 == m.X0;
   const long XC = comb ? m.X0 * m.X1 : m.X0;  // contiguous input extent
   const long ntile = (XC + XT - 1) / XT;
@@ -314,22 +320,24 @@ __global__ __launch_bounds__(XT == 256 ? 1024 : 512) void k_spline_tile(const T 
   // recursion down column col = tid / P, lane p = tid % P of the column group
   {
     const int col = tid / P, p = tid & (P - 1);
-    const bool act = col < nx;
-    T *cp = tile + (act ? col : 0);
+    const bool act = col < nx && (!RAG || p < nl);
+    T *cp = tile + (col < nx ? col : 0);
+    const int k0 = RAG ? min(p * C, N - C) : p * C;  // first row of the lane's chunk
     double v[C];
 #pragma unroll
-    for (int i = 0; i < C; i++) v[i] = (double)cp[(2 + p * C + i) * XT];
+    for (int i = 0; i < C; i++) v[i] = (double)cp[(2 + k0 + i) * XT];
     double cm2, cm1, cN, cN1;
-    scan_recursion<C>(v, p, P, sc, aC, aN3, cm2, cm1, cN, cN1);
+    scan_recursion<C, RAG>(v, p, P, sc, aC, aN3, cm2, cm1, cN, cN1, nl, skip);
     __syncthreads();  // all reads of the input rows done before rows are rewritten
     if (act) {
 #pragma unroll
-      for (int i = 0; i < C; i++) cp[(2 + p * C + i) * XT] = (T)v[i];
+      for (int i = 0; i < C; i++)
+        if (!RAG || i >= skip || p < nl - 1) cp[(2 + k0 + i) * XT] = (T)v[i];
       if (p == 0) {
         cp[0] = (T)cm2;
         cp[XT] = (T)cm1;
       }
-      if (p == P - 1) {
+      if (p == nl - 1) {
         cp[(N + 2) * XT] = (T)cN;
         cp[(N + 3) * XT] = (T)cN1;
       }
@@ -337,15 +345,21 @@ __global__ __launch_bounds__(XT == 256 ? 1024 : 512) void k_spline_tile(const T 
   }
   __syncthreads();
   // N+4 coefficient rows out.  When the contiguous extent X0 splits into
-  // whole 16-byte chunks, no chunk straddles two runs of X0, so a chunk stays
+  // whole 16-byte chunks, no chunk straddles two runs of X0, or when the
+  // runs follow one another in the output as in the input, a chunk stays
   // contiguous in the output: a lane keeps one chunk column of the tile and
   // writes it down the rows, one 16-byte LDS read and one multi-dword store
   // per row (output rows are only element-aligned, which global stores
-  // allow).  Else element by element.
+  // allow); a last chunk past the extent goes by its elements.  Else element
+  // by element.
   T *dst = out + i1 * m.os1 + o * m.oos;
-  if (m.X0 % VPL == 0) {
+  if (m.X0 % VPL == 0 || !comb || m.os1 == m.X0) {
     const int c = tid % CPR, rpp = (int)blockDim.x / CPR;
-    if (c * VPL < nx) {
+    if (c * VPL < nx && c * VPL + VPL > nx) {
+      const long J = i0 + (long)c * VPL;  // (X0 is no multiple of VPL: the runs are one)
+      for (int k = tid / CPR; k < N + 4; k += rpp)
+        for (int e = 0; c * VPL + e < nx; e++) dst[(long)k * m.ols + J + e] = tile[k * XT + c * VPL + e];
+    } else if (c * VPL < nx) {
       const long J = i0 + (long)c * VPL;
       const long ox = comb ? (J % m.X0) + (J / m.X0) * m.os1 : J;
       for (int k = tid / CPR; k < N + 4; k += rpp) {
@@ -413,19 +427,19 @@ static void launch_line_scan(const T *in, T *out, const LineMap &m, int P, int l
 #define VLP_LINE_CASE(CC) \
   case CC: return launch_line_scan<T, CC>(in, out, m, P, logP, s);
 
-template <typename T, int C, int XT>
+template <typename T, int C, int XT, bool RAG = false>
 static void launch_tile(const T *in, T *out, const LineMap &m, int P, hipStream_t s) {
   const SplineConsts sc = spline_consts();
   double aC = 1.0, aN3 = 1.0;
   for (int i = 0; i < C; i++) aC *= sc.alpha;
-  for (int i = 0; i < P * C + 3; i++) aN3 *= sc.alpha;
+  for (int i = 0; i < m.N + 3; i++) aN3 *= sc.alpha;
   const bool comb = m.is1 == m.X0;
   const long XC = comb ? m.X0 * m.X1 : m.X0;
   const long ntile = (XC + XT - 1) / XT;
-  const size_t lds = (size_t)(P * C + 4) * XT * sizeof(T);
-  const void *fn = (const void *)k_spline_tile<T, C, XT>;
+  const size_t lds = (size_t)(m.N + 4) * XT * sizeof(T);
+  const void *fn = (const void *)k_spline_tile<T, C, XT, RAG>;
   if (lds > 64 * 1024) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL((k_spline_tile<T, C, XT>), dim3((unsigned)(ntile * (comb ? 1 : m.X1) * m.A)), dim3(XT * P), lds,
+  hipLaunchKernelGGL((k_spline_tile<T, C, XT, RAG>), dim3((unsigned)(ntile * (comb ? 1 : m.X1) * m.A)), dim3(XT * P), lds,
                      s, in, out, m, P, sc, aC, aN3);
 }
 
@@ -435,7 +449,10 @@ static void launch_tile(const T *in, T *out, const LineMap &m, int P, hipStream_
 // 512), the tile in LDS.  Wide tiles move twice the bytes per page a tile
 // touches: each tile row sits on its own memory page when the line stride is
 // large, and the address translations per byte halve.
-static int tile_chunk(const LineMap &m, size_t tsz, int &P, int &XT, int mode = SPLINE_AUTO) {
+// Lines of other lengths up to 128 take 64-position tiles in the RAG form
+// (rag), planes that are no whole chunks where they are padded to some.
+static int tile_chunk(const LineMap &m, size_t tsz, int &P, int &XT, bool &rag, int mode = SPLINE_AUTO) {
+  rag = false;
   if (mode == SPLINE_LINES) return 0;
   if (const char *e = getenv("VLP4D_SPLINE_TILE"))
     if (atoi(e) == 0) return 0;
@@ -464,13 +481,24 @@ static int tile_chunk(const LineMap &m, size_t tsz, int &P, int &XT, int mode = 
   XT = 64;
   int logP, C;
   x_split(m.N, P, logP, C);
-  if (!C || P * 64 > 512) return 0;
+  rag = !C || P * 64 > 512;
+  if (rag) {
+    // float lines of 68, 72 and 76 points keep the line kernel, whose four
+    // lanes fit them (72^4: 0.110 ms for both passes against 0.121)
+    int logQ, D;
+    line_split(m.N, 20, P, logQ, D);
+    if (tsz == sizeof(float) && P == 4 && D > 16) return 0;
+    rag_split(m.N, 8, P, C);
+  }
+  if (!C) return 0;
   if ((size_t)(m.N + 4) * 64 * tsz > 160 * 1024) return 0;
   // input rows start 16-byte aligned (LDS-DMA of whole 16-byte chunks; the
   // buffers themselves are 256-byte aligned)
-  if ((m.ils * tsz) % 16 || (m.is1 * tsz) % 16 || (m.ios * tsz) % 16) return 0;
-  const long XC = m.is1 == m.X0 ? m.X0 * m.X1 : m.X0;
-  if ((XC * (long)tsz) % 16) return 0;  // the last tile's chunks end inside the line family
+  const bool comb = m.is1 == m.X0;  // (then i1 is part of the contiguous index)
+  if ((m.ils * tsz) % 16 || (!comb && (m.is1 * tsz) % 16) || (m.ios * tsz) % 16) return 0;
+  // the last tile's chunks end inside the line family, or in its planes' padding
+  const long XC = comb ? m.X0 * m.X1 : m.X0, XP = (XC * (long)tsz + 15) / 16 * 16 / (long)tsz;
+  if (XP != XC && !((comb ? m.ios : m.ils) >= XP && m.ils >= XP)) return 0;
   return C;
 }
 
@@ -478,7 +506,15 @@ template <typename T> void launch_spline_line(const T *in, T *out, const LineMap
   int P, logP, C;
   {
     int Pt, XT;
-    switch (tile_chunk(m, sizeof(T), Pt, XT, mode)) {
+    bool rag;
+    const int C = tile_chunk(m, sizeof(T), Pt, XT, rag, mode);
+    if (rag) switch (C) {
+      case 10: return launch_tile<T, 10, 64, true>(in, out, m, Pt, s);
+      case 12: return launch_tile<T, 12, 64, true>(in, out, m, Pt, s);
+      case 16: return launch_tile<T, 16, 64, true>(in, out, m, Pt, s);
+      default: break;
+    }
+    else switch (C) {
       case 10: return launch_tile<T, 10, 64>(in, out, m, Pt, s);
       case 11: return launch_tile<T, 11, 64>(in, out, m, Pt, s);
       case 12: return launch_tile<T, 12, 64>(in, out, m, Pt, s);
@@ -515,7 +551,8 @@ template <typename T> void launch_spline_line(const T *in, T *out, const LineMap
 
 int spline_tile_width(const LineMap &m, size_t tsz, int mode) {
   int P, XT;
-  return tile_chunk(m, tsz, P, XT, mode) ? XT : 0;
+  bool rag;
+  return tile_chunk(m, tsz, P, XT, rag, mode) ? XT : 0;
 }
 
 int spline_variant_bits(const Geom &g) {

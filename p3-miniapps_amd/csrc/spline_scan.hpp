@@ -18,22 +18,32 @@ namespace vlp {
 // of the two alpha-sums).  On return v[] holds c[p*C .. p*C+C-1]; lane 0 also
 // gets c[-2], c[-1] and lane P-1 c[N], c[N+1].  Every lane of the group must
 // call this together (cross-lane shuffles).
+//
+// RAG: a line of any length N >= C.  Its last chunk belongs to lane nl - 1,
+// nl = ceil(N / C) <= P, which holds f[N-C .. N-1] -- its own chunk behind
+// the last `skip` = nl C - N values of the one before -- and passes over those
+// skip values where a recursion must not advance; lanes from nl on hold
+// anything and only take part in the shuffles.  v[skip..] of lane nl - 1 are
+// its coefficients.
 // ---------------------------------------------------------------------------
-template <int C>
+template <int C, bool RAG = false>
 __device__ __forceinline__ void scan_recursion(double (&v)[C], int p, int P, const SplineConsts &sc, double aC,
-                                               double aN3, double &cm2, double &cm1, double &cN, double &cN1) {
+                                               double aN3, double &cm2, double &cm1, double &cN, double &cN1,
+                                               int nl_ = 0, int skip_ = 0) {
+  const int nl = RAG ? nl_ : P, skip = RAG ? skip_ : 0;
+  const bool tail = RAG && p == nl - 1;
   const double a = sc.alpha, b = sc.beta, s3 = sc.sqrt3;
   double gp2 = 0., gm3 = 0., ap = a;
 #pragma unroll
   for (int j = 1; j <= 8; j++) {
     gp2 += v[1 + j] * ap;      // meaningful in lane 0
-    gm3 += v[C - 2 - j] * ap;  // meaningful in lane P-1
+    gm3 += v[C - 2 - j] * ap;  // meaningful in lane nl-1
     ap *= a;
   }
   const double f0 = __shfl(v[0], 0, P), f1 = __shfl(v[1], 0, P);
   gp2 = __shfl(gp2, 0, P);
-  const double fm1 = __shfl(v[C - 1], P - 1, P), fm2 = __shfl(v[C - 2], P - 1, P);
-  gm3 = __shfl(gm3, P - 1, P);
+  const double fm1 = __shfl(v[C - 1], nl - 1, P), fm2 = __shfl(v[C - 2], nl - 1, P);
+  gm3 = __shfl(gm3, nl - 1, P);
   // causal
   const double cpm2 = gm3 + fm2;
   const double cpm1 = fm1 + a * cpm2;
@@ -51,28 +61,32 @@ __device__ __forceinline__ void scan_recursion(double (&v)[C], int p, int P, con
   cp = cin;
 #pragma unroll
   for (int i = 0; i < C; i++) {
-    cp = v[i] + a * cp;
+    const double next = v[i] + a * cp;
+    cp = RAG && i < skip && tail ? cp : next;
     v[i] = cp;
   }
-  // lane P-1 holds cp[N-1]: positions N, N+1 and the anti-causal start, using
+  // lane nl-1 holds cp[N-1]: positions N, N+1 and the anti-causal start, using
   // sum_{n=-2}^{N+1} alpha^(N+1-n) g[n] = cp[N+1] - alpha^(N+3) g[-3].
   const double cpN = f0 + a * cp;
   const double cpN1 = f1 + a * cpN;
   const double fnend = gp2 + (cpN1 - aN3 * gm3);
   cN1 = s3 * fnend;
   cN = b * cpN + a * cN1;
-  double cr = (p == P - 1) ? cN : 0.;
+  double cr = (p == nl - 1) ? cN : 0.;
 #pragma unroll
-  for (int i = C - 1; i >= 0; i--) cr = b * v[i] + a * cr;
+  for (int i = C - 1; i >= 0; i--) {
+    const double next = b * v[i] + a * cr;
+    cr = RAG && i < skip && tail ? cr : next;
+  }
   double first = cr;
   mult = aC;
   for (int d = 1; d < P; d <<= 1) {
     const double o = __shfl_down(first, d, P);
-    if (p + d < P) first += mult * o;
+    if (p + d < nl) first += mult * o;
     mult *= mult;
   }
   double cin2 = __shfl_down(first, 1, P);
-  if (p == P - 1) cin2 = cN;
+  if (p == nl - 1) cin2 = cN;
   cr = cin2;
 #pragma unroll
   for (int i = C - 1; i >= 0; i--) {
@@ -81,6 +95,23 @@ __device__ __forceinline__ void scan_recursion(double (&v)[C], int p, int P, con
   }
   cm1 = b * cpm1 + a * cr;  // meaningful in lane 0 (cr = c[0])
   cm2 = b * cpm2 + a * cm1;
+}
+
+// Lanes and chunk of a line of any length N <= 16 pmax for the RAG form: the
+// fewest lanes P (a power of two, at most pmax), then the shortest chunk; C = 0
+// when there is none.
+inline void rag_split(int N, int pmax, int &P, int &C) {
+  P = C = 0;
+  for (int c : {10, 12, 16}) {
+    if (c > N) continue;
+    const int nl = (N + c - 1) / c;
+    int p = 1;
+    while (p < nl) p *= 2;
+    if (p <= pmax && (!C || p < P)) {
+      P = p;
+      C = c;
+    }
+  }
 }
 
 }  // namespace vlp

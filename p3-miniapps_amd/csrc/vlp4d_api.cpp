@@ -42,6 +42,7 @@ struct vlp_ctx {
   void *f = nullptr, *fnext = nullptr, *cxy = nullptr, *tv = nullptr, *c4 = nullptr;
   void *c4_alloc = nullptr;  // allocation holding c4 (c4_shift elements in)
   size_t n_f = 0, n_cxy = 0, n_tv = 0, n_c4 = 0;
+  size_t n_cxys = 0;  // stored CXY (padded planes)
   size_t n_c4s = 0;  // stored C4 (layout of c4_pitch) plus a zeroed tail
   double *rho_part = nullptr, *l2_part = nullptr;
   long n_l2 = 0;
@@ -184,7 +185,7 @@ template <typename T> int run_spline_xy(vlp_ctx *c) {
     }
   }
   const long N1 = g.n[1], N2 = g.n[2], N3 = g.n[3];
-  const long E0 = g.n[0] + 4, E1 = N1 + 4;
+  const long E0 = g.n[0] + 4;
   T *tx = (T *)c->tv;
   vlp::launch_spline_x<T>(g, (const T *)c->f, tx, c->stream);
   // y-pass: tx (E0, N1, N2, N3) -> cxy (E0, E1, N2, N3); lanes along x
@@ -192,18 +193,19 @@ template <typename T> int run_spline_xy(vlp_ctx *c) {
   m.N = (int)N1;
   m.X0 = E0; m.X1 = N2; m.A = N3;
   m.is0 = 1; m.is1 = E0 * N1; m.ios = E0 * N1 * N2; m.ils = E0;
-  m.os0 = 1; m.os1 = E0 * E1; m.oos = E0 * E1 * N2; m.ols = E0;
+  const long P = vlp::xy_plane(g.n[0], N1);
+  m.os0 = 1; m.os1 = P; m.oos = P * N2; m.ols = E0;
   vlp::launch_spline_line<T>(tx, (T *)c->cxy, m, c->stream);
   return VLP_OK;
 }
 
-// vx-pass: cxy (E0*E1, N2, N3) -> tv (E0*E1, E2, N3); lanes along (x, y)
+// vx-pass: cxy (planes, N2, N3) -> tv (planes, E2, N3); lanes along (x, y)
 vlp::LineMap vx_map(const Geom &g) {
   const long N2 = g.n[2], N3 = g.n[3];
-  const long P = (long)(g.n[0] + 4) * (g.n[1] + 4), E2 = N2 + 4;
+  const long P = vlp::xy_plane(g.n[0], g.n[1]), E2 = N2 + 4;
   vlp::LineMap m{};
   m.N = (int)N2;
-  m.X0 = P; m.X1 = N3; m.A = 1;
+  m.X0 = (long)(g.n[0] + 4) * (g.n[1] + 4); m.X1 = N3; m.A = 1;
   m.is0 = 1; m.is1 = P * N2; m.ios = 0; m.ils = P;
   m.os0 = 1; m.os1 = P * E2; m.oos = 0; m.ols = P;
   return m;
@@ -226,7 +228,8 @@ vlp::LineMap vy_map(const Geom &g) {
   vlp::LineMap q{};
   q.N = g.n[3];
   q.X0 = E0; q.X1 = E1; q.A = E2;
-  q.is0 = 1; q.is1 = E0; q.ios = E0 * E1; q.ils = E0 * E1 * E2;
+  const long P = vlp::xy_plane(g.n[0], g.n[1]);
+  q.is0 = 1; q.is1 = E0; q.ios = P; q.ils = P * E2;
   q.os0 = 1; q.os1 = cp.s1; q.oos = cp.s2; q.ols = cp.s3;
   return q;
 }
@@ -668,7 +671,8 @@ static int create_ctx(const vlp_config *cfg_in, int precision, int device, int s
   c->n_f = N0 * N1 * N2 * N3;
   // the Lagrange solver keeps no spline coefficients
   c->n_cxy = lag ? 0 : (N0 + 4) * (N1 + 4) * N2 * N3;
-  c->n_tv = lag ? 0 : (N0 + 4) * (N1 + 4) * (N2 + 4) * N3;
+  c->n_cxys = lag ? 0 : (size_t)vlp::xy_plane(N0, N1) * N2 * N3;
+  c->n_tv = lag ? 0 : (size_t)vlp::xy_plane(N0, N1) * (N2 + 4) * N3;
   c->n_c4 = lag ? 0 : (N0 + 4) * (N1 + 4) * (N2 + 4) * (N3 + 4);
   c->n_c4s = lag ? 0 : vlp::c4_elems(N0, N1, N2, N3);
   c->n_l2 = vlp::l2_partials(c->g);
@@ -696,7 +700,7 @@ static int create_ctx(const vlp_config *cfg_in, int precision, int device, int s
   ALLOC(c->fnext, c->n_f * c->esz);
   if (lag) ALLOC(c->lag_tab, vlp::lag_tables_bytes(c->g));
   if (!lag) {
-    ALLOC(c->cxy, c->n_cxy * c->esz);
+    ALLOC(c->cxy, c->n_cxys * c->esz);
     ALLOC(c->tv, c->n_tv * c->esz);
     // C4 starts c4_shift elements into its allocation, so that each line of
     // the vy pass's output starts on a 64-byte boundary
@@ -937,7 +941,14 @@ int vlp_get_buffer(vlp_ctx *c, int which, double *host, size_t n) {
   if (!host || n != vlp_buffer_size(c, which) || n == 0) return set_err(c, VLP_E_SIZE, "buffer size mismatch");
   switch (which) {
     case VLP_BUF_F: return download(c, c->f, n, host);
-    case VLP_BUF_CXY: return download(c, c->cxy, n, host);
+    case VLP_BUF_CXY: {
+      std::vector<double> full(c->n_cxys);
+      rc = download(c, c->cxy, c->n_cxys, full.data());
+      if (rc) return rc;
+      const size_t P = (size_t)vlp::xy_plane(c->cfg.nxmax[0], c->cfg.nxmax[1]), np = c->n_cxys / P, w = n / np;
+      for (size_t k = 0; k < np; k++) memcpy(host + k * w, full.data() + k * P, w * sizeof(double));
+      return VLP_OK;
+    }
     case VLP_BUF_C4: {
       // from the allocation's start, which is aligned
       const size_t sh = (size_t)c4_shift(c->g);

@@ -2,8 +2,10 @@
 //
 // Device data layout (all x fastest, like the reference's layout_left views):
 //   F    : interior f, N0*N1*N2*N3                         (positions 0..N-1 per dim)
-//   CXY  : (N0+4)*(N1+4)*N2*N3, x,y on -2..N+1, v interior  (spline along x and y)
-//   TV   : (N0+4)*(N1+4)*(N2+4)*N3, also holds the x-pass output (N0+4)*N1*N2*N3
+//   CXY  : (N0+4)*(N1+4)*N2*N3, x,y on -2..N+1, v interior  (spline along x and y),
+//          (x, y) planes padded to 16 elements (xy_plane)
+//   TV   : (N0+4)*(N1+4)*(N2+4)*N3, the same planes; also holds the x-pass
+//          output (N0+4)*N1*N2*N3
 //   C4   : positions -3..N+2 along y, vx, vy (the coefficients fill -2..N+1,
 //          the outer layer stays 0) and -2..N+1 along x, in rows of N0+4:
 //          position (p0, p1, p2, p3) at (p0+3) + s1 (p1+3) + s2 (p2+3) +
@@ -28,6 +30,10 @@
 #include "../../include/vlp4d.h"
 
 namespace vlp {
+
+// Pitch of an (x, y) plane of CXY and TV (elements): whole 64-byte blocks for
+// floats, so that planes start 16-byte aligned whatever the extents.
+__host__ __device__ inline long xy_plane(long N0, long N1) { return ((N0 + 4) * (N1 + 4) + 15) / 16 * 16; }
 
 // Pitches of the C4 storage (elements): row (y), plane (vx), volume (vy).
 struct C4Pitch {

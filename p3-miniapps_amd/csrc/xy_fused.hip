@@ -35,10 +35,16 @@ template <typename A> __device__ __forceinline__ void eta4(A w, A e[4]) { bsplin
 // density sums of those points in registers across the vx planes.
 constexpr int XY_NT = 512, XY_NPT = 32;
 
-template <typename T, typename A, int C>
+// RAG: lines of any length (the RAG form of the recursion, Px and Py lanes).
+// Such planes used to run the single-lane x kernel, a strided y kernel and
+// k_advect2d_rho, three passes over the plane with one lane per line: xy
+// phases of 113 x 118 x 101 x 126 in float 2.32 -> 0.92 ms, 90 x 77 x 84 x 75
+// in double 1.17 -> 0.41, 33 x 33 x 39 x 37 0.095 -> 0.061.
+template <typename T, typename A, int C, bool RAG>
 __global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *__restrict__ cxy, Geom g, double dth,
                                                    int G, double *__restrict__ rho_part, int *__restrict__ err,
-                                                   SplineConsts sc, double aC, double aN3x, double aN3y) {
+                                                   SplineConsts sc, double aC, double aN3x, double aN3y, int Px_,
+                                                   int Py_) {
   extern __shared__ __align__(16) unsigned char xy_smem[];
   T *pl = (T *)xy_smem;
   const int N0 = g.n[0], N1 = g.n[1], N2 = g.n[2], N3 = g.n[3];
@@ -47,10 +53,12 @@ __global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *
   // ety[y][4], and the stencil base row jy0 in jty[y]
   A *ety = (A *)(xy_smem + (((size_t)E1 * R * sizeof(T) + 15) & ~(size_t)15));
   int *jty = (int *)(ety + 4 * N1);
-  const int Px = N0 / C, Py = N1 / C;
+  const int Px = RAG ? Px_ : N0 / C, Py = RAG ? Py_ : N1 / C;
+  const int nlx = RAG ? (N0 + C - 1) / C : Px, nly = RAG ? (N1 + C - 1) / C : Py;
+  const int skx = RAG ? nlx * C - N0 : 0, sky = RAG ? nly * C - N1 : 0;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int grp = blockIdx.x % G, ivy = blockIdx.x / G;
-  const int VG = N2 / G, v0 = grp * VG;
+  const int VG = (N2 + G - 1) / G, v0 = min(N2, grp * VG), v1 = min(N2, v0 + VG);
   // advection lanes
   const int nseg = XY_NT / N0, seg = tid / N0, xi = tid - seg * N0;
   const int ylen = (N1 + nseg - 1) / nseg, y0 = seg * ylen;
@@ -71,25 +79,27 @@ __global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *
   // (the first plane's barriers order these writes before their reads)
   // x pass lane: first plane's chunk in registers
   const int px = tid & (Px - 1), xl = tid / Px;
-  for (int ivx = v0; ivx < v0 + VG; ivx++) {
+  for (int ivx = v0; ivx < v1; ivx++) {
     // 1. x recursions, rows 2..N1+1 of the plane
     for (int r0 = 0; r0 < N1; r0 += XY_NT / Px) {
       const int y = r0 + xl;
       double v[C];
-      const T *src = f + ((long)ivx + (long)N2 * ivy) * N0 * N1 + (long)(y < N1 ? y : 0) * N0 + px * C;
+      const int x0 = RAG ? min(px * C, N0 - C) : px * C;  // first point of the lane's chunk
+      const T *src = f + ((long)ivx + (long)N2 * ivy) * N0 * N1 + (long)(y < N1 ? y : 0) * N0 + x0;
 #pragma unroll
       for (int i = 0; i < C; i++) v[i] = (double)src[i];
       double cm2, cm1, cN, cN1;
-      scan_recursion<C>(v, px, Px, sc, aC, aN3x, cm2, cm1, cN, cN1);
-      if (y < N1) {
+      scan_recursion<C, RAG>(v, px, Px, sc, aC, aN3x, cm2, cm1, cN, cN1, nlx, skx);
+      if (y < N1 && (!RAG || px < nlx)) {
         T *row = pl + (y + 2) * R;
 #pragma unroll
-        for (int i = 0; i < C; i++) row[2 + px * C + i] = (T)v[i];
+        for (int i = 0; i < C; i++)
+          if (!RAG || i >= skx || px < nlx - 1) row[2 + x0 + i] = (T)v[i];
         if (px == 0) {
           row[0] = (T)cm2;
           row[1] = (T)cm1;
         }
-        if (px == Px - 1) {
+        if (px == nlx - 1) {
           row[N0 + 2] = (T)cN;
           row[N0 + 3] = (T)cN1;
         }
@@ -102,22 +112,24 @@ __global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *
       const int py = tid & (Py - 1), yl = tid / Py, yl0 = (wave * 64) / Py;
       for (int c0 = 0; c0 + yl0 < E0; c0 += XY_NT / Py) {
         const int xc = c0 + yl;
-        const bool act = xc < E0;
+        const bool act = xc < E0 && (!RAG || py < nly);
         double w[C];
-        const T *col = pl + (act ? xc : 0) + (2 + py * C) * R;
+        const int r0 = RAG ? min(py * C, N1 - C) : py * C;  // first row of the lane's chunk
+        const T *col = pl + (xc < E0 ? xc : 0) + (2 + r0) * R;
 #pragma unroll
         for (int i = 0; i < C; i++) w[i] = (double)col[i * R];
         double cm2, cm1, cN, cN1;
-        scan_recursion<C>(w, py, Py, sc, aC, aN3y, cm2, cm1, cN, cN1);
+        scan_recursion<C, RAG>(w, py, Py, sc, aC, aN3y, cm2, cm1, cN, cN1, nly, sky);
         if (act) {
           T *cw = pl + xc;
 #pragma unroll
-          for (int i = 0; i < C; i++) cw[(2 + py * C + i) * R] = (T)w[i];
+          for (int i = 0; i < C; i++)
+            if (!RAG || i >= sky || py < nly - 1) cw[(2 + r0 + i) * R] = (T)w[i];
           if (py == 0) {
             cw[0] = (T)cm2;
             cw[R] = (T)cm1;
           }
-          if (py == Py - 1) {
+          if (py == nly - 1) {
             cw[(N1 + 2) * R] = (T)cN;
             cw[(N1 + 3) * R] = (T)cN1;
           }
@@ -129,12 +141,12 @@ __global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *
     // contiguous in global memory, so it leaves as 16-byte chunks, lane after
     // lane (row and column of a chunk tracked incrementally), as
     // non-temporal stores (the plane is read again only by the vx spline
-    // pass, after the whole kernel); per element when the rows do not split
-    // into whole chunks.
+    // pass, after the whole kernel).  A chunk may straddle two rows when they
+    // do not split into whole chunks; the last one ends in the plane's padding.
     {
-      T *dst = cxy + ((long)ivx + (long)N2 * ivy) * E0 * E1;
+      T *dst = cxy + ((long)ivx + (long)N2 * ivy) * xy_plane(N0, N1);
       constexpr int VPC = 16 / (int)sizeof(T);
-      if (E0 % VPC == 0 && ((size_t)dst & 15) == 0) {
+      if (E0 % VPC == 0) {
         const int cpr = E0 / VPC, nch = cpr * E1;
         const int drow = XY_NT / cpr, dcol = XY_NT - drow * cpr;
         int row = tid / cpr, col = tid - row * cpr;
@@ -153,8 +165,23 @@ __global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *
           }
         }
       } else {
-        for (int yr = wave; yr < E1; yr += XY_NT / 64)
-          for (int xc = lane; xc < E0; xc += 64) dst[(long)yr * E0 + xc] = pl[yr * R + xc];
+        const int nch = (E0 * E1 + VPC - 1) / VPC;
+        const int drow = VPC * XY_NT / E0, dcol = VPC * XY_NT - drow * E0;
+        int row = VPC * tid / E0, col = VPC * tid - row * E0;
+        for (int k = tid; k < nch; k += XY_NT) {
+          const T *s = pl + row * R + col;
+          typedef T chunk_t __attribute__((ext_vector_type(VPC)));
+          chunk_t v;
+#pragma unroll
+          for (int e = 0; e < VPC; e++) v[e] = s[col + e < E0 ? e : e + R - E0];
+          __builtin_nontemporal_store(v, (chunk_t *)(dst + (long)VPC * k));
+          row += drow;
+          col += dcol;
+          if (col >= E0) {
+            col -= E0;
+            row++;
+          }
+        }
       }
     }
     // 4. 2-D advection at (x - dt/2 vx, y - dt/2 vy), interp_2D's spline branch
@@ -281,22 +308,41 @@ size_t xy_lds(const Geom &g, size_t tsz) {
   return plane + (size_t)g.n[1] * (4 * sizeof(double) + sizeof(int));
 }
 
-// C of the fused kernel for a geometry (0: not eligible): N0 = Px C and
-// N1 = Py C with Px, Py powers of two, the plane fits in LDS, every lane owns
-// at most XY_NPT advection points.
-int xy_chunk(const Geom &g, size_t tsz) {
+// Chunk and lanes of the fused kernel for a geometry (C = 0: not eligible): the
+// plane fits in LDS, every lane owns at most XY_NPT advection points, and N0 =
+// Px C and N1 = Py C with Px, Py powers of two, or (rag) Px C and Py C cover
+// N0 and N1 with the fewest lanes.
+struct XyPlan {
+  int C = 0, Px = 0, Py = 0;
+  bool rag = false;
+};
+XyPlan xy_plan(const Geom &g, size_t tsz) {
+  XyPlan p;
   const int N0 = g.n[0], N1 = g.n[1];
+  if (N0 > XY_NT || xy_lds(g, tsz) > 160 * 1024) return p;
+  const int nseg = XY_NT / N0, ylen = (N1 + nseg - 1) / nseg;
+  if (ylen > XY_NPT) return p;
   for (int C : {16, 12}) {
     if (N0 % C || N1 % C) continue;
     const int Px = N0 / C, Py = N1 / C;
     if ((Px & (Px - 1)) || (Py & (Py - 1)) || Px > 16 || Py > 16) continue;
-    if (N0 > XY_NT) continue;
-    const int nseg = XY_NT / N0, ylen = (N1 + nseg - 1) / nseg;
-    if (ylen > XY_NPT) continue;
-    if (xy_lds(g, tsz) > 160 * 1024) continue;
-    return C;
+    p.C = C;
+    p.Px = Px;
+    p.Py = Py;
+    return p;
   }
-  return 0;
+  for (int C : {10, 12, 16}) {
+    if (C > N0 || C > N1) continue;
+    int Px = 1, Py = 1;
+    while (Px * C < N0) Px *= 2;
+    while (Py * C < N1) Py *= 2;
+    if (Px > 16 || Py > 16 || (p.C && Px + Py >= p.Px + p.Py)) continue;
+    p.C = C;
+    p.Px = Px;
+    p.Py = Py;
+    p.rag = true;
+  }
+  return p;
 }
 
 }  // namespace
@@ -304,36 +350,44 @@ int xy_chunk(const Geom &g, size_t tsz) {
 int xy_fused_groups(const Geom &g, size_t tsz) {
   if (const char *e = getenv("VLP4D_XY_FUSED"))
     if (atoi(e) == 0) return 0;
-  if (!xy_chunk(g, tsz)) return 0;
+  if (!xy_plan(g, tsz).C) return 0;
   // about two rounds of workgroups over the 256 CUs (one or two per CU)
   const int per_cu = xy_lds(g, tsz) > 80 * 1024 ? 1 : 2;
   int G = 1;
-  while (G * 2 <= g.n[2] && g.n[2] % (G * 2) == 0 && (long)G * g.n[3] < 256L * per_cu) G *= 2;
+  // (the last group may be shorter)
+  while (G * 2 <= g.n[2] && (long)G * g.n[3] < 256L * per_cu) G *= 2;
   return G;
 }
 
-template <typename T, typename A, int C>
+template <typename T, typename A, int C, bool RAG>
 static void launch_xy_t(const Geom &g, const T *f, T *cxy, double dth, int G, double *rho_part, int *err,
-                        hipStream_t s) {
+                        const XyPlan &p, hipStream_t s) {
   const SplineConsts sc = spline_consts();
   double aC = 1.0, aN3x = 1.0, aN3y = 1.0;
   for (int i = 0; i < C; i++) aC *= sc.alpha;
   for (int i = 0; i < g.n[0] + 3; i++) aN3x *= sc.alpha;
   for (int i = 0; i < g.n[1] + 3; i++) aN3y *= sc.alpha;
   const size_t lds = xy_lds(g, sizeof(T));
-  const void *fn = (const void *)k_xy_adv2d<T, A, C>;
+  const void *fn = (const void *)k_xy_adv2d<T, A, C, RAG>;
   if (lds > 64 * 1024) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL((k_xy_adv2d<T, A, C>), dim3((unsigned)(G * g.n[3])), dim3(XY_NT), lds, s, f, cxy, g, dth, G,
-                     rho_part, err, sc, aC, aN3x, aN3y);
+  hipLaunchKernelGGL((k_xy_adv2d<T, A, C, RAG>), dim3((unsigned)(G * g.n[3])), dim3(XY_NT), lds, s, f, cxy, g, dth, G,
+                     rho_part, err, sc, aC, aN3x, aN3y, p.Px, p.Py);
 }
 
 template <typename T, typename A>
 bool launch_xy_adv2d(const Geom &g, const T *f, T *cxy, double dt_half, double *rho_part, int *err, hipStream_t s) {
   const int G = xy_fused_groups(g, sizeof(T));
   if (!G) return false;
-  switch (xy_chunk(g, sizeof(T))) {
-    case 16: launch_xy_t<T, A, 16>(g, f, cxy, dt_half, G, rho_part, err, s); return true;
-    case 12: launch_xy_t<T, A, 12>(g, f, cxy, dt_half, G, rho_part, err, s); return true;
+  const XyPlan p = xy_plan(g, sizeof(T));
+  if (p.rag) switch (p.C) {
+    case 16: launch_xy_t<T, A, 16, true>(g, f, cxy, dt_half, G, rho_part, err, p, s); return true;
+    case 12: launch_xy_t<T, A, 12, true>(g, f, cxy, dt_half, G, rho_part, err, p, s); return true;
+    case 10: launch_xy_t<T, A, 10, true>(g, f, cxy, dt_half, G, rho_part, err, p, s); return true;
+    default: return false;
+  }
+  switch (p.C) {
+    case 16: launch_xy_t<T, A, 16, false>(g, f, cxy, dt_half, G, rho_part, err, p, s); return true;
+    case 12: launch_xy_t<T, A, 12, false>(g, f, cxy, dt_half, G, rho_part, err, p, s); return true;
     default: return false;
   }
 }
