@@ -121,48 +121,52 @@ __device__ __forceinline__ unsigned long long to_fixed(double x) {
 }
 
 // The same scatter by blocks of cells, with reproducible sums.  A workgroup
-// takes BX x 2 x 2 x 2 cells (x fastest, one cell per lane) and adds their
-// coefficient-adjoint contributions, as 64-bit fixed-point integers (scale
-// S = *scl, a power of two with |g| S < 2^50), into an LDS copy of the
-// coefficient region they reach when every foot lies within one cell below
-// its own (ip_d - c_d in {-1, 0}: positions c - 2 .. c + 2 per dimension);
-// a contribution outside it goes straight to lc4 (read as 64-bit integers).
-// The region is then added to lc4, one atomic per nonzero entry instead of
-// one per cell and stencil point: (BX + 4) 6^3 / (8 BX) ~ 29 global atomics
-// per cell instead of 256.  With the field term, each cell's pair
-// (ax, ay) -- g times the derivative of the interpolation along the foot,
-// times d foot / d E-bar -- is written to axy, for the E gathers below.
-template <int BX>
-__global__ __launch_bounds__(8 * BX) void k_adj_advect4d_blk(const double *__restrict__ c4,
-                                                           const double *__restrict__ ex,
-                                                           const double *__restrict__ ey, Geom g, FeetConsts fc,
-                                                           double dt, const double *__restrict__ gin,
-                                                           unsigned long long *__restrict__ lc4,
-                                                           double *__restrict__ axy, const double *__restrict__ scl,
-                                                           int field_term) {
-  constexpr int RX = BX + 4, RY = 6, RV = 6;  // coefficient region (x, y, vx, vy)
-  constexpr int NREG = RX * RY * RV * RV;
-  constexpr int NT = 8 * BX;
+// takes BX x BV x BV x BV cells and adds their coefficient-adjoint
+// contributions, as 64-bit fixed-point integers (scale S = *scl, a power of two
+// with |g| S < 2^50), into an LDS copy of the coefficient region they reach
+// when every foot lies within one cell below its own (ip_d - c_d in {-1, 0}:
+// positions c - 2 .. c + 2 per dimension); a contribution outside it goes
+// straight to lc4 (read as 64-bit integers).  The region is then added to lc4,
+// one atomic per nonzero entry instead of one per cell and stencil point:
+// (BX + 4) (BV + 4)^3 per BX BV^3 cells, 9 per cell for BX = 32, BV = 4
+// instead of 256.  With the field term, each cell's pair (ax, ay) -- g times
+// the derivative of the interpolation along the foot, times d foot / d E-bar --
+// is written to axy, for the E gathers below.
+//
+// Bound: the flush's device atomics and the latency of 2 waves per SIMD (LDS
+// and registers).  BV = 4 flushes 3 times fewer entries than BV = 2 (29 per
+// cell): 48^4 2.02 -> 1.30 ms.
+template <int BV>
+__global__ __launch_bounds__(512) void k_adj_advect4d_blk(const double *__restrict__ c4,
+                                                          const double *__restrict__ ex,
+                                                          const double *__restrict__ ey, Geom g, FeetConsts fc,
+                                                          double dt, const double *__restrict__ gin,
+                                                          unsigned long long *__restrict__ lc4,
+                                                          double *__restrict__ axy, const double *__restrict__ scl,
+                                                          int field_term, int BX) {
+  constexpr int RY = BV + 4, RV = BV + 4;  // coefficient region along y, vx, vy
+  const int RX = BX + 4, NREG = RX * RY * RV * RV, NT = blockDim.x;
   extern __shared__ __align__(16) unsigned char adj_smem[];
   unsigned long long *reg = (unsigned long long *)adj_smem;
   const int N0 = g.n[0], N1 = g.n[1], N2 = g.n[2], N3 = g.n[3];
-  const int nbx = (N0 + BX - 1) / BX, nby = (N1 + 1) / 2, nbv = (N2 + 1) / 2;
+  const int nbx = (N0 + BX - 1) / BX, nby = (N1 + BV - 1) / BV, nbv = (N2 + BV - 1) / BV;
   long b = blockIdx.x;
   const int bx = (int)(b % nbx);
   b /= nbx;
   const int by = (int)(b % nby);
   b /= nby;
   const int bvx = (int)(b % nbv), bvy = (int)(b / nbv);
-  const int x0 = bx * BX, y0 = 2 * by, vx0 = 2 * bvx, vy0 = 2 * bvy;
+  const int x0 = bx * BX, y0 = BV * by, vx0 = BV * bvx, vy0 = BV * bvy;
   const int tid = threadIdx.x;
   const double S = scl[0];
   for (int i = tid; i < NREG; i += NT) reg[i] = 0ull;
   __syncthreads();
-  const int lx = tid % BX, r = tid / BX;
-  const int ix = x0 + lx, iy = y0 + (r & 1), ivx = vx0 + ((r >> 1) & 1), ivy = vy0 + (r >> 2);
   const C4Pitch cp = c4_pitch(N0, N1, N2);
   const long S1 = cp.s1, S2 = cp.s2, S3 = cp.s3;
-  if (ix < N0 && iy < N1 && ivx < N2 && ivy < N3) {
+  for (int cell = tid; cell < BX * BV * BV * BV; cell += NT) {
+    const int lx = cell % BX, r = cell / BX;
+    const int ix = x0 + lx, iy = y0 + r % BV, ivx = vx0 + r / BV % BV, ivy = vy0 + r / (BV * BV);
+    if (ix >= N0 || iy >= N1 || ivx >= N2 || ivy >= N3) continue;
     const long t = ix + (long)N0 * (iy + (long)N1 * (ivx + (long)N2 * ivy));
     const double gv = gin[t];
     const double x = g.minPhy[0] + ix * g.dx[0], y = g.minPhy[1] + iy * g.dx[1];
@@ -252,13 +256,16 @@ __global__ __launch_bounds__(8 * BX) void k_adj_advect4d_blk(const double *__res
   __syncthreads();
   // the region to global memory: region position (r0, r1, r2, r3) is the
   // coefficient at position (x0 - 2 + r0, ...), storage index + 3 per
-  // dimension; only entries some cell reached are nonzero
-  for (int i = tid; i < NREG; i += NT) {
-    const unsigned long long v = reg[i];
-    if (v != 0ull) {
-      const int q0 = i % RX, q1 = (i / RX) % RY, q2 = (i / (RX * RY)) % RV, q3 = i / (RX * RY * RV);
-      const long o = (x0 + 1 + q0) + S1 * (y0 + 1 + q1) + S2 * (vx0 + 1 + q2) + S3 * (long)(vy0 + 1 + q3);
-      atomicAdd(lc4 + o, v);
+  // dimension; only entries some cell reached are nonzero.  A wave takes a
+  // row at a time.
+  const int lane = tid & 63;
+  for (int row = tid >> 6; row < RY * RV * RV; row += NT >> 6) {
+    const int q1 = row % RY, q2 = row / RY % RV, q3 = row / (RY * RV);
+    unsigned long long *dst =
+        lc4 + ((x0 + 1) + S1 * (y0 + 1 + q1) + S2 * (vx0 + 1 + q2) + S3 * (long)(vy0 + 1 + q3));
+    if (lane < RX) {
+      const unsigned long long v = reg[row * RX + lane];
+      if (v != 0ull) atomicAdd(dst + lane, v);
     }
   }
 }
@@ -268,7 +275,9 @@ __global__ __launch_bounds__(8 * BX) void k_adj_advect4d_blk(const double *__res
 // S = 2^(50 - e) with max|g| < 2^e, and 1/S.
 __global__ __launch_bounds__(256) void k_absmax_bits(const double *__restrict__ gin, long n,
                                                      unsigned long long *__restrict__ mx) {
+  __shared__ unsigned long long sh[4];
   unsigned long long m = 0ull;
+#pragma unroll 4
   for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
     const unsigned long long b = (unsigned long long)__double_as_longlong(fabs(gin[t]));
     m = b > m ? b : m;
@@ -277,7 +286,12 @@ __global__ __launch_bounds__(256) void k_absmax_bits(const double *__restrict__ 
     const unsigned long long o = __shfl_down(m, off, 64);
     m = o > m ? o : m;
   }
-  if ((threadIdx.x & 63) == 0) atomicMax(mx, m);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {  // one atomic per workgroup: they all meet at one address
+    for (int w = 1; w < 4; w++) m = sh[w] > m ? sh[w] : m;
+    atomicMax(mx, m);
+  }
 }
 __global__ void k_fixed_zero(unsigned long long *__restrict__ mx) {
   if (threadIdx.x == 0) *mx = 0ull;
@@ -600,13 +614,23 @@ __global__ __launch_bounds__(256) void k_add_density_adj(const double *__restric
 }
 
 // out(x, y) = sum_{vx, vy} w(vx, vy) in(x, y, vx, vy), summed in a fixed order.
-__global__ __launch_bounds__(256) void k_vmoment(const double *__restrict__ in, const double *__restrict__ w, long nxy,
-                                                 long nv, double *__restrict__ out) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nxy) return;
+__global__ __launch_bounds__(1024) void k_vmoment(const double *__restrict__ in, const double *__restrict__ w, long nxy,
+                                                  long nv, double *__restrict__ out) {
+  // 64 points by 16 parts of the velocities (one lane per point ran 0.55 ms at
+  // 48^4, bound by the latency of its nv loads)
+  __shared__ double sh[16][64];
+  const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
+  const long t = (long)blockIdx.x * 64 + lane;
   double s = 0.;
-  for (long v = 0; v < nv; v++) s += w[v] * in[t + nxy * v];
-  out[t] = s;
+  if (t < nxy)
+#pragma unroll 8
+    for (long v = part; v < nv; v += 16) s += w[v] * in[t + nxy * v];
+  sh[part][lane] = s;
+  __syncthreads();
+  if (part == 0 && t < nxy) {
+    for (int p = 1; p < 16; p++) s += sh[p][lane];
+    out[t] = s;
+  }
 }
 
 void launch_scale_pairs(const double *exy, double scale, long n, double *lE, hipStream_t s) {
@@ -619,19 +643,21 @@ void launch_add_density_adj(const double *lrho, double scale, long nxy, long nce
 }
 
 void launch_vmoment(const double *in, const double *w, long nxy, long nv, double *out, hipStream_t s) {
-  hipLaunchKernelGGL(k_vmoment, dim3((unsigned)((nxy + 255) / 256)), dim3(256), 0, s, in, w, nxy, nv, out);
+  hipLaunchKernelGGL(k_vmoment, dim3((unsigned)((nxy + 63) / 64)), dim3(1024), 0, s, in, w, nxy, nv, out);
 }
 
-template <int BX>
+template <int BV>
 static void launch_adj_blk(const Geom &g, const double *c4, const double *ex, const double *ey, double dt,
                            const double *gin, double *lc4, double *axy, const double *scl, bool field_term,
                            hipStream_t s) {
-  const size_t lds = sizeof(unsigned long long) * (size_t)(BX + 4) * 6 * 6 * 6;
-  const void *fn = (const void *)k_adj_advect4d_blk<BX>;
-  (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  const long nb = (long)((g.n[0] + BX - 1) / BX) * ((g.n[1] + 1) / 2) * ((g.n[2] + 1) / 2) * ((g.n[3] + 1) / 2);
-  hipLaunchKernelGGL(k_adj_advect4d_blk<BX>, dim3((unsigned)nb), dim3(8 * BX), lds, s, c4, ex, ey, g,
-                     feet_consts(g), dt, gin, (unsigned long long *)lc4, axy, scl, field_term ? 1 : 0);
+  // x extents of up to 32, equal ones where N0 is not a multiple
+  const int nbx = (g.n[0] + 31) / 32, BX = (g.n[0] + nbx - 1) / nbx;
+  const size_t lds = (size_t)(BX + 4) * (BV + 4) * (BV + 4) * (BV + 4) * sizeof(unsigned long long);
+  const void *fn = (const void *)k_adj_advect4d_blk<BV>;
+  if (lds > 64 * 1024) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  const long nb = (long)nbx * ((g.n[1] + BV - 1) / BV) * ((g.n[2] + BV - 1) / BV) * ((g.n[3] + BV - 1) / BV);
+  hipLaunchKernelGGL(k_adj_advect4d_blk<BV>, dim3((unsigned)nb), dim3(BV == 4 ? 512 : 256), lds, s, c4, ex, ey, g,
+                     feet_consts(g), dt, gin, (unsigned long long *)lc4, axy, scl, field_term ? 1 : 0, BX);
 }
 
 bool adj_blocked() {
@@ -652,8 +678,11 @@ void launch_adj_advect4d(const Geom &g, const double *c4, const double *ex, cons
     hipLaunchKernelGGL(k_fixed_zero, dim3(1), dim3(64), 0, s, mx);
     hipLaunchKernelGGL(k_absmax_bits, dim3(1024), dim3(256), 0, s, gin, n, mx);
     hipLaunchKernelGGL(k_fixed_scale, dim3(1), dim3(64), 0, s, (const unsigned long long *)mx, wk->scl);
-    if (g.n[0] % 64 == 0) launch_adj_blk<64>(g, c4, ex, ey, dt, gin, lc4, wk->axy, wk->scl, field_term, s);
-    else launch_adj_blk<32>(g, c4, ex, ey, dt, gin, lc4, wk->axy, wk->scl, field_term, s);
+    // 4^3 blocks when they give every CU two workgroups to run in turn (one
+    // fits at a time), else 2^3
+    const long big = (long)((g.n[0] + 31) / 32) * (g.n[1] / 4) * (g.n[2] / 4) * (g.n[3] / 4);
+    if (big >= 512) launch_adj_blk<4>(g, c4, ex, ey, dt, gin, lc4, wk->axy, wk->scl, field_term, s);
+    else launch_adj_blk<2>(g, c4, ex, ey, dt, gin, lc4, wk->axy, wk->scl, field_term, s);
     if (field_term) {
       const long np = (long)g.n[0] * g.n[1] * g.n[3], ne = (long)g.n[0] * g.n[1];
       hipLaunchKernelGGL(k_adjE_x, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, s, wk->axy, g, dt, wk->part);
