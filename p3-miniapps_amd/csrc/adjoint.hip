@@ -133,9 +133,12 @@ __device__ __forceinline__ unsigned long long to_fixed(double x) {
 // the derivative of the interpolation along the foot, times d foot / d E-bar --
 // is written to axy, for the E gathers below.
 //
-// Bound: the flush's device atomics and the latency of 2 waves per SIMD (LDS
-// and registers).  BV = 4 flushes 3 times fewer entries than BV = 2 (29 per
-// cell): 48^4 2.02 -> 1.30 ms.
+// Bound: the 256 LDS atomics per cell at 2 waves per SIMD (LDS and registers).
+// BV = 4 flushes 3 times fewer entries than BV = 2 (29 per cell): 48^4 2.02 ->
+// 1.30 ms.  The coefficients of the foot term are loaded 16 at a time, one
+// (vx, vy) point ahead of the atomics that hide them: 1.30 -> 0.81 ms (they
+// took 0.54 ms while each was loaded where it was used; from an LDS copy of
+// the region, which needs a second pass over the cells, 1.38 ms).
 template <int BV>
 __global__ __launch_bounds__(512) void k_adj_advect4d_blk(const double *__restrict__ c4,
                                                           const double *__restrict__ ex,
@@ -201,34 +204,52 @@ __global__ __launch_bounds__(512) void k_adj_advect4d_blk(const double *__restri
       double gw0[4];
 #pragma unroll
       for (int k0 = 0; k0 < 4; k0++) gw0[k0] = gv * S * w[0][k0];
+      // the 4 x 4 coefficients of the next (vx, vy) point are loaded while this
+      // one's 16 contributions go to LDS
+      double cv[4][4], cn[4][4];
+      auto load = [&](int k2, int k3, double (&c)[4][4]) {
+        const double *q = c4 + base + S2 * k2 + S3 * k3;
+#pragma unroll
+        for (int k1 = 0; k1 < 4; k1++)
+#pragma unroll
+          for (int k0 = 0; k0 < 4; k0++) c[k1][k0] = q[S1 * k1 + k0];
+      };
+      if (field_term) load(0, 0, cv);
+#pragma unroll
       for (int k3 = 0; k3 < 4; k3++) {
         double v = 0., vd0 = 0., vd1 = 0., vd2 = 0.;
+#pragma unroll
         for (int k2 = 0; k2 < 4; k2++) {
-          double u = 0., ud0 = 0., ud1 = 0.;
+          if (field_term && 4 * k3 + k2 < 15) load((k2 + 1) & 3, k3 + (k2 + 1) / 4, cn);
+          __builtin_amdgcn_sched_barrier(0);
           const double w23 = w[2][k2] * w[3][k3];
+          if (inreg) {
+            unsigned long long *lrow = reg + (((r3 + k3) * RV + (r2 + k2)) * RY + r1) * RX + r0;
+#pragma unroll
+            for (int k1 = 0; k1 < 4; k1++)
+#pragma unroll
+              for (int k0 = 0; k0 < 4; k0++) atomicAdd(lrow + k1 * RX + k0, to_fixed(gw0[k0] * (w[1][k1] * w23)));
+          } else {
+            unsigned long long *grow = lc4 + base + S2 * k2 + S3 * k3;
+#pragma unroll
+            for (int k1 = 0; k1 < 4; k1++)
+#pragma unroll
+              for (int k0 = 0; k0 < 4; k0++) atomicAdd(grow + S1 * k1 + k0, to_fixed(gw0[k0] * (w[1][k1] * w23)));
+          }
+          if (!field_term) continue;
+          double u = 0., ud0 = 0., ud1 = 0.;
 #pragma unroll
           for (int k1 = 0; k1 < 4; k1++) {
-            const double w123 = w[1][k1] * w23;
-            const int lrow = ((r3 + k3) * RV + (r2 + k2)) * RY + (r1 + k1);
-            const long orow = base + S1 * k1 + S2 * k2 + S3 * k3;
+            double s0 = 0., sd = 0.;
 #pragma unroll
             for (int k0 = 0; k0 < 4; k0++) {
-              const unsigned long long q = to_fixed(gw0[k0] * w123);
-              if (inreg) atomicAdd(reg + lrow * RX + r0 + k0, q);
-              else atomicAdd(lc4 + orow + k0, q);
+              s0 += w[0][k0] * cv[k1][k0];
+              sd += dw[0][k0] * cv[k1][k0];
+              cv[k1][k0] = cn[k1][k0];
             }
-            if (field_term) {
-              double s0 = 0., sd = 0.;
-#pragma unroll
-              for (int k0 = 0; k0 < 4; k0++) {
-                const double cv = c4[orow + k0];
-                s0 += w[0][k0] * cv;
-                sd += dw[0][k0] * cv;
-              }
-              u += w[1][k1] * s0;
-              ud0 += w[1][k1] * sd;
-              ud1 += dw[1][k1] * s0;
-            }
+            u += w[1][k1] * s0;
+            ud0 += w[1][k1] * sd;
+            ud1 += dw[1][k1] * s0;
           }
           v += w[2][k2] * u;
           vd0 += w[2][k2] * ud0;
