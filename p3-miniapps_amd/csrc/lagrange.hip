@@ -5,12 +5,10 @@
 // of the result and the FFT Poisson solve (field.hip, shared with the spline
 // path), 1-D advections along vx and vy by dt (displacement dt*E(x, y)), and x,
 // y by dt/2 again.  Every advection is the 6-point order-5 interpolation of
-// VO/advect.hpp:72-86 on a periodic axis (velocity too).  Each pass streams f
-// once (8 B read + 8 B write per cell in FP64): lanes run along x, so the six
-// stencil reads of every lane are coalesced rows that stay in L2 between
-// neighbouring lanes, lines or planes.  Each lane computes its stencil (the
-// fmod/floor foot and the six weights) once and applies it along the axis the
-// weights do not depend on.
+// VO/advect.hpp:72-86 on a periodic axis (velocity too).  The x and
+// y passes go through an LDS-resident (x, y) plane, the velocity passes through
+// LDS rows of vx and register windows of vy, so a step in a run of steps
+// streams f twice (8 B read + 8 B write per cell each).
 #include <cstdlib>
 
 #include "device_common.hpp"
@@ -122,50 +120,102 @@ __global__ __launch_bounds__(256) void k_lag_y(const double *__restrict__ in, do
   if (rho_part) rho_part[t] = sum;
 }
 
-// advect_1D_vx / _vy (VO/advect.hpp:206-301): displacement dt*E(x, y) along
-// velocity axis D (2 or 3).  Lane per (x, y, other velocity), x fastest; the
-// lane runs along the advected axis.  The shift dt*E is the same for the
-// whole line, so the foot of point iv is that of point 0 moved by iv cells:
-// one set of weights, and a window of six values that slides by one load per
-// output (the reference recomputes the foot per point; the two agree to
-// rounding, and where rounding moves a foot across a node the interpolant,
-// continuous there, gives the same value).
-template <int D>
-__global__ __launch_bounds__(256) void k_lag_v(const double *__restrict__ in, double *__restrict__ out, Geom g,
-                                               const double *__restrict__ e, double dt) {
-  const int N0 = g.n[0], N1 = g.n[1], N2 = g.n[2], N3 = g.n[3];
-  const int ND = D == 2 ? N2 : N3, NO = D == 2 ? N3 : N2;  // advected axis, other axis
-  const unsigned t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  const unsigned plane = (unsigned)N0 * N1;
-  if (t >= plane * NO) return;
-  const unsigned pxy = t % plane;
-  const int io = (int)(t / plane);
+// advect_1D_vx then advect_1D_vy (VO/advect.hpp:206-301), displacements
+// dt*E(x, y) along the velocity axes, in one pass over f.  A shift is the same
+// for a whole line, so the foot of point iv is that of point 0 moved by iv
+// cells: one set of weights per (x, y) point and axis, and a window of six
+// values that slides by one per output (the reference recomputes the foot per
+// point; the two agree to rounding, and where rounding moves a foot across a
+// node the interpolant, continuous there, gives the same value).
+//
+// A workgroup takes WP points of the (x, y) plane, all of vx and a segment of
+// len rows of vy; a lane one point, S consecutive vx and the segment's rows in
+// turn.  A row's values go through LDS (two buffers, one barrier a row) for the
+// vx pass, whose results enter the lane's windows of six rows for the vy pass,
+// while the next row's values are in flight.  The rows that a wave reads may
+// differ from lane to lane, as the shifts do.
+//
+// Bound: HBM (16 bytes per cell and 5 rows' halo per segment; 0.91 ms at 128^4
+// at the 4.7 TB/s of a large copy).  WP = 16 points are one 128-byte line of
+// every (vx, vy) row, S = 4 keeps the windows within 4 waves per SIMD.  128^4
+// 0.87 ms, 1.69 ms as a pass per axis; 48^4 23 us (34), 100 x 91 x 77 x 64
+// 0.24 ms (0.33).
+constexpr int VV_WP = 16, VV_S = 4;
+
+template <int WP, int S>
+__global__ __launch_bounds__(1024) void k_lag_vv(const double *__restrict__ in, double *__restrict__ out, Geom g,
+                                                const double *__restrict__ ex, const double *__restrict__ ey,
+                                                double dt, int len, int nseg) {
+  extern __shared__ double rows[];  // two rows of N2 x WP
+  const int N2 = g.n[2], N3 = g.n[3];
+  const unsigned P = (unsigned)g.n[0] * g.n[1];
+  const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
+  const int k0 = (int)(blk % nseg) * len, k1 = min(N3, k0 + len);
+  const int l = threadIdx.x % WP;
+  const unsigned at = (blk / nseg) * WP + l, pxy = min(at, P - 1);
+  const int vx0 = (threadIdx.x / WP) * S;  // (lanes past the plane or the vx axis repeat its last point)
+  const int nv = at < P ? min(S, max(0, N2 - vx0)) : 0;  // results to store
+  double c2[6], c3[6];
   int j[6];
-  double c[6];
-  lag_stencil(g, D, g.minPhy[D], dt * e[pxy], j, c);
-  // strides (in cells) of the advected and the other velocity axes
-  const size_t sD = D == 2 ? plane : (size_t)plane * N2, sO = D == 2 ? (size_t)plane * N2 : plane;
-  const double *src = in + pxy + (size_t)io * sO;
-  double *dst = out + pxy + (size_t)io * sO;
-  double w0 = src[(size_t)j[0] * sD], w1 = src[(size_t)j[1] * sD], w2 = src[(size_t)j[2] * sD];
-  double w3 = src[(size_t)j[3] * sD], w4 = src[(size_t)j[4] * sD], w5 = src[(size_t)j[5] * sD];
-  int nxt = j[5];  // index of the window's last point
-#pragma unroll 8
-  for (int iv = 0; iv < ND; iv++) {
-    double s = c[0] * w0;
-    s += c[1] * w1;
-    s += c[2] * w2;
-    s += c[3] * w3;
-    s += c[4] * w4;
-    s += c[5] * w5;
-    dst[(size_t)iv * sD] = s;
-    nxt = nxt + 1 == ND ? 0 : nxt + 1;
-    w0 = w1;
-    w1 = w2;
-    w2 = w3;
-    w3 = w4;
-    w4 = w5;
-    w5 = src[(size_t)nxt * sD];
+  lag_stencil(g, 2, g.minPhy[2], dt * ex[pxy], j, c2);
+  int q0 = j[0] + min(vx0, N2 - 1);
+  q0 = q0 >= N2 ? q0 - N2 : q0;
+  lag_stencil(g, 3, g.minPhy[3], dt * ey[pxy], j, c3);
+  int r = (j[0] + k0) % N3;  // the row to load next
+  unsigned o[S];
+#pragma unroll
+  for (int i = 0; i < S; i++) o[i] = pxy + (unsigned)min(vx0 + i, N2 - 1) * P;
+  const size_t sR = (size_t)P * N2;
+  double v[S], w[S][6];
+  auto load = [&] {
+    const double *src = in + (size_t)r * sR;
+#pragma unroll
+    for (int i = 0; i < S; i++) v[i] = src[o[i]];
+    r = r + 1 == N3 ? 0 : r + 1;
+  };
+#pragma unroll
+  for (int i = 0; i < S; i++)
+#pragma unroll
+    for (int m = 0; m < 6; m++) w[i][m] = 0.;
+  load();
+  double *dst = out + (size_t)k0 * sR;
+  for (int k = k0 - 5; k < k1; k++) {
+    double *buf = rows + ((k - k0) & 1) * N2 * WP;
+#pragma unroll
+    for (int i = 0; i < S; i++)
+      if (vx0 + i < N2) buf[(vx0 + i) * WP + l] = v[i];
+    __syncthreads();
+    if (k + 1 < k1) load();
+    {
+      int q = q0;
+      double u[6];
+#pragma unroll
+      for (int m = 0; m < 5; m++) {
+        u[m] = buf[q * WP + l];
+        q = q + 1 == N2 ? 0 : q + 1;
+      }
+#pragma unroll
+      for (int i = 0; i < S; i++) {
+        u[(5 + i) % 6] = buf[q * WP + l];
+        q = q + 1 == N2 ? 0 : q + 1;
+        double s = c2[0] * u[i % 6];
+#pragma unroll
+        for (int m = 1; m < 6; m++) s += c2[m] * u[(i + m) % 6];
+#pragma unroll
+        for (int m = 0; m < 5; m++) w[i][m] = w[i][m + 1];
+        w[i][5] = s;
+      }
+    }
+    if (k >= k0) {
+#pragma unroll
+      for (int i = 0; i < S; i++) {
+        double s = c3[0] * w[i][0];
+#pragma unroll
+        for (int m = 1; m < 6; m++) s += c3[m] * w[i][m];
+        if (i < nv) dst[o[i]] = s;
+      }
+      dst += sR;
+    }
   }
 }
 
@@ -502,10 +552,22 @@ void launch_lag_y(const Geom &g, const double *in, double *out, double dt, doubl
   hipLaunchKernelGGL(k_lag_y, dim3(blocks(n)), dim3(256), 0, s, in, out, g, dt, rho_part);
 }
 
-void launch_lag_v(const Geom &g, int d, const double *in, double *out, const double *e, double dt, hipStream_t s) {
-  const long n = (long)g.n[0] * g.n[1] * g.n[d == 2 ? 3 : 2];
-  if (d == 2) hipLaunchKernelGGL(k_lag_v<2>, dim3(blocks(n)), dim3(256), 0, s, in, out, g, e, dt);
-  else hipLaunchKernelGGL(k_lag_v<3>, dim3(blocks(n)), dim3(256), 0, s, in, out, g, e, dt);
+void launch_lag_vv(const Geom &g, const double *in, double *out, const double *ex, const double *ey, double dt,
+                   hipStream_t s) {
+  // (an axis has at most 251 points: nt <= 1024, 32-bit offsets in a row)
+  const long P = (long)g.n[0] * g.n[1], nchunk = (P + VV_WP - 1) / VV_WP;
+  const int nt = (VV_WP * ((g.n[2] + VV_S - 1) / VV_S) + 63) / 64 * 64;
+  // 16 rows a segment: a segment loads five rows more than it has, but
+  // workgroups on far-apart rows read HBM better than all on one row after the
+  // other (128^4: one segment 1.02 ms, 8 rows 0.91, 16 rows 0.87, 32 rows
+  // 0.96).  Fewer where the launch would have under two waves per SIMD (32^4:
+  // 16 rows 19 us, 2 rows 13 us; 16 x 16 x 200 x 200, enough waves with 16
+  // rows: 43 us, 8 rows 49 us).
+  int len = 16;
+  while (len > 2 && nchunk * ((g.n[3] + len - 1) / len) * (nt / 64) < 2048) len /= 2;
+  const int nseg = (g.n[3] + len - 1) / len;
+  hipLaunchKernelGGL((k_lag_vv<VV_WP, VV_S>), dim3((unsigned)(nchunk * nseg)), dim3(nt),
+                     2 * sizeof(double) * VV_WP * g.n[2], s, in, out, g, ex, ey, dt, len, nseg);
 }
 
 }  // namespace vlp

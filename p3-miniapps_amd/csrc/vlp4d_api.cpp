@@ -405,8 +405,8 @@ int lag_steps(vlp_ctx *c, int nsteps) {
     int rc = field(c, c->iter + 1, true, false);
     if (rc) return rc;
     HIP_TRY(c, hipEventRecord(ev[1], s));
-    vlp::launch_lag_v(g, 2, (double *)c->f, (double *)c->fnext, c->fb.ex, dt, s);
-    vlp::launch_lag_v(g, 3, (double *)c->fnext, (double *)c->f, c->fb.ey, dt, s);
+    vlp::launch_lag_vv(g, (double *)c->f, (double *)c->fnext, c->fb.ex, c->fb.ey, dt, s);
+    std::swap(c->f, c->fnext);
     HIP_TRY(c, hipEventRecord(ev[2], s));
     const bool last = n + 1 == nsteps;
     xy(!last, !last);

@@ -159,7 +159,9 @@ int kernel_variants(const Geom &g, bool fp32_storage, bool arith32);
 void launch_lag_init(const Geom &g, double *f, hipStream_t s);
 void launch_lag_x(const Geom &g, const double *in, double *out, double dt, hipStream_t s);
 void launch_lag_y(const Geom &g, const double *in, double *out, double dt, double *rho_part, hipStream_t s);
-void launch_lag_v(const Geom &g, int d, const double *in, double *out, const double *e, double dt, hipStream_t s);
+// vx then vy in one pass, from in to out
+void launch_lag_vv(const Geom &g, const double *in, double *out, const double *ex, const double *ey, double dt,
+                   hipStream_t s);
 // Fused x/2 + y/2 (one pass over f) when the (x, y) plane fits in LDS:
 // lag_xy_chunks gives the vx runs per vy, 0 when not eligible;
 // launch_lag_xy returns false for nchunk 0.  twice: the pair two times over
