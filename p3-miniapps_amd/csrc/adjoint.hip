@@ -338,60 +338,105 @@ __global__ void k_fixed_scale(const unsigned long long *__restrict__ mx, double 
 // with d = -dt vx / (2 dx) up to rounding, so x is one of five candidates,
 // each checked exactly; then for every node (jx, jy) the same over (y, vy)
 // with cy.
-__global__ __launch_bounds__(256) void k_adjE_x(const double *__restrict__ axy, Geom g, double dt,
-                                                double *__restrict__ part) {
+//
+// Bound: latency and the candidates' arithmetic.  Shifts are reduced modulo
+// the axis once per velocity (uniform), not per candidate, and the velocity
+// sums are split over ADJE_PARTS waves of a workgroup and added in order:
+// 48^4 k_adjE_x 48 us (113 us), k_adjE_y 15 us (93 us; one wave per 64 nodes).
+constexpr int ADJE_PARTS = 8;
+
+// Quadratic weight of node ip + k at p = x - ip.
+__device__ __forceinline__ double node_weight(double p, int k) {
+  return k == 0 ? .5 * (p - 1.) * (p - 2.) : k == 1 ? -1. * (p) * (p - 2.) : .5 * (p) * (p - 1.);
+}
+// r in [0, N) for q within one N of it
+__device__ __forceinline__ int wrap1(int q, int N) { return q < 0 ? q + N : q >= N ? q - N : q; }
+
+// Lane (64 per workgroup and part) per (jx, y, vy); node j and axis length N of
+// the gather along it; foot(i, v) the displaced position of point i in cells,
+// visit(i, v, weight) in ascending candidate order for every velocity v of the
+// part.  base: round(-dt v / (2 dx)) - 1.
+template <typename B, typename F, typename V>
+__device__ __forceinline__ void gather_nodes(int j, int N, int nv, int part, B base, F foot, V visit) {
+  for (int v = part * nv / ADJE_PARTS; v < (part + 1) * nv / ADJE_PARTS; v++) {
+    const int sh = base(v);
+    int red = sh % N;  // (uniform)
+    if (red < 0) red += N;
+    const int turns = sh - red;  // a multiple of N
+#pragma unroll
+    for (int q = -3; q <= 1; q++) {
+      const int i = wrap1(wrap1(j - red + q, N), N);
+      const double xt = foot(i, v);
+      const int ip = (int)(round(xt) - 1);
+      // (j - ip) mod N: ip + 3 N > j > ip - 3 N after the turns are taken out
+      const int k = wrap1(wrap1(wrap1(j - (ip - turns), N), N), N);
+      if ((unsigned)k <= 2u) visit(i, v, node_weight(xt - ip, k));
+    }
+  }
+}
+
+__global__ __launch_bounds__(64 * ADJE_PARTS) void k_adjE_x(const double *__restrict__ axy, Geom g, double dt,
+                                                            double *__restrict__ part) {
+  __shared__ double2 sh[ADJE_PARTS][64];
   const int N0 = g.n[0], N1 = g.n[1], N2 = g.n[2], N3 = g.n[3];
   const long n = (long)N0 * N1 * N3;
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int jx = (int)(t % N0), iy = (int)((t / N0) % N1), ivy = (int)(t / ((long)N0 * N1));
+  const int lane = threadIdx.x & 63, pt = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long t = (long)blockIdx.x * 64 + lane, tc = t < n ? t : n - 1;
+  const int jx = (int)(tc % N0), iy = (int)((tc / N0) % N1), ivy = (int)(tc / ((long)N0 * N1));
+  const double2 *src = (const double2 *)axy + (long)N0 * (iy + (long)N1 * N2 * ivy);
   double sx = 0., sy = 0.;
-  for (int ivx = 0; ivx < N2; ivx++) {
-    const double vx = g.minPhy[2] + ivx * g.dx[2];
-    const int sh = (int)round(-0.5 * dt * vx * g.inv_dx[0]) - 1;
-    for (int q = -3; q <= 1; q++) {
-      const int ix = ((jx - sh + q) % N0 + N0) % N0;
-      double xt0 = (g.minPhy[0] + ix * g.dx[0]) - 0.5 * dt * vx;
-      xt0 = g.inv_dx[0] * (xt0 - g.minPhy[0]);
-      const int ip0 = (int)(round(xt0) - 1);
-      const int k0 = ((jx - ip0) % N0 + N0) % N0;
-      if (k0 > 2) continue;
-      const double px = xt0 - ip0;
-      const double cx = k0 == 0 ? .5 * (px - 1.) * (px - 2.) : k0 == 1 ? -1. * (px) * (px - 2.) : .5 * (px) * (px - 1.);
-      const long c = ix + (long)N0 * (iy + (long)N1 * (ivx + (long)N2 * ivy));
-      sx += cx * axy[2 * c];
-      sy += cx * axy[2 * c + 1];
+  gather_nodes(
+      jx, N0, N2, pt,
+      [&](int v) { return (int)round(-0.5 * dt * (g.minPhy[2] + v * g.dx[2]) * g.inv_dx[0]) - 1; },
+      [&](int i, int v) {
+        const double xt0 = (g.minPhy[0] + i * g.dx[0]) - 0.5 * dt * (g.minPhy[2] + v * g.dx[2]);
+        return g.inv_dx[0] * (xt0 - g.minPhy[0]);
+      },
+      [&](int i, int v, double w) {
+        const double2 a = src[i + (long)N0 * N1 * v];
+        sx += w * a.x;
+        sy += w * a.y;
+      });
+  sh[pt][lane] = make_double2(sx, sy);
+  __syncthreads();
+  if (pt == 0 && t < n) {
+    for (int p = 1; p < ADJE_PARTS; p++) {
+      sx += sh[p][lane].x;
+      sy += sh[p][lane].y;
     }
+    part[2 * t] = sx;
+    part[2 * t + 1] = sy;
   }
-  part[2 * t] = sx;
-  part[2 * t + 1] = sy;
 }
-__global__ __launch_bounds__(256) void k_adjE_y(const double *__restrict__ part, Geom g, double dt,
-                                                double *__restrict__ lE) {
+__global__ __launch_bounds__(64 * ADJE_PARTS) void k_adjE_y(const double *__restrict__ part, Geom g, double dt,
+                                                            double *__restrict__ lE) {
+  __shared__ double2 sh[ADJE_PARTS][64];
   const int N0 = g.n[0], N1 = g.n[1], N3 = g.n[3];
   const long n = (long)N0 * N1;
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int jx = (int)(t % N0), jy = (int)(t / N0);
+  const int lane = threadIdx.x & 63, pt = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long t = (long)blockIdx.x * 64 + lane, tc = t < n ? t : n - 1;
+  const int jx = (int)(tc % N0), jy = (int)(tc / N0);
+  const double2 *src = (const double2 *)part + jx;
   double sx = 0., sy = 0.;
-  for (int ivy = 0; ivy < N3; ivy++) {
-    const double vy = g.minPhy[3] + ivy * g.dx[3];
-    const int sh = (int)round(-0.5 * dt * vy * g.inv_dx[1]) - 1;
-    for (int q = -3; q <= 1; q++) {
-      const int iy = ((jy - sh + q) % N1 + N1) % N1;
-      const double xt1 = half_y(g, g.minPhy[1] + iy * g.dx[1], vy, dt);
-      const int ip1 = (int)(round(xt1) - 1);
-      const int k1 = ((jy - ip1) % N1 + N1) % N1;
-      if (k1 > 2) continue;
-      const double py = xt1 - ip1;
-      const double cy = k1 == 0 ? .5 * (py - 1.) * (py - 2.) : k1 == 1 ? -1. * (py) * (py - 2.) : .5 * (py) * (py - 1.);
-      const long pidx = jx + (long)N0 * (iy + (long)N1 * ivy);
-      sx += cy * part[2 * pidx];
-      sy += cy * part[2 * pidx + 1];
+  gather_nodes(
+      jy, N1, N3, pt,
+      [&](int v) { return (int)round(-0.5 * dt * (g.minPhy[3] + v * g.dx[3]) * g.inv_dx[1]) - 1; },
+      [&](int i, int v) { return half_y(g, g.minPhy[1] + i * g.dx[1], g.minPhy[3] + v * g.dx[3], dt); },
+      [&](int i, int v, double w) {
+        const double2 a = src[(long)N0 * (i + (long)N1 * v)];
+        sx += w * a.x;
+        sy += w * a.y;
+      });
+  sh[pt][lane] = make_double2(sx, sy);
+  __syncthreads();
+  if (pt == 0 && t < n) {
+    for (int p = 1; p < ADJE_PARTS; p++) {
+      sx += sh[p][lane].x;
+      sy += sh[p][lane].y;
     }
+    lE[2 * t] = sx;
+    lE[2 * t + 1] = sy;
   }
-  lE[2 * t] = sx;
-  lE[2 * t + 1] = sy;
 }
 
 // out[o][n][i] (+)= sum_m Mt[n][m] in[o][m][i]: a line operator's transpose
@@ -415,11 +460,22 @@ __global__ __launch_bounds__(256) void k_axis_contract(const double *__restrict_
 // 64 consecutive o) and each wave forms 16 outputs n per pass from it, the
 // operator entries M[m][n] (M = Mt^T, Min x Nout row-major) arriving as
 // wave-uniform scalar loads.  Same sums in the same order as k_axis_contract.
+//
+// Bound: HBM for I > 1 (48^4 36 us a pass).  For I = 1 the axis is the fastest
+// index: the tile is transposed through an odd LDS pitch and a wave's outputs
+// go through LDS eight at a time, so that both sides of the pass are coalesced
+// (48^4 46 us; 74 us with a lane's outputs stored down its own row, and
+// staging stores that all met in one bank).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 template <bool COLO>
 __global__ __launch_bounds__(256) void k_axis_contract_t(const double *__restrict__ M, int Min, int Nout,
                                                          const double *__restrict__ in, double *__restrict__ out,
                                                          long O, long I, int accumulate) {
-  extern __shared__ __align__(16) double ctile[];  // [Min][64]
+  constexpr int CP = COLO ? 65 : 64;
+  extern __shared__ __align__(16) double ctile[];  // [Min][CP], then for COLO 8 x CP per wave
   const int tid = threadIdx.x, c = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   long o0, i0;
@@ -437,7 +493,7 @@ __global__ __launch_bounds__(256) void k_axis_contract_t(const double *__restric
   if (COLO) {
     for (int e = tid; e < 64 * Min; e += 256) {
       const int cc = e / Min, m = e - cc * Min;
-      ctile[m * 64 + cc] = cc < ncol ? in[(o0 + cc) * Min + m] : 0.;
+      ctile[m * CP + cc] = cc < ncol ? in[o0 * Min + e] : 0.;
     }
   } else {
     const double *src = in + o0 * Min * I + i0;
@@ -454,25 +510,42 @@ __global__ __launch_bounds__(256) void k_axis_contract_t(const double *__restric
     for (int j = 0; j < 16; j++) acc[j] = 0.;
     if (jmax == 16) {  // whole chunk: 16 consecutive entries per m, loaded together
       for (int m = 0; m < Min; m++) {
-        const double x = ctile[m * 64 + c];
+        const double x = ctile[m * CP + c];
         const double *mr = M + (long)m * Nout + n0;
 #pragma unroll
         for (int j = 0; j < 16; j++) acc[j] += mr[j] * x;
       }
     } else {
       for (int m = 0; m < Min; m++) {
-        const double x = ctile[m * 64 + c];
+        const double x = ctile[m * CP + c];
         const double *mr = M + (long)m * Nout + n0;
 #pragma unroll
         for (int j = 0; j < 16; j++)
           if (j < jmax) acc[j] += mr[j] * x;
       }
     }
-    if (c < ncol) {
+    if (COLO) {
+      double *ot = ctile + Min * CP + wv * 8 * CP;
+#pragma unroll
+      for (int h = 0; h < 16; h += 8) {
+        wave_lds_fence();  // (the previous eight are read)
+#pragma unroll
+        for (int j = 0; j < 8; j++) ot[j * CP + c] = acc[h + j];
+        wave_lds_fence();
+        // eight lanes a row of eight outputs
+        const int j = c & 7;
+        if (h + j < jmax)
+          for (int cc = c >> 3; cc < ncol; cc += 8) {
+            const long idx = (o0 + cc) * Nout + n0 + h + j;
+            const double v = ot[j * CP + cc];
+            out[idx] = accumulate ? out[idx] + v : v;
+          }
+      }
+    } else if (c < ncol) {
 #pragma unroll
       for (int j = 0; j < 16; j++)
         if (j < jmax) {
-          const long idx = COLO ? (o0 + c) * Nout + n0 + j : (o0 * Nout + n0 + j) * I + i0 + c;
+          const long idx = (o0 * Nout + n0 + j) * I + i0 + c;
           out[idx] = accumulate ? out[idx] + acc[j] : acc[j];
         }
     }
@@ -565,57 +638,70 @@ __global__ __launch_bounds__(256) void k_adj_advect2d(const double *__restrict__
 // [X - 5 - floor(d), X - floor(d)]; each candidate's jx0 and weights are
 // recomputed exactly as the scatter (and the forward) computes them, and
 // likewise in y.  No atomics: the result does not depend on scheduling.
+//
+// The y sums depend on (ix, Y, vy) only and the x weights on (X, vx): a
+// workgroup takes ADJ2_Y rows of one vy, forms their y sums in LDS and runs
+// through its part of the vx, a lane with one column and all the rows.
+// Bound: the writes of lcxy and the weights' arithmetic; 48^4 24 us (104 us
+// with a lane per entry that formed both).
+constexpr int ADJ2_Y = 8;
+
+// Candidate point c of column (or row) X of an axis: true if its half-step
+// stencil covers X, with the weight there.
+__device__ __forceinline__ bool half_weight(const Geom &g, int d, double dth, double v, int c, int X, double &w) {
+  if (c < 0 || c >= g.n[d]) return false;
+  const double x = g.minPhy[d] + c * g.dx[d];
+  const double f = ((x - dth * v) - g.minPhy[d]) * g.inv_dx[d];
+  const int j0 = (int)floor(f), k = X - 1 - j0;
+  if (j0 < -1 || j0 > g.n[d] - 1 || k < 0 || k > 3) return false;
+  double e[4];
+  bspline_eta<double>(f - j0, e);
+  w = k == 0 ? e[0] : k == 1 ? e[1] : k == 2 ? e[2] : e[3];
+  return true;
+}
+
 __global__ __launch_bounds__(256) void k_adj_advect2d_g(const double *__restrict__ lrho, Geom g, double dth,
-                                                        double *__restrict__ lcxy) {
-  const int N0 = g.n[0], N1 = g.n[1], N2 = g.n[2], N3 = g.n[3];
-  const long E0 = N0 + 4, E1 = N1 + 4;
-  const long n = E0 * E1 * N2 * N3;
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int X = (int)(t % E0), Y = (int)((t / E0) % E1);
-  const long plane = t / (E0 * E1);
-  const int ivx = (int)(plane % N2), ivy = (int)(plane / N2);
-  const double vx = g.minPhy[2] + ivx * g.dx[2], vy = g.minPhy[3] + ivy * g.dx[3];
-  const int fdx = (int)floor(-dth * vx * g.inv_dx[0]), fdy = (int)floor(-dth * vy * g.inv_dx[1]);
-  // y candidates: weight of row Y for each, 0 where it does not reach Y
-  double wy[6];
-  int iyc[6];
-#pragma unroll
-  for (int q = 0; q < 6; q++) {
-    const int iy = Y - 5 - fdy + q;
-    iyc[q] = iy;
-    wy[q] = 0.;
-    if (iy >= 0 && iy < N1) {
-      const double y = g.minPhy[1] + iy * g.dx[1];
-      const double fy = ((y - dth * vy) - g.minPhy[1]) * g.inv_dx[1];
-      const int jy0 = (int)floor(fy);
-      const int ky = Y - 1 - jy0;
-      if (jy0 >= -1 && jy0 <= N1 - 1 && ky >= 0 && ky < 4) {
-        double e[4];
-        bspline_eta<double>(fy - jy0, e);
-        wy[q] = e[ky];
-      }
-    }
-  }
-  double acc = 0.;
-#pragma unroll
-  for (int p = 0; p < 6; p++) {
-    const int ix = X - 5 - fdx + p;
-    if (ix < 0 || ix >= N0) continue;
-    const double x = g.minPhy[0] + ix * g.dx[0];
-    const double fx = ((x - dth * vx) - g.minPhy[0]) * g.inv_dx[0];
-    const int jx0 = (int)floor(fx);
-    const int kx = X - 1 - jx0;
-    if (jx0 < -1 || jx0 > N0 - 1 || kx < 0 || kx > 3) continue;
-    double e[4];
-    bspline_eta<double>(fx - jx0, e);
+                                                        double *__restrict__ lcxy, int nyt, int nvp) {
+  extern __shared__ __align__(16) double ysum[];  // [ADJ2_Y][N0]
+  const int N0 = g.n[0], N1 = g.n[1], N2 = g.n[2], E0 = N0 + 4, E1 = N1 + 4;
+  unsigned b = blockIdx.x;
+  const int vp = b % nvp;
+  b /= nvp;
+  const int Y0 = (int)(b % nyt) * ADJ2_Y, ivy = b / nyt, ny = min(ADJ2_Y, E1 - Y0);
+  const double vy = g.minPhy[3] + ivy * g.dx[3];
+  const int fdy = (int)floor(-dth * vy * g.inv_dx[1]);
+  for (int e = threadIdx.x; e < ny * N0; e += 256) {
+    const int r = e / N0, ix = e - r * N0, Y = Y0 + r;
     double sy = 0.;
 #pragma unroll
-    for (int q = 0; q < 6; q++)
-      if (wy[q] != 0.) sy += wy[q] * lrho[(long)iyc[q] * N0 + ix];
-    acc += e[kx] * sy;
+    for (int q = 0; q < 6; q++) {
+      const int iy = Y - 5 - fdy + q;
+      double w;
+      if (half_weight(g, 1, dth, vy, iy, Y, w) && w != 0.) sy += w * lrho[(long)iy * N0 + ix];
+    }
+    ysum[r * N0 + ix] = sy;
   }
-  lcxy[t] = acc * g.dx[2] * g.dx[3];
+  __syncthreads();
+  // lanes: columns, several vx at a time where a row is short
+  const int nx = 256 / E0 > 0 ? 256 / E0 : 1, sub = threadIdx.x / E0, X = threadIdx.x - sub * E0;
+  if (sub >= nx) return;
+  const int v1 = (int)((long)(vp + 1) * N2 / nvp);
+  for (int ivx = (int)((long)vp * N2 / nvp) + sub; ivx < v1; ivx += nx) {
+    const double vx = g.minPhy[2] + ivx * g.dx[2];
+    const int ix0 = X - 5 - (int)floor(-dth * vx * g.inv_dx[0]);
+    double w[6];
+    bool in[6];
+#pragma unroll
+    for (int p = 0; p < 6; p++) in[p] = half_weight(g, 0, dth, vx, ix0 + p, X, w[p]);
+    double *dst = lcxy + ((long)ivx + (long)N2 * ivy) * E0 * E1 + (long)Y0 * E0 + X;
+    for (int r = 0; r < ny; r++) {
+      double acc = 0.;
+#pragma unroll
+      for (int p = 0; p < 6; p++)
+        if (in[p]) acc += w[p] * ysum[r * N0 + ix0 + p];
+      dst[(long)r * E0] = acc * g.dx[2] * g.dx[3];
+    }
+  }
 }
 
 // Field-energy source: W(f) = dx dy sum (Ex^2 + Ey^2) of the field solved
@@ -706,8 +792,10 @@ void launch_adj_advect4d(const Geom &g, const double *c4, const double *ex, cons
     else launch_adj_blk<2>(g, c4, ex, ey, dt, gin, lc4, wk->axy, wk->scl, field_term, s);
     if (field_term) {
       const long np = (long)g.n[0] * g.n[1] * g.n[3], ne = (long)g.n[0] * g.n[1];
-      hipLaunchKernelGGL(k_adjE_x, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, s, wk->axy, g, dt, wk->part);
-      hipLaunchKernelGGL(k_adjE_y, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, s, wk->part, g, dt, lE);
+      hipLaunchKernelGGL(k_adjE_x, dim3((unsigned)((np + 63) / 64)), dim3(64 * ADJE_PARTS), 0, s, wk->axy, g, dt,
+                         wk->part);
+      hipLaunchKernelGGL(k_adjE_y, dim3((unsigned)((ne + 63) / 64)), dim3(64 * ADJE_PARTS), 0, s, wk->part, g, dt,
+                         lE);
     }
     return;
   }
@@ -721,6 +809,7 @@ void launch_axis_contract(const double *Mt, int Min, int Nout, const double *in,
   if (M) {  // tiled form (M = Mt^T)
     const size_t lds = (size_t)Min * 64 * sizeof(double);
     if (I == 1) {
+      const size_t lds = (size_t)(Min + 32) * 65 * sizeof(double);
       (void)hipFuncSetAttribute((const void *)k_axis_contract_t<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds);
       hipLaunchKernelGGL(k_axis_contract_t<true>, dim3((unsigned)((O + 63) / 64)), dim3(256), lds, s, M, Min, Nout,
@@ -752,8 +841,12 @@ void launch_adj_advect2d(const double *lrho, const Geom &g, double dth, double *
   const long n = (long)g.n[0] * g.n[1] * g.n[2] * g.n[3];
   // VLP4D_ADJ_BLOCK=0 also selects the scatter form here (lcxy zeroed by the caller)
   if (adj_blocked()) {
-    const long ng = (long)(g.n[0] + 4) * (g.n[1] + 4) * g.n[2] * g.n[3];
-    hipLaunchKernelGGL(k_adj_advect2d_g, dim3((unsigned)((ng + 255) / 256)), dim3(256), 0, s, lrho, g, dth, lcxy);
+    // vx in parts until there are four workgroups per CU
+    const int nyt = (g.n[1] + 4 + ADJ2_Y - 1) / ADJ2_Y;
+    int nvp = 1;
+    while (nvp < 8 && nyt * g.n[3] * nvp < 1024) nvp *= 2;
+    hipLaunchKernelGGL(k_adj_advect2d_g, dim3((unsigned)(nyt * g.n[3] * nvp)), dim3(256),
+                       sizeof(double) * ADJ2_Y * g.n[0], s, lrho, g, dth, lcxy, nyt, nvp);
     return;
   }
   hipLaunchKernelGGL(k_adj_advect2d, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, lrho, g, dth, lcxy);
