@@ -29,10 +29,22 @@ template <typename A> __device__ __forceinline__ void eta4(A w, A e[4]) { bsplin
 
 }  // namespace
 
-// Block of NT = 512 lanes.  x pass: line y = r0 + tid / Px, lane p = tid % Px;
+// Block of NT lanes.  x pass: line y = r0 + tid / Px, lane p = tid % Px;
 // y pass: column xc = c0 + tid / Py, lane p = tid % Py; advection: column
 // x = tid % N0, rows y0 .. y0+ylen-1 (ylen <= NPT) of segment tid / N0, the
 // density sums of those points in registers across the vx planes.
+//
+// Bound: HBM (16 bytes per cell in double; 0.94 ms at 128^4 at the 4.7 TB/s of a
+// large copy, 1.45 ms taken) and, as a plane goes through its phases between
+// barriers, the waves that hide one another's latency.  A lane with 32
+// points' sums leaves room for two waves per SIMD; with 8 (512 lanes, planes up
+// to about 64 x 64) or 16 points (1024 lanes) and no addresses held across the
+// planes there is room for four, as two workgroups or one:
+//   64^4 double 133 -> 90 us, 48^4 float 55 -> 36, 32^4 double 31 -> 17;
+//   96^4 float storage 0.41 -> 0.34 ms, 128^4 float 0.92 -> 0.82, 90 x 77 x 84 x
+//   75 float 0.36 -> 0.32.
+// The RAG form with C = 16 and over 8 points does not fit in those registers
+// (113 x 118 x 60 x 62 float 0.31 ms, with two waves per SIMD 0.28) and keeps 32.
 constexpr int XY_NT = 512, XY_NPT = 32;
 
 // RAG: lines of any length (the RAG form of the recursion, Px and Py lanes).
@@ -40,8 +52,8 @@ constexpr int XY_NT = 512, XY_NPT = 32;
 // k_advect2d_rho, three passes over the plane with one lane per line: xy
 // phases of 113 x 118 x 101 x 126 in float 2.32 -> 0.92 ms, 90 x 77 x 84 x 75
 // in double 1.17 -> 0.41, 33 x 33 x 39 x 37 0.095 -> 0.061.
-template <typename T, typename A, int C, bool RAG>
-__global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *__restrict__ cxy, Geom g, double dth,
+template <typename T, typename A, int C, bool RAG, int NT, int NPT>
+__global__ __launch_bounds__(NT, NPT > 16 ? 2 : 4) void k_xy_adv2d(const T *__restrict__ f, T *__restrict__ cxy, Geom g, double dth,
                                                    int G, double *__restrict__ rho_part, int *__restrict__ err,
                                                    SplineConsts sc, double aC, double aN3x, double aN3y, int Px_,
                                                    int Py_) {
@@ -60,16 +72,16 @@ __global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *
   const int grp = blockIdx.x % G, ivy = blockIdx.x / G;
   const int VG = (N2 + G - 1) / G, v0 = min(N2, grp * VG), v1 = min(N2, v0 + VG);
   // advection lanes
-  const int nseg = XY_NT / N0, seg = tid / N0, xi = tid - seg * N0;
+  const int nseg = NT / N0, seg = tid / N0, xi = tid - seg * N0;
   const int ylen = (N1 + nseg - 1) / nseg, y0 = seg * ylen;
   const bool aact = seg < nseg;
-  double rho[XY_NPT];
+  double rho[NPT];
 #pragma unroll
-  for (int k = 0; k < XY_NPT; k++) rho[k] = 0.;
+  for (int k = 0; k < NPT; k++) rho[k] = 0.;
   int bad = 0;
   const double vy = g.minPhy[3] + ivy * g.dx[3];
   const double xx = g.minPhy[0] + xi * g.dx[0];
-  for (int y = tid; y < N1; y += XY_NT) {
+  for (int y = tid; y < N1; y += NT) {
     const double yy = g.minPhy[1] + y * g.dx[1];
     const double fy = ((yy - dth * vy) - g.minPhy[1]) * g.inv_dx[1];
     const int jy0 = (int)floor(fy);
@@ -81,7 +93,7 @@ __global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *
   const int px = tid & (Px - 1), xl = tid / Px;
   for (int ivx = v0; ivx < v1; ivx++) {
     // 1. x recursions, rows 2..N1+1 of the plane
-    for (int r0 = 0; r0 < N1; r0 += XY_NT / Px) {
+    for (int r0 = 0; r0 < N1; r0 += NT / Px) {
       const int y = r0 + xl;
       double v[C];
       const int x0 = RAG ? min(px * C, N0 - C) : px * C;  // first point of the lane's chunk
@@ -109,8 +121,11 @@ __global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *
     // 2. y recursions on columns 0..E0-1 (a wave stops when its first
     // column is past the plane: its lines are whole within the wave)
     {
+      int R_ = R;
+      asm volatile("" : "+s"(R_));
+      const int R = R_;
       const int py = tid & (Py - 1), yl = tid / Py, yl0 = (wave * 64) / Py;
-      for (int c0 = 0; c0 + yl0 < E0; c0 += XY_NT / Py) {
+      for (int c0 = 0; c0 + yl0 < E0; c0 += NT / Py) {
         const int xc = c0 + yl;
         const bool act = xc < E0 && (!RAG || py < nly);
         double w[C];
@@ -148,9 +163,9 @@ __global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *
       constexpr int VPC = 16 / (int)sizeof(T);
       if (E0 % VPC == 0) {
         const int cpr = E0 / VPC, nch = cpr * E1;
-        const int drow = XY_NT / cpr, dcol = XY_NT - drow * cpr;
+        const int drow = NT / cpr, dcol = NT - drow * cpr;
         int row = tid / cpr, col = tid - row * cpr;
-        for (int k = tid; k < nch; k += XY_NT) {
+        for (int k = tid; k < nch; k += NT) {
           const T *s = pl + row * R + VPC * col;
           typedef T chunk_t __attribute__((ext_vector_type(VPC)));
           chunk_t v;
@@ -166,9 +181,9 @@ __global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *
         }
       } else {
         const int nch = (E0 * E1 + VPC - 1) / VPC;
-        const int drow = VPC * XY_NT / E0, dcol = VPC * XY_NT - drow * E0;
+        const int drow = VPC * NT / E0, dcol = VPC * NT - drow * E0;
         int row = VPC * tid / E0, col = VPC * tid - row * E0;
-        for (int k = tid; k < nch; k += XY_NT) {
+        for (int k = tid; k < nch; k += NT) {
           const T *s = pl + row * R + col;
           typedef T chunk_t __attribute__((ext_vector_type(VPC)));
           chunk_t v;
@@ -195,8 +210,12 @@ __global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *
       const T *pc = pl + (xbad ? 0 : jx0 + 1);  // stencil column jx0-1 at LDS column jx0+1
       A gw[4];  // x-interpolated rows jw .. jw+3 (LDS rows)
       int jw = -1000;
+      // (an opaque copy: the points' table addresses and conditions are not to be
+      // held in registers across the planes)
+      int y0v = y0;
+      asm volatile("" : "+v"(y0v));
       constexpr int GP = sizeof(A) == sizeof(float) ? 4 : 2;
-      static_assert(XY_NPT % GP == 0, "groups tile the point range");
+      static_assert(NPT % GP == 0, "groups tile the point range");
       // Points go in groups of GP consecutive y (four for float arithmetic,
       // two for double, whose tables take twice the registers).  The
       // segment's lanes share y, so jy0 and the group's path are uniform in a
@@ -206,8 +225,8 @@ __global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *
       // LDS round trip per group instead of several per point); otherwise the
       // points go one at a time.
 #pragma unroll
-      for (int k0 = 0; k0 < XY_NPT; k0 += GP) {
-        const int yg = y0 + k0;
+      for (int k0 = 0; k0 < NPT; k0 += GP) {
+        const int yg = y0v + k0;
         if (k0 < ylen && yg < N1) {
           int jr[GP];
           A ey[GP][4];
@@ -292,7 +311,7 @@ __global__ __launch_bounds__(XY_NT) void k_xy_adv2d(const T *__restrict__ f, T *
   if (aact) {
     double *rp = rho_part + ((long)grp * N3 + ivy) * N0 * N1;
 #pragma unroll
-    for (int k = 0; k < XY_NPT; k++) {
+    for (int k = 0; k < NPT; k++) {
       const int y = y0 + k;
       if (k < ylen && y < N1) rp[(long)y * N0 + xi] = rho[k];
     }
@@ -309,7 +328,8 @@ size_t xy_lds(const Geom &g, size_t tsz) {
 }
 
 // Chunk and lanes of the fused kernel for a geometry (C = 0: not eligible): the
-// plane fits in LDS, every lane owns at most XY_NPT advection points, and N0 =
+// plane fits in LDS, every lane of XY_NT owns at most XY_NPT advection points
+// (then one of 2 XY_NT at most half as many), and N0 =
 // Px C and N1 = Py C with Px, Py powers of two, or (rag) Px C and Py C cover
 // N0 and N1 with the fewest lanes.
 struct XyPlan {
@@ -359,8 +379,8 @@ int xy_fused_groups(const Geom &g, size_t tsz) {
   return G;
 }
 
-template <typename T, typename A, int C, bool RAG>
-static void launch_xy_t(const Geom &g, const T *f, T *cxy, double dth, int G, double *rho_part, int *err,
+template <typename T, typename A, int C, bool RAG, int NT, int NPT>
+static void launch_xy_n(const Geom &g, const T *f, T *cxy, double dth, int G, double *rho_part, int *err,
                         const XyPlan &p, hipStream_t s) {
   const SplineConsts sc = spline_consts();
   double aC = 1.0, aN3x = 1.0, aN3y = 1.0;
@@ -368,10 +388,19 @@ static void launch_xy_t(const Geom &g, const T *f, T *cxy, double dth, int G, do
   for (int i = 0; i < g.n[0] + 3; i++) aN3x *= sc.alpha;
   for (int i = 0; i < g.n[1] + 3; i++) aN3y *= sc.alpha;
   const size_t lds = xy_lds(g, sizeof(T));
-  const void *fn = (const void *)k_xy_adv2d<T, A, C, RAG>;
+  const void *fn = (const void *)k_xy_adv2d<T, A, C, RAG, NT, NPT>;
   if (lds > 64 * 1024) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL((k_xy_adv2d<T, A, C, RAG>), dim3((unsigned)(G * g.n[3])), dim3(XY_NT), lds, s, f, cxy, g, dth, G,
-                     rho_part, err, sc, aC, aN3x, aN3y, p.Px, p.Py);
+  hipLaunchKernelGGL((k_xy_adv2d<T, A, C, RAG, NT, NPT>), dim3((unsigned)(G * g.n[3])), dim3(NT), lds, s, f, cxy, g,
+                     dth, G, rho_part, err, sc, aC, aN3x, aN3y, p.Px, p.Py);
+}
+
+template <typename T, typename A, int C, bool RAG>
+static void launch_xy_t(const Geom &g, const T *f, T *cxy, double dth, int G, double *rho_part, int *err,
+                        const XyPlan &p, hipStream_t s) {
+  const int nseg = XY_NT / g.n[0], ylen = (g.n[1] + nseg - 1) / nseg;
+  if (ylen <= 8) launch_xy_n<T, A, C, RAG, XY_NT, 8>(g, f, cxy, dth, G, rho_part, err, p, s);
+  else if constexpr (RAG && C == 16) launch_xy_n<T, A, C, RAG, XY_NT, XY_NPT>(g, f, cxy, dth, G, rho_part, err, p, s);
+  else launch_xy_n<T, A, C, RAG, 2 * XY_NT, XY_NPT / 2>(g, f, cxy, dth, G, rho_part, err, p, s);
 }
 
 template <typename T, typename A>
