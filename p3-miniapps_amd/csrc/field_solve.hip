@@ -12,6 +12,7 @@
 // carved out of one device buffer.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstddef>
 
@@ -21,9 +22,10 @@ namespace vlp {
 namespace {
 
 // exp(-2 pi i m / n) with exact values on the axes, interleaved complex (the
-// same table the contexts build on the host).
-__global__ __launch_bounds__(256) void k_twiddles(double *tw, int n) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+// same table the contexts build on the host), for both axes (block row 0: x).
+__global__ __launch_bounds__(256) void k_twiddles(double *twx, int nx, double *twy, int ny) {
+  double *tw = blockIdx.y == 0 ? twx : twy;
+  const int n = blockIdx.y == 0 ? nx : ny, m = blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= n) return;
   double re, im;
   if (m == 0) { re = 1.0; im = 0.0; }
@@ -103,8 +105,8 @@ int field_solve_enqueue(const Geom &g, const void *f, int f_bits, double *phi, d
   b.rho_tmp = g.n[3] > 64 ? scratch + L.rho_tmp : nullptr;
   b.diag = diag;  // nbiter 0: the five values at index 0
   b.nbiter = 0;
-  hipLaunchKernelGGL(k_twiddles, dim3((unsigned)((g.n[0] + 255) / 256)), dim3(256), 0, s, b.twx, g.n[0]);
-  hipLaunchKernelGGL(k_twiddles, dim3((unsigned)((g.n[1] + 255) / 256)), dim3(256), 0, s, b.twy, g.n[1]);
+  hipLaunchKernelGGL(k_twiddles, dim3((unsigned)((std::max(g.n[0], g.n[1]) + 255) / 256), 2), dim3(256), 0, s, b.twx,
+                     g.n[0], b.twy, g.n[1]);
   double *rho_part = scratch + L.rho_part, *l2_part = scratch + L.l2_part;
   if (f_bits == 64) launch_moments<double>(g, (const double *)f, rho_part, l2_part, s);
   else launch_moments<float>(g, (const float *)f, rho_part, l2_part, s);
