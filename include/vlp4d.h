@@ -135,9 +135,11 @@ int vlp_destroy(vlp_ctx *ctx);
 /* `nsteps` iterations of onetimestep (VMO/Timestep.hpp:34-97) followed by
  * fn.swap(fnp1) (VMO/Vlp4d.cpp:137-147).  Returns VLP_E_CFL if a foot left the
  * domain (state is then invalid; vlp_iter names the failing step).  With
- * nsteps > 1 (spline solver) step s + 1 is queued before step s's error flag
- * is read, so the GPU does not wait for the host between steps; results are
- * those of nsteps calls of one step. */
+ * nsteps > 1 step s + 1 is queued before the host waits for step s (spline
+ * solver: reads its error flag), so the GPU does not wait for the host between
+ * steps; results are those of nsteps calls of one step (Lagrange solver: to
+ * rounding, as the last x/2, y/2 of a step and the first of the next are one
+ * pass). */
 int vlp_step(vlp_ctx *ctx, int nsteps);
 
 /* Current iteration count (the reference's `iter`). */

@@ -383,9 +383,9 @@ void launch_field(const Geom &g, const FieldBufs &b, const double *rho_part, lon
   } else {
     const int sub1 = (g.idcase == 10 || g.idcase == 20);
     // along x a thread per eight planes and point of the density sum, 256 to
-    // 1024 (48 x 48 points of 48 planes: 5.3 us, with 1024 6.4); along y a
-    // thread per output of the inverse transforms, or two or more lanes per
-    // output of a direct sum
+    // 1024 (a solve of 48 x 48 x 32 x 48: 58 us with 1024 and a launch more for
+    // the twiddles, 54.7); along y a thread per output of the inverse
+    // transforms, or two or more lanes per output of a direct sum
     const int Ax = dft_factor(N0), Ay = dft_factor(N1);
     const int ty = Ay == 1 ? (N1 > 128 ? 512 : 256) : std::min(FIELD_NT, (3 * N1 + 63) / 64 * 64);
     const int XL = (N0 + 63) & ~63;
