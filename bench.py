@@ -272,9 +272,10 @@ def lagrange_cpu_baseline(n, steps=1):
 
 def lagrange_bench(pkg, n, steps, warmup, with_cpu):
     """The Lagrange split-step solver (miniapps/vlp4d) on the SLD10 deck at
-    n^4: six 1-D order-5 advections per step (x/2, y/2, vx, vy, x/2, y/2),
-    each streaming f once (16 B per cell in FP64), plus the field solve; the
-    x/2 + y/2 pairs run as one fused pass where the (x, y) plane fits in LDS."""
+    n^4: six 1-D order-5 advections per step (x/2, y/2, vx, vy, x/2, y/2) and
+    the field solve.  Every pass streams f once (16 B per cell in FP64): vx and
+    vy are one pass; where the (x, y) plane fits in LDS so are the x/2, y/2
+    pairs, the last of a step joined with the first of the next."""
     nb = warmup + steps
     cfg = pkg.VlpConfig.make(n, SLD10["minphy"], SLD10["maxphy"], SLD10["idcase"], SLD10["dt"], nb)
     sim = pkg.Vlp4d(cfg, scheme=pkg.SCHEME_LAGRANGE)
@@ -289,12 +290,12 @@ def lagrange_bench(pkg, n, steps, warmup, with_cpu):
     fused = bool(sim.kernel_variants() & 1)
     sim.close()
     ph = {lab: (ta[lab][0] - tb[lab][0]) / steps for lab in ("advec2D", "field", "advec4D")}
-    # the x/y phase holds 2 launches of the fused pass (kernel_variants bit 0)
-    # or 2 x (k_lag_x + k_lag_y); the velocity phase k_lag_v<2> + k_lag_v<3>.
+    # passes per step of the timed call: steps + 1 fused x/y passes
+    # (kernel_variants bit 0) or 2 x (k_lag_x + k_lag_y); one k_lag_vv.
     # The dominant family is the one with the larger share of the step.
-    xy = ("k_lag_xy", ph["advec2D"] / 2) if fused else ("k_lag_x/k_lag_y", ph["advec2D"] / 4)
-    kern, launch_s = max([xy + (ph["advec2D"],), ("k_lag_v", ph["advec4D"] / 2, ph["advec4D"])],
-                         key=lambda r: r[2])[:2]
+    n_xy = (steps + 1) / steps if fused else 4
+    kern, launch_s = max([("k_lag_plane" if fused else "k_lag_x/k_lag_y", ph["advec2D"] / n_xy, ph["advec2D"]),
+                          ("k_lag_vv", ph["advec4D"], ph["advec4D"])], key=lambda r: r[2])[:2]
     launch_bytes = 16 * n ** 4
     achieved = launch_bytes / launch_s / 1e9
     res = {
@@ -307,7 +308,7 @@ def lagrange_bench(pkg, n, steps, warmup, with_cpu):
         "roofline": {"bound": "hbm", "kernel": kern, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic(kern, 64, n, LAG_TRAFFIC_FILE),
                      "algorithmic_bytes_per_launch": launch_bytes, "avg_launch_ms": 1e3 * launch_s},
-        "step_hbm_fraction": (4 if fused else 6) * launch_bytes / (dt / steps) / 1e9 / HBM_PEAK_GBS,
+        "step_hbm_fraction": (n_xy + 1) * launch_bytes / (dt / steps) / 1e9 / HBM_PEAK_GBS,
         "phases_ms": {k: round(1e3 * v, 4) for k, v in ph.items()},
         "final_nrj": float(d["nrj"][-1]),
     }
