@@ -693,6 +693,11 @@ YsPlan ys_plan(const Geom &g, size_t tsz, int want_tvx = 0, int want_nb = 0) {
   // (vx tile 2, two buffers), whose barriers are independent, run best for
   // both slab types (double: 8.0 ms against 8.7 at tile 4; float storage 7.5
   // against 8.1; float arithmetic, three waves per SIMD, 5.2 against 6.2).
+  // Tiles of 2 in rows of 33 to 64 points make workgroups of two waves; tile 4,
+  // as the same three or four waves as tile 2 in longer rows, is taken first
+  // there: it stages 8 slab rows for 4 of vx instead of 12 (64 x 48 x 100 x 100
+  // 1.17 -> 0.78 ms in double, 0.70 -> 0.48 in float; 48^4 0.226 -> 0.200, 56^4
+  // 0.333 -> 0.311; 96^4 stays with tile 2, 2.6 ms against 3.0).
   // A tile is passed over when another has over 1/0.9 times as many lanes with
   // cells on a CU: lanes past N0 TVX (to whole waves) and past N2 (last tile)
   // do nothing, and the workgroups of a CU are bounded by LDS and waves (three
@@ -705,9 +710,11 @@ YsPlan ys_plan(const Geom &g, size_t tsz, int want_tvx = 0, int want_nb = 0) {
   // slab does not fit LDS.
   static const int pref_f[][2] = {{2, 2}, {4, 2}, {8, 2}, {4, 3}, {2, 3}, {8, 3}};
   static const int pref_d[][2] = {{2, 2}, {4, 2}, {8, 2}, {4, 3}, {8, 3}, {2, 3}};
+  static const int pref_4[][2] = {{4, 2}, {2, 2}, {8, 2}, {4, 3}, {8, 3}, {2, 3}};
+  const auto &pref = N0 > 32 && N0 <= 64 ? pref_4 : tsz == sizeof(float) ? pref_f : pref_d;
   double best = 0.;
   for (int pass = 0; pass < 2; pass++)
-    for (const auto &c : (tsz == sizeof(float) ? pref_f : pref_d)) {
+    for (const auto &c : pref) {
       const int tvx = c[0], nb = c[1];
       if (force && tvx != force) continue;
       if (force_nb && nb != force_nb) continue;
