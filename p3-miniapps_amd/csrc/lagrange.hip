@@ -424,21 +424,16 @@ static size_t lag_xy_lds(const Geom &g) { return ((size_t)(g.n[0] | 1) * g.n[1] 
 
 // 16 or 32 points per lane where that takes at most 8 waves (the plane's loads
 // run a pass ahead and the density is summed along), else 32 and up to 16
-// waves (longest planes: neither, registers); 0: the plane does not fit,
-// separate kernels.  VLP4D_LAG_FUSED=0 disables the fusion.
+// waves (longest planes: neither, registers); 0: the plane does not fit.
 static int lag_points(const Geom &g) {
-  if (const char *e = getenv("VLP4D_LAG_FUSED"))
-    if (atoi(e) == 0) return 0;
   if (lag_xy_lds(g) > 160 * 1024) return 0;
   return lag_waves(g, 16) <= 8 ? 16 : lag_waves(g, 32) <= 16 ? 32 : 0;
 }
 
-// vx runs per vy of the fused pass (0: separate kernels): the fewest rounds of
+// vx runs per vy for S points per lane: the fewest rounds of
 // workgroups over the CUs, counting one plane time for a run's start, with
 // runs of at least four planes (their density sums are stored per run).
-int lag_xy_chunks(const Geom &g) {
-  const int S = lag_points(g);
-  if (!S) return 0;
+static int lag_chunks(const Geom &g, int S) {
   int per_cu = (int)(160 * 1024 / lag_xy_lds(g));
   if (per_cu > 32 / lag_waves(g, S)) per_cu = 32 / lag_waves(g, S);
   if (per_cu > 8) per_cu = 8;
@@ -458,9 +453,15 @@ int lag_xy_chunks(const Geom &g) {
   return best;
 }
 
-bool lag_xy_sums(const Geom &g) {
-  const int S = lag_points(g);
-  return S && lag_waves(g, S) <= 8;
+LagPlan lag_xy_plan(const Geom &g) {
+  LagPlan p;
+  if (const char *e = getenv("VLP4D_LAG_FUSED"))
+    if (atoi(e) == 0) return p;
+  p.points = lag_points(g);
+  if (!p.points) return p;
+  p.chunks = lag_chunks(g, p.points);
+  p.sums = lag_waves(g, p.points) <= 8;
+  return p;
 }
 
 // Initial conditions of VO/init.cpp:144-285 (TSI20 differs from the spline
@@ -533,18 +534,17 @@ static void launch_plane_sums(const Geom &g, const double *in, double *out, cons
   else launch_plane<S, 512, false, false>(g, in, out, tab, nchunk, nullptr, s);
 }
 
-bool launch_lag_xy(const Geom &g, const double *in, double *out, const void *tab, int nchunk, bool twice,
+void launch_lag_xy(const Geom &g, const LagPlan &plan, const double *in, double *out, const void *tab, bool twice,
                    double *rho_part, hipStream_t s) {
-  if (nchunk <= 0 || !tab) return false;
-  if (!lag_xy_sums(g)) {
+  const int nchunk = plan.chunks;
+  if (!plan.sums) {
     if (twice) launch_plane<32, 1024, true, false>(g, in, out, tab, nchunk, nullptr, s);
     else launch_plane<32, 1024, false, false>(g, in, out, tab, nchunk, nullptr, s);
-  } else if (lag_points(g) == 16) {
+  } else if (plan.points == 16) {
     launch_plane_sums<16>(g, in, out, tab, nchunk, twice, rho_part, s);
   } else {
     launch_plane_sums<32>(g, in, out, tab, nchunk, twice, rho_part, s);
   }
-  return true;
 }
 
 void launch_lag_y(const Geom &g, const double *in, double *out, double dt, double *rho_part, hipStream_t s) {

@@ -36,6 +36,7 @@ struct vlp_ctx {
   int precision = VLP_FP64;
   int scheme = VLP_SCHEME_SPLINE;  // VLP_SCHEME_LAGRANGE: the split-step Lagrange solver (lagrange.hip)
   void *lag_tab = nullptr;          // stencil tables of its fused x/2, y/2 pass
+  vlp::LagPlan lag;                 // that pass, fixed at creation (rho_part is sized for it)
   int device = 0;
   hipStream_t stream = nullptr;
   size_t esz = 8;
@@ -356,13 +357,12 @@ int lag_steps(vlp_ctx *c, int nsteps) {
   const Geom &g = c->g;
   const double dt = c->cfg.dt;
   hipStream_t s = c->stream;
-  const int nch = vlp::lag_xy_chunks(g);
-  const bool fused = nch > 0, sums = fused && vlp::lag_xy_sums(g);
+  const bool fused = c->lag.points > 0, sums = c->lag.sums;
   // the x/2, y/2 pair from f into f, `twice` over; rho: with its density
   auto xy = [&](bool twice, bool rho) {
     double *f = (double *)c->f, *t = (double *)c->fnext;
     if (fused) {
-      vlp::launch_lag_xy(g, f, t, c->lag_tab, nch, twice, rho && sums ? c->rho_part : nullptr, s);
+      vlp::launch_lag_xy(g, c->lag, f, t, c->lag_tab, twice, rho && sums ? c->rho_part : nullptr, s);
       std::swap(c->f, c->fnext);
       if (rho && !sums) vlp::launch_moments<double>(g, t, c->rho_part, c->l2_part, s);
     } else {
@@ -371,7 +371,7 @@ int lag_steps(vlp_ctx *c, int nsteps) {
         vlp::launch_lag_y(g, t, f, 0.5 * dt, rho && k == (twice ? 1 : 0) ? c->rho_part : nullptr, s);
       }
     }
-    c->rho_outer = (long)(sums ? nch : 1) * g.n[3];
+    c->rho_outer = (long)(sums ? c->lag.chunks : 1) * g.n[3];
   };
   // ev[4], ev[5] of the first set: around the first pass
   hipEvent_t *sets[2] = {c->ev, c->evb};
@@ -677,6 +677,7 @@ static int create_ctx(const vlp_config *cfg_in, int precision, int device, int s
   c->n_c4s = lag ? 0 : vlp::c4_elems(N0, N1, N2, N3);
   c->n_l2 = vlp::l2_partials(c->g);
   c->xy_groups = lag ? 0 : vlp::xy_fused_groups(c->g, c->esz);
+  if (lag) c->lag = vlp::lag_xy_plan(c->g);
   c->rho_outer = N3;
   const size_t nxh = N0 / 2 + 1;
   auto fail = [&](int code) {
@@ -707,7 +708,7 @@ static int create_ctx(const vlp_config *cfg_in, int precision, int device, int s
     ALLOC(c->c4_alloc, (c->n_c4s + 16) * c->esz);
     c->c4 = (char *)c->c4_alloc + c4_shift(c->g) * c->esz;
   }
-  const int rho_runs = lag ? vlp::lag_xy_chunks(c->g) : c->xy_groups;
+  const int rho_runs = lag ? (c->lag.sums ? c->lag.chunks : 1) : c->xy_groups;
   ALLOC(c->rho_part, N0 * N1 * N3 * (size_t)std::max(rho_runs, 1) * sizeof(double));
   ALLOC(c->l2_part, (size_t)c->n_l2 * sizeof(double));
   ALLOC(c->fb.rho, N0 * N1 * sizeof(double));
@@ -1033,7 +1034,7 @@ const char *vlp_last_error(const vlp_ctx *c) { return c ? c->err.c_str() : g_las
 
 int vlp_kernel_variants(const vlp_ctx *c) {
   if (!c) return -1;
-  if (c->scheme == VLP_SCHEME_LAGRANGE) return vlp::lag_xy_chunks(c->g) > 0 ? 1 : 0;  // bit 0: fused x/y pass
+  if (c->scheme == VLP_SCHEME_LAGRANGE) return c->lag.points > 0 ? 1 : 0;  // bit 0: fused x/y pass
   int bits = vlp::kernel_variants(c->g, c->precision != VLP_FP64, c->precision == VLP_FP32_ACC);
   if ((bits & 128) && c->ys_tvx) bits = (bits & ~(15 << 8)) | (c->ys_tvx << 8);
   if (vlp::spline_tile_width(vx_map(c->g), c->esz, c->sp_mode[0]) == 128) bits |= 1 << 13;

@@ -162,19 +162,24 @@ void launch_lag_y(const Geom &g, const double *in, double *out, double dt, doubl
 // vx then vy in one pass, from in to out
 void launch_lag_vv(const Geom &g, const double *in, double *out, const double *ex, const double *ey, double dt,
                    hipStream_t s);
-// Fused x/2 + y/2 (one pass over f) when the (x, y) plane fits in LDS:
-// lag_xy_chunks gives the vx runs per vy, 0 when not eligible;
-// launch_lag_xy returns false for nchunk 0.  twice: the pair two times over
-// (the end of one step and the start of the next).  With lag_xy_sums(g), a
+// Fused x/2 + y/2 (one pass over f) when the (x, y) plane fits in LDS.
+struct LagPlan {
+  int points = 0;     // points per lane and pass; 0: separate kernels
+  int chunks = 0;     // vx runs per vy
+  bool sums = false;  // the pass can sum the density of its result
+};
+// The plan of a geometry; VLP4D_LAG_FUSED=0: separate kernels.  Read once per
+// context: the size of rho_part follows from it.
+LagPlan lag_xy_plan(const Geom &g);
+// The pass of a plan with points > 0.  twice: the pair two times over
+// (the end of one step and the start of the next).  With plan.sums, a
 // non-null rho_part (always for twice) receives the density of the result,
-// nchunk * N3 partial planes; without, the caller takes it from the result.
+// chunks * N3 partial planes; without, the caller takes it from the result.
 // The stencil tables of the x/2, y/2 passes (lag_tables_bytes) are built once
 // per context for the half step dt.
-int lag_xy_chunks(const Geom &g);
-bool lag_xy_sums(const Geom &g);
 size_t lag_tables_bytes(const Geom &g);
 void launch_lag_tables(const Geom &g, void *tab, double dt, hipStream_t s);
-bool launch_lag_xy(const Geom &g, const double *in, double *out, const void *tab, int nchunk, bool twice,
+void launch_lag_xy(const Geom &g, const LagPlan &plan, const double *in, double *out, const void *tab, bool twice,
                    double *rho_part, hipStream_t s);
 
 // Work buffers of the reproducible adjoint scatter: scl (4 doubles: the
