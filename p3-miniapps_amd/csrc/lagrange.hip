@@ -225,10 +225,12 @@ __global__ __launch_bounds__(1024) void k_lag_vv(const double *__restrict__ in, 
 // workgroup's vx planes (field_rho).  Workgroup per (vy, run of G vx planes).
 // A plane goes from registers (loaded during the previous plane's passes)
 // to LDS; each pass gives a wave 64 lines across the lanes and S consecutive
-// points along them.  The displacement is that of the line's velocity, the same
+// points along them (FLAT: the lanes take the lines' segments one after another,
+// so that no lane idles where a plane has few lines).  The displacement is that
+// of the line's velocity, the same
 // for all its points, so a lane has one set of weights and slides a six-value
 // window along its points: (S + 5) / S LDS reads per point, at addresses
-// uniform in the wave up to the lane's line.  A pass in place reads, waits for
+// uniform in the wave up to the lane's line (and, FLAT, its segment).  A pass in place reads, waits for
 // the workgroup and writes; the last y pass goes from LDS to HBM, and its
 // points are the same in every plane, so their density sums stay in
 // registers.  The LDS row pitch is odd, so neither direction has bank conflicts.
@@ -255,15 +257,23 @@ __global__ __launch_bounds__(256) void k_lag_tables(LagTab *__restrict__ tab, Ge
   tab[i].b = j[0];
 }
 
+// A copy of v that the compiler takes for a new value: uniform in the wave, or
+// (VEC) one per lane.
+template <bool VEC> __device__ __forceinline__ void opaque(int &v) {
+  if constexpr (VEC) asm volatile("" : "+v"(v));
+  else asm volatile("" : "+s"(v));
+}
+
 // Results of the line at `line` (LDS, stride st between its N points) at the S
 // points from p0 on (periodic), each handed to out(i, value).  Everything but
-// `line` is uniform in the wave.  (The empty asm keeps the positions from being
-// hoisted out of the loop over planes, where they would be spilled.)
-template <int S, typename F>
+// `line` and (FLAT) p0 is uniform in the wave.  (The opaque copy keeps the
+// positions from being hoisted out of the loop over planes, where they would be
+// spilled.)
+template <int S, bool FLAT, typename F>
 __device__ __forceinline__ void lag_slide(const double *line, int st, int N, int p0, const LagTab &t, F out) {
   int q = t.b + p0;
   q = q >= N ? q - N : q;
-  asm volatile("" : "+s"(q));
+  opaque<FLAT>(q);
   const double *p = line + q * st;
   const int wrap = st - N * st;
   double w[6];
@@ -289,7 +299,7 @@ __device__ __forceinline__ void lag_slide(const double *line, int st, int N, int
   }
 }
 
-template <int S, int NT, bool TWICE, bool RHO>
+template <int S, int NT, bool TWICE, bool RHO, bool FLAT>
 __global__ __launch_bounds__(NT) void k_lag_plane(const double *__restrict__ in, double *__restrict__ out, Geom g,
                                                     const LagTab *__restrict__ tab, int G, int nchunk,
                                                     double *__restrict__ rho_part) {
@@ -303,12 +313,14 @@ __global__ __launch_bounds__(NT) void k_lag_plane(const double *__restrict__ in,
   const LagTab &ty = tab[N2 + ivy];
   // x pass: rows 64 rg + lane, points xs .. xs + xn - 1
   const int nsx = (N0 + S - 1) / S, nsy = (N1 + S - 1) / S;
-  const int xrow = 64 * (wave / nsx) + lane, xs = S * (wave % nsx), xn = min(S, N0 - xs);
-  const bool xact = xrow < N1;
+  const int xrow = FLAT ? l % N1 : 64 * (wave / nsx) + lane, xs = S * (FLAT ? l / N1 : wave % nsx);
+  const int xn = min(S, N0 - xs);
+  const bool xact = FLAT ? xn > 0 : xrow < N1;
   double *const xl = pl + (xact ? xrow : 0) * pitch;
   // y pass: columns 64 cg + lane, points ys .. ys + yn - 1
-  const int ycol = 64 * (wave / nsy) + lane, ys = S * (wave % nsy), yn = min(S, N1 - ys);
-  const bool yact = ycol < N0;
+  const int ycol = FLAT ? l % N0 : 64 * (wave / nsy) + lane, ys = S * (FLAT ? l / N0 : wave % nsy);
+  const int yn = min(S, N1 - ys);
+  const bool yact = FLAT ? yn > 0 : ycol < N0;
   double *const yl = pl + (yact ? ycol : 0);
   // this lane's plane points l, l + nl, ..., at most S of them
   const int dcol = nl % N0, drow = nl / N0, col0 = l % N0, row0 = l / N0;
@@ -359,22 +371,23 @@ __global__ __launch_bounds__(NT) void k_lag_plane(const double *__restrict__ in,
       if (ivx + 1 < v1) load(in + off + P);  // in flight during the passes
 #pragma unroll
     for (int half = 0; half < (TWICE ? 2 : 1); half++) {
-      if (xact) lag_slide<S>(xl, 1, N0, xs, tx, keep);
+      if (xact) lag_slide<S, FLAT>(xl, 1, N0, xs, tx, keep);
       __syncthreads();
       if (xact) {
         int n = xn;
-        asm volatile("" : "+s"(n));
+        opaque<FLAT>(n);
 #pragma unroll
         for (int i = 0; i < S; i++)
           if (i < n) xl[xs + i] = o[i];
       }
       __syncthreads();
       if (TWICE && half == 0) {
-          if (yact) lag_slide<S>(yl, pitch, N1, ys, ty, keep);
+        if (yact) lag_slide<S, FLAT>(yl, pitch, N1, ys, ty, keep);
         __syncthreads();
         if (yact) {
           int n = yn, row = pitch;
-          asm volatile("" : "+s"(n), "+s"(row));
+          opaque<FLAT>(n);
+          opaque<false>(row);
 #pragma unroll
           for (int i = 0; i < S; i++)
             if (i < n) yl[(ys + i) * row] = o[i];
@@ -383,20 +396,21 @@ __global__ __launch_bounds__(NT) void k_lag_plane(const double *__restrict__ in,
       }
     }
     if (yact) {
-      // a scalar row address and the lane's column
-      char *dst = (char *)(out + off + (size_t)ys * N0);
-      unsigned at = 8u * (unsigned)ycol;
-      int n = yn, row = 8 * N0;
-      asm volatile("" : "+v"(at), "+s"(n), "+s"(row));
-      if (n == S) {  // (no branch between the points)
-        lag_slide<S>(yl, pitch, N1, ys, ty, [&](int i, double v) {
-          *(double *)(dst + at) = v;
+      // a scalar row address and the lane's offset: its column and (FLAT) first row
+      char *dst = (char *)(out + off + (FLAT ? 0 : (size_t)ys * N0));
+      int at = 8 * (ycol + (FLAT ? ys * N0 : 0)), n = yn, row = 8 * N0;
+      opaque<true>(at);
+      opaque<FLAT>(n);
+      opaque<false>(row);
+      if (!FLAT && n == S) {  // (no branch between the points)
+        lag_slide<S, FLAT>(yl, pitch, N1, ys, ty, [&](int i, double v) {
+          *(double *)(dst + (unsigned)at) = v;
           dst += row;
           if constexpr (RHO) rho[i] += v;
         });
       } else {
-        lag_slide<S>(yl, pitch, N1, ys, ty, [&](int i, double v) {
-          if (i < n) *(double *)(dst + at) = v;
+        lag_slide<S, FLAT>(yl, pitch, N1, ys, ty, [&](int i, double v) {
+          if (i < n) *(double *)(dst + (unsigned)at) = v;
           dst += row;
           if constexpr (RHO) rho[i] += v;
         });
@@ -413,36 +427,38 @@ __global__ __launch_bounds__(NT) void k_lag_plane(const double *__restrict__ in,
 }
 
 // Waves of a workgroup for S points per lane and pass: every pass has a wave
-// for each of its 64-line groups and S-point segments.
-static int lag_waves(const Geom &g, int S) {
-  const int N0 = g.n[0], N1 = g.n[1];
-  const int x = (N1 + 63) / 64 * ((N0 + S - 1) / S), y = (N0 + 63) / 64 * ((N1 + S - 1) / S);
+// for each of its 64-line groups and S-point segments, or (flat) a lane for
+// each line and segment.
+static int lag_waves(const Geom &g, int S, bool flat) {
+  const int N0 = g.n[0], N1 = g.n[1], nsx = (N0 + S - 1) / S, nsy = (N1 + S - 1) / S;
+  const int x = flat ? (N1 * nsx + 63) / 64 : (N1 + 63) / 64 * nsx;
+  const int y = flat ? (N0 * nsy + 63) / 64 : (N0 + 63) / 64 * nsy;
   return x > y ? x : y;
 }
 
 static size_t lag_xy_lds(const Geom &g) { return ((size_t)(g.n[0] | 1) * g.n[1] + 1) * sizeof(double); }
 
-// 16 or 32 points per lane where that takes at most 8 waves (the plane's loads
-// run a pass ahead and the density is summed along), else 32 and up to 16
-// waves (longest planes: neither, registers); 0: the plane does not fit.
-static int lag_points(const Geom &g) {
-  if (lag_xy_lds(g) > 160 * 1024) return 0;
-  return lag_waves(g, 16) <= 8 ? 16 : lag_waves(g, 32) <= 16 ? 32 : 0;
-}
-
-// vx runs per vy for S points per lane: the fewest rounds of
+// vx runs per vy for workgroups of `waves`: the fewest rounds of
 // workgroups over the CUs, counting one plane time for a run's start, with
-// runs of at least four planes (their density sums are stored per run).
-static int lag_chunks(const Geom &g, int S) {
+// runs of at least four planes (their density sums are stored per run) unless
+// there are at most three workgroups per CU, whose planes one after another are
+// latency: one step a call of 10^4 85 -> 70 us, 24^4 89 -> 80, 100 x 91 x 12 x 12
+// 134 -> 102; 16 x 16 x 64 x 64 with runs of two 103 us, with four 100.  (Counting
+// 32 waves per CU, not those whose registers fit, 72 x 60 x 60 x 60 took one
+// workgroup per CU more than there is room for: four steps a call 250 -> 197 us
+// per step.)
+static int lag_chunks(const Geom &g, int waves, int points) {
   int per_cu = (int)(160 * 1024 / lag_xy_lds(g));
-  if (per_cu > 32 / lag_waves(g, S)) per_cu = 32 / lag_waves(g, S);
+  // the waves whose registers fit a CU
+  const int fit = points == 16 ? 12 : waves <= 8 ? 8 : 16;
+  if (per_cu > fit / waves) per_cu = fit / waves;
   if (per_cu > 8) per_cu = 8;
   const long cap = 256L * (per_cu < 1 ? 1 : per_cu);
   int best = 1;
   long cost = -1;
   for (int n = 1; n <= g.n[2]; n++) {
     const int G = (g.n[2] + n - 1) / n;
-    if (n > 1 && G < 4) break;
+    if (n > 1 && G < 4 && (long)g.n[3] * n > 3 * 256) break;
     if ((g.n[2] + G - 1) / G != n) continue;  // the same runs in fewer workgroups
     const long c = ((long)g.n[3] * n + cap - 1) / cap * (G + 1);
     if (cost < 0 || c < cost) {
@@ -453,14 +469,37 @@ static int lag_chunks(const Geom &g, int S) {
   return best;
 }
 
+// 16 points per lane where that takes at most 8 waves, or 32 (the plane's loads
+// run a pass ahead and the density is summed along), else 32 and up to 16 waves
+// (longest planes: neither, registers).  The 16-point form goes flat where only
+// that fits 8 waves (against 32 points in 64-line groups, one step a call: 68 x
+// 68 x 24 x 24 144 -> 116 us, 10 x 251 x 60 x 60 405 -> 218, 160 x 10 x 60 x 60
+// 329 -> 153) or takes half the waves (100 x 10 x 60 x 60 183 -> 127; 31 x 64 x 40 x
+// 40, 3 instead of 4, 84 -> 87).
+// With 32 points a lane's density sums do not fit the registers (54 spills, one
+// workgroup per CU): a pass of one pair takes 16 points, up to 16 waves and no
+// sums as long as the density pass finds f in the 256 MB last-level cache: one
+// step a call of 90 x 90 x 24 x 24 162 -> 145 us, 100 x 91 x 60 x 60 (262 MB) 628
+// -> 585; but 90 x 128 x 60 x 60 (332 MB) 597 -> 613.
 LagPlan lag_xy_plan(const Geom &g) {
   LagPlan p;
   if (const char *e = getenv("VLP4D_LAG_FUSED"))
     if (atoi(e) == 0) return p;
-  p.points = lag_points(g);
-  if (!p.points) return p;
-  p.chunks = lag_chunks(g, p.points);
-  p.sums = lag_waves(g, p.points) <= 8;
+  if (lag_xy_lds(g) > 160 * 1024) return p;
+  const struct { int points; bool flat; int waves; } forms[] = {{16, false, 8}, {16, true, 8}, {32, false, 16}};
+  for (const auto &f : forms) {
+    const int w = lag_waves(g, f.points, f.flat);
+    if (w > f.waves || (f.points == 16 && !f.flat && 2 * lag_waves(g, 16, true) <= w)) continue;
+    p.points = f.points;
+    p.flat = f.flat;
+    p.waves = w;
+    p.chunks = lag_chunks(g, w, f.points);
+    p.sums = w <= 8;
+    break;
+  }
+  const int w16 = lag_waves(g, 16, false);
+  const double mib = 8. * g.n[0] * g.n[1] * g.n[2] * g.n[3] / (1 << 20);
+  if (p.points == 32 && p.sums && w16 <= 16 && mib <= 256.) p.waves1 = w16;
   return p;
 }
 
@@ -515,35 +554,39 @@ void launch_lag_tables(const Geom &g, void *tab, double dt, hipStream_t s) {
   hipLaunchKernelGGL(k_lag_tables, dim3(blocks(g.n[2] + g.n[3])), dim3(256), 0, s, (LagTab *)tab, g, dt);
 }
 
-template <int S, int NT, bool TWICE, bool RHO>
-static void launch_plane(const Geom &g, const double *in, double *out, const void *tab, int nchunk, double *rho_part,
-                         hipStream_t s) {
-  const int G = (g.n[2] + nchunk - 1) / nchunk;
-  const void *fn = (const void *)k_lag_plane<S, NT, TWICE, RHO>;
+template <int S, int NT, bool TWICE, bool RHO, bool FLAT = false>
+static void launch_plane(const Geom &g, const LagPlan &p, const double *in, double *out, const void *tab,
+                         double *rho_part, hipStream_t s) {
+  const int G = (g.n[2] + p.chunks - 1) / p.chunks;
+  const void *fn = (const void *)k_lag_plane<S, NT, TWICE, RHO, FLAT>;
   if (lag_xy_lds(g) > 64 * 1024)
     (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lag_xy_lds(g));
-  hipLaunchKernelGGL((k_lag_plane<S, NT, TWICE, RHO>), dim3((unsigned)(g.n[3] * nchunk)), dim3(64 * lag_waves(g, S)),
-                     lag_xy_lds(g), s, in, out, g, (const LagTab *)tab, G, nchunk, rho_part);
+  hipLaunchKernelGGL((k_lag_plane<S, NT, TWICE, RHO, FLAT>), dim3((unsigned)(g.n[3] * p.chunks)), dim3(64 * p.waves),
+                     lag_xy_lds(g), s, in, out, g, (const LagTab *)tab, G, p.chunks, rho_part);
 }
 
-template <int S>
-static void launch_plane_sums(const Geom &g, const double *in, double *out, const void *tab, int nchunk, bool twice,
-                              double *rho_part, hipStream_t s) {
-  if (twice) launch_plane<S, 512, true, true>(g, in, out, tab, nchunk, rho_part, s);
-  else if (rho_part) launch_plane<S, 512, false, true>(g, in, out, tab, nchunk, rho_part, s);
-  else launch_plane<S, 512, false, false>(g, in, out, tab, nchunk, nullptr, s);
+template <int S, bool FLAT>
+static void launch_plane_sums(const Geom &g, const LagPlan &p, const double *in, double *out, const void *tab,
+                              bool twice, double *rho_part, hipStream_t s) {
+  if (twice) launch_plane<S, 512, true, true, FLAT>(g, p, in, out, tab, rho_part, s);
+  else if (rho_part) launch_plane<S, 512, false, true, FLAT>(g, p, in, out, tab, rho_part, s);
+  else launch_plane<S, 512, false, false, FLAT>(g, p, in, out, tab, nullptr, s);
 }
 
-void launch_lag_xy(const Geom &g, const LagPlan &plan, const double *in, double *out, const void *tab, bool twice,
+void launch_lag_xy(const Geom &g, const LagPlan &p, const double *in, double *out, const void *tab, bool twice,
                    double *rho_part, hipStream_t s) {
-  const int nchunk = plan.chunks;
-  if (!plan.sums) {
-    if (twice) launch_plane<32, 1024, true, false>(g, in, out, tab, nchunk, nullptr, s);
-    else launch_plane<32, 1024, false, false>(g, in, out, tab, nchunk, nullptr, s);
-  } else if (plan.points == 16) {
-    launch_plane_sums<16>(g, in, out, tab, nchunk, twice, rho_part, s);
+  if (!twice && p.waves1) {
+    LagPlan q = p;
+    q.waves = p.waves1;
+    launch_plane<16, 1024, false, false>(g, q, in, out, tab, nullptr, s);
+  } else if (!p.sums) {
+    if (twice) launch_plane<32, 1024, true, false>(g, p, in, out, tab, nullptr, s);
+    else launch_plane<32, 1024, false, false>(g, p, in, out, tab, nullptr, s);
+  } else if (p.points == 16) {
+    if (p.flat) launch_plane_sums<16, true>(g, p, in, out, tab, twice, rho_part, s);
+    else launch_plane_sums<16, false>(g, p, in, out, tab, twice, rho_part, s);
   } else {
-    launch_plane_sums<32>(g, in, out, tab, nchunk, twice, rho_part, s);
+    launch_plane_sums<32, false>(g, p, in, out, tab, twice, rho_part, s);
   }
 }
 

@@ -357,10 +357,11 @@ int lag_steps(vlp_ctx *c, int nsteps) {
   const Geom &g = c->g;
   const double dt = c->cfg.dt;
   hipStream_t s = c->stream;
-  const bool fused = c->lag.points > 0, sums = c->lag.sums;
+  const bool fused = c->lag.points > 0;
   // the x/2, y/2 pair from f into f, `twice` over; rho: with its density
   auto xy = [&](bool twice, bool rho) {
     double *f = (double *)c->f, *t = (double *)c->fnext;
+    const bool sums = c->lag.sums && (twice || !c->lag.waves1);
     if (fused) {
       vlp::launch_lag_xy(g, c->lag, f, t, c->lag_tab, twice, rho && sums ? c->rho_part : nullptr, s);
       std::swap(c->f, c->fnext);

@@ -165,14 +165,18 @@ void launch_lag_vv(const Geom &g, const double *in, double *out, const double *e
 // Fused x/2 + y/2 (one pass over f) when the (x, y) plane fits in LDS.
 struct LagPlan {
   int points = 0;     // points per lane and pass; 0: separate kernels
+  bool flat = false;  // lanes along the lines' segments
+  int waves = 0;      // of a workgroup
   int chunks = 0;     // vx runs per vy
   bool sums = false;  // the pass can sum the density of its result
+  int waves1 = 0;     // a pass of one pair: 16 points and no sums, these waves (0: as above)
 };
 // The plan of a geometry; VLP4D_LAG_FUSED=0: separate kernels.  Read once per
 // context: the size of rho_part follows from it.
 LagPlan lag_xy_plan(const Geom &g);
 // The pass of a plan with points > 0.  twice: the pair two times over
-// (the end of one step and the start of the next).  With plan.sums, a
+// (the end of one step and the start of the next).  With plan.sums and (not
+// twice) no plan.waves1, a
 // non-null rho_part (always for twice) receives the density of the result,
 // chunks * N3 partial planes; without, the caller takes it from the result.
 // The stencil tables of the x/2, y/2 passes (lag_tables_bytes) are built once
