@@ -529,12 +529,33 @@ int spline_only(vlp_ctx *c) {
 // holds nothing between calls, in whole 16-byte chunks of floats.
 size_t stage_values(const vlp_ctx *c) { return c->n_tv * c->esz / sizeof(double) / 4 * 4; }
 
+// Whether a transfer of n floats is converted on the host.  On the device the
+// host side of the copy is the doubles, twice the bytes, and each piece is a
+// launch; the host's conversion takes about 1.3 ns a value.  From and to pinned
+// memory the device wins from 2^18 values on (get_f of 20^4 62 us there, 52 on
+// the host; 24^4 86 and 134), pageable memory, whose copies are slower, from 2^21
+// (to the device; 36^4 458 and 440 us, 40^4 642 and 751) or 3 2^20 values (40^4
+// 1.16 and 1.06 ms, 48^4 2.36 and 2.79).
+bool convert_on_host(const void *host, size_t n, size_t pageable_limit) {
+  if (n < (1u << 18)) return true;
+  if (n >= pageable_limit) return false;
+  hipPointerAttribute_t a;
+  const bool pinned = hipPointerGetAttributes(&a, host) == hipSuccess && a.type == hipMemoryTypeHost;
+  (void)hipGetLastError();  // (memory that HIP does not know may be an error there)
+  return !pinned;
+}
+
 // Host doubles into f.  For float storage the doubles go to the device as they
 // are and are converted there, in pieces staged in TV (converting on the host
-// took 0.3 s for 128^4, the copy of the doubles takes 40 ms).
+// took 0.3 s for 128^4, the copy of the doubles takes 40 ms); few are converted
+// on the host.
 int upload_f(vlp_ctx *c, const double *host) {
+  std::vector<float> tmp;
   if (c->esz == sizeof(double)) {
     HIP_TRY(c, hipMemcpyAsync(c->f, host, c->n_f * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  } else if (convert_on_host(host, c->n_f, 1u << 21)) {
+    tmp.assign(host, host + c->n_f);  // (each rounded to float)
+    HIP_TRY(c, hipMemcpyAsync(c->f, tmp.data(), c->n_f * sizeof(float), hipMemcpyHostToDevice, c->stream));
   } else {
     const size_t m = stage_values(c);
     for (size_t k = 0; k < c->n_f; k += m) {
@@ -554,6 +575,12 @@ int upload_f(vlp_ctx *c, const double *host) {
 int download(vlp_ctx *c, const void *dev, size_t n, double *host) {
   if (c->esz == sizeof(double)) {
     HIP_TRY(c, hipMemcpyAsync(host, dev, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  } else if (convert_on_host(host, n, 3u << 20)) {
+    std::vector<float> tmp(n);
+    HIP_TRY(c, hipMemcpyAsync(tmp.data(), dev, n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    std::copy(tmp.begin(), tmp.end(), host);
+    return VLP_OK;
   } else {
     const size_t m = stage_values(c);
     for (size_t k = 0; k < n; k += m) {
