@@ -458,6 +458,21 @@ __global__ __launch_bounds__(256) void k_narrow(const double *__restrict__ in, f
     for (long k = i; k < n; k++) out[k] = (float)in[k];
   }
 }
+template <typename S, typename D>
+__global__ __launch_bounds__(256) void k_strip(const S *__restrict__ in, long P, long w, D *__restrict__ out) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x, k = blockIdx.y;
+  if (i < w) out[k * w + i] = (D)in[k * P + i];
+}
+// (at most 251 x 251 planes: within a grid's y extent)
+template <typename S, typename D>
+void launch_strip(const S *in, size_t P, size_t w, size_t np, D *out, hipStream_t s) {
+  hipLaunchKernelGGL((k_strip<S, D>), dim3((unsigned)((w + 255) / 256), (unsigned)np), dim3(256), 0, s, in, (long)P,
+                     (long)w, out);
+}
+template void launch_strip<double, double>(const double *, size_t, size_t, size_t, double *, hipStream_t);
+template void launch_strip<float, float>(const float *, size_t, size_t, size_t, float *, hipStream_t);
+template void launch_strip<float, double>(const float *, size_t, size_t, size_t, double *, hipStream_t);
+
 void launch_widen(const float *in, double *out, long n, hipStream_t s) {
   hipLaunchKernelGGL(k_widen, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, s, in, out, n);
 }

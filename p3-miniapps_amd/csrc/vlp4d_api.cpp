@@ -536,6 +536,7 @@ size_t stage_values(const vlp_ctx *c) { return c->n_tv * c->esz / sizeof(double)
 // the host; 24^4 86 and 134), pageable memory, whose copies are slower, from 2^21
 // (to the device; 36^4 458 and 440 us, 40^4 642 and 751) or 3 2^20 values (40^4
 // 1.16 and 1.06 ms, 48^4 2.36 and 2.79).
+constexpr size_t kSetPageable = 1u << 21, kGetPageable = 3u << 20;
 bool convert_on_host(const void *host, size_t n, size_t pageable_limit) {
   if (n < (1u << 18)) return true;
   if (n >= pageable_limit) return false;
@@ -553,7 +554,7 @@ int upload_f(vlp_ctx *c, const double *host) {
   std::vector<float> tmp;
   if (c->esz == sizeof(double)) {
     HIP_TRY(c, hipMemcpyAsync(c->f, host, c->n_f * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  } else if (convert_on_host(host, c->n_f, 1u << 21)) {
+  } else if (convert_on_host(host, c->n_f, kSetPageable)) {
     tmp.assign(host, host + c->n_f);  // (each rounded to float)
     HIP_TRY(c, hipMemcpyAsync(c->f, tmp.data(), c->n_f * sizeof(float), hipMemcpyHostToDevice, c->stream));
   } else {
@@ -575,7 +576,7 @@ int upload_f(vlp_ctx *c, const double *host) {
 int download(vlp_ctx *c, const void *dev, size_t n, double *host) {
   if (c->esz == sizeof(double)) {
     HIP_TRY(c, hipMemcpyAsync(host, dev, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  } else if (convert_on_host(host, n, 3u << 20)) {
+  } else if (convert_on_host(host, n, kGetPageable)) {
     std::vector<float> tmp(n);
     HIP_TRY(c, hipMemcpyAsync(tmp.data(), dev, n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
@@ -971,11 +972,27 @@ int vlp_get_buffer(vlp_ctx *c, int which, double *host, size_t n) {
   switch (which) {
     case VLP_BUF_F: return download(c, c->f, n, host);
     case VLP_BUF_CXY: {
-      std::vector<double> full(c->n_cxys);
-      rc = download(c, c->cxy, c->n_cxys, full.data());
-      if (rc) return rc;
+      // the planes without their padding, gathered in TV (128^4 FP64 2.3 GB: a host
+      // copy of the padded planes took another such allocation and 3 times as
+      // long, 96 x 96 x 60 x 60 85 ms against 28)
       const size_t P = (size_t)vlp::xy_plane(c->cfg.nxmax[0], c->cfg.nxmax[1]), np = c->n_cxys / P, w = n / np;
-      for (size_t k = 0; k < np; k++) memcpy(host + k * w, full.data() + k * P, w * sizeof(double));
+      if (P == w) return download(c, c->cxy, n, host);
+      if (c->esz == sizeof(double)) {
+        vlp::launch_strip((const double *)c->cxy, P, w, np, (double *)c->tv, c->stream);
+        return download(c, c->tv, n, host);
+      }
+      if (convert_on_host(host, n, kGetPageable)) {
+        vlp::launch_strip((const float *)c->cxy, P, w, np, (float *)c->tv, c->stream);
+        return download(c, c->tv, n, host);
+      }
+      const size_t m = stage_values(c) / w;  // planes per piece
+      for (size_t k = 0; k < np; k += m) {
+        const size_t q = std::min(m, np - k);
+        vlp::launch_strip((const float *)c->cxy + k * P, P, w, q, (double *)c->tv, c->stream);
+        HIP_TRY(c, hipMemcpyAsync(host + k * w, c->tv, q * w * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+      }
+      HIP_TRY(c, hipGetLastError());
+      HIP_TRY(c, hipStreamSynchronize(c->stream));
       return VLP_OK;
     }
     case VLP_BUF_C4: {

@@ -138,6 +138,10 @@ void launch_moments(const Geom &g, const T *f, double *rho_part, double *l2_part
 // float <-> double copies of n device values (both pointers 16-byte aligned).
 void launch_widen(const float *in, double *out, long n, hipStream_t s);
 void launch_narrow(const double *in, float *out, long n, hipStream_t s);
+// np planes of w values, P apart, one after another: double to double, float to
+// float or double.
+template <typename S, typename D>
+void launch_strip(const S *in, size_t P, size_t w, size_t np, D *out, hipStream_t s);
 
 // Number of l2 partial sums written by launch_advect4d / launch_moments.
 long l2_partials(const Geom &g);
