@@ -353,7 +353,8 @@ bool launch_advect4d<float>(const Geom &g, const float *c4, const double *ex, co
 
 // moments of a given f: rho partials (sum over vx) and L2 partials.  A
 // thread takes VX consecutive points of one (x, y) plane and vy and walks vx; for VX > 1 with
-// one 16-byte load per vx and four independent sums.  A block covers 256
+// one load of all of them per vx (a caller's f need only be aligned to its
+// elements, as multi-dword loads need no more) and four independent sums.  A block covers 256
 // points (x, y, vy), so there are l2_partials(g) blocks as for the other
 // producers.
 template <typename T, int VX>
@@ -389,7 +390,7 @@ __global__ __launch_bounds__(256) void k_moments(const T *__restrict__ f, Geom g
       for (; ivx + 4 <= N2; ivx += 4) {
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-          typedef T vec_t __attribute__((ext_vector_type(VX)));
+          typedef T vec_t __attribute__((ext_vector_type(VX), aligned(sizeof(T))));
           const vec_t w = *(const vec_t *)(src + plane * (ivx + u));
 #pragma unroll
           for (int j = 0; j < VX; j++) {
@@ -419,7 +420,7 @@ __global__ __launch_bounds__(256) void k_moments(const T *__restrict__ f, Geom g
 
 template <typename T> void launch_moments(const Geom &g, const T *f, double *rho_part, double *l2_part, hipStream_t s) {
   // float: four consecutive points per thread (one 16-byte load per vx) where
-  // the planes hold whole 16-byte chunks (measured at 128^4: 0.22 ms against 0.32
+  // the planes hold whole groups of four (measured at 128^4: 0.22 ms against 0.32
   // for one x per thread); double: one x and one running sum per thread
   // (0.39 ms against 0.42 for two x per thread and 0.41 for four sums)
   // (the points of a plane are contiguous across rows, so the plane's size
