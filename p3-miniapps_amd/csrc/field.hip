@@ -21,9 +21,13 @@ namespace vlp {
 // transform, half as many real terms, stays a direct sum: 8.6 us against 9.5.)
 //
 // Bound: LDS reads and latency of the few workgroups (one per row or column).
-// The direct sums read 6 N^2 complex values per column: the transforms of a
-// 128 x 128 solve along x and y took 7.4 and 17.9 us, now 14.3 (with the sum of
-// 512 density planes, 11 us in a launch of its own before) and 11.4 us.
+// The direct sums read 6 N^2 complex values per column: the transform of 128
+// points along y took 17.9 us, now 8.6; of 128 along x 7.4, now 5.2 and 14.3 with
+// the sum of 512 density planes (11 us in a launch of its own before).  The data
+// of a sum are broadcasts or runs from LDS; the twiddles, one per lane at strides
+// that meet in the banks, stay in global memory (copied to LDS too: 128 points
+// along y 10.5 us, 251 45.3 against 33.8, where direct sums without a second
+// lane per output took 36.7).
 // ---------------------------------------------------------------------------
 constexpr int FIELD_NT = 1024;
 
@@ -97,13 +101,12 @@ __device__ __forceinline__ void dft(const double *x, double *y, const double *tw
 // by the threads of a part), then the r2c transform of row iy.
 __global__ __launch_bounds__(FIELD_NT) void k_rho_rfftx(const double *__restrict__ rho_part, long rho_outer, Geom g,
                                                         FieldBufs b, int sub1, int A) {
-  extern __shared__ double sh[];  // twiddles, row, stage 1 ([N0][2] each); part sums [parts][XL]
+  extern __shared__ double sh[];  // row, stage 1 ([N0][2] each); part sums [parts][XL]
   const int N0 = g.n[0], N1 = g.n[1], nt = blockDim.x, tid = threadIdx.x;
   const int iy = blockIdx.x;
   const int nxh = N0 / 2 + 1;
-  double *tw = sh, *row = sh + 2 * N0, *y = row + 2 * N0, *ps = y + 2 * N0;
+  double *row = sh, *y = row + 2 * N0, *ps = y + 2 * N0;
   const int XL = (N0 + 63) & ~63, parts = nt / XL, x = tid % XL, part = tid / XL;
-  for (int i = tid; i < 2 * N0; i += nt) tw[i] = b.twx[i];
   if (x < N0 && part < parts) {
     const double *src = rho_part + x + (long)N0 * iy;
     const long plane = (long)N0 * N1;
@@ -122,7 +125,7 @@ __global__ __launch_bounds__(FIELD_NT) void k_rho_rfftx(const double *__restrict
     row[2 * tid + 1] = 0.;
   }
   __syncthreads();
-  dft(row, y, tw, 1, N0, A, nxh, 1., [&](int, int k, double re, double im) {
+  dft(row, y, b.twx, 1, N0, A, nxh, 1., [&](int, int k, double re, double im) {
     *(double2 *)(b.spec1 + 2 * (k + (long)nxh * iy)) = make_double2(re, im);
   });
 }
@@ -132,14 +135,11 @@ __global__ __launch_bounds__(FIELD_NT) void k_poisson_y(Geom g, FieldBufs b, int
   const int N0 = g.n[0], N1 = g.n[1], nt = blockDim.x, tid = threadIdx.x;
   const int nxh = N0 / 2 + 1, nyh = N1 / 2 + 1;
   const int kcol = blockIdx.x;
-  double *tw = sh;               // N1 complex
-  double *hat = sh + 2 * N1;     // 3 * N1 complex: phi, ex, ey
-  double *y = sh + 8 * N1;       // 3 * N1 complex: stage 1
+  const double *tw = b.twy;
+  double *hat = sh;              // 3 * N1 complex: phi, ex, ey
+  double *y = sh + 6 * N1;       // 3 * N1 complex: stage 1
   double *col = hat + 4 * N1;    // N1 complex, in ey's place until stage 2 of the forward transform
-  for (int i = tid; i < 2 * N1; i += nt) {
-    col[i] = b.spec1[2 * (kcol + (long)nxh * (i >> 1)) + (i & 1)];
-    tw[i] = b.twy[i];
-  }
+  for (int i = tid; i < 2 * N1; i += nt) col[i] = b.spec1[2 * (kcol + (long)nxh * (i >> 1)) + (i & 1)];
   __syncthreads();
   if (A == 1) {  // stage 2 reads the column itself: move it out of the result's way
     for (int i = tid; i < 2 * N1; i += nt) y[i] = col[i];
@@ -390,9 +390,9 @@ void launch_field(const Geom &g, const FieldBufs &b, const double *rho_part, lon
     const int ty = Ay == 1 ? (N1 > 128 ? 512 : 256) : std::min(FIELD_NT, (3 * N1 + 63) / 64 * 64);
     const int XL = (N0 + 63) & ~63;
     const int tx = std::min((long)FIELD_NT, std::max(256l, XL * ((rho_outer + 7) / 8)));
-    hipLaunchKernelGGL(k_rho_rfftx, dim3(N1), dim3(tx), sizeof(double) * (6 * N0 + tx / XL * XL), s,
+    hipLaunchKernelGGL(k_rho_rfftx, dim3(N1), dim3(tx), sizeof(double) * (4 * N0 + tx / XL * XL), s,
                        rho_part, rho_outer, g, b, sub1, Ax);
-    hipLaunchKernelGGL(k_poisson_y, dim3(nxh), dim3(ty), sizeof(double) * 14 * N1, s, g, b, Ay);
+    hipLaunchKernelGGL(k_poisson_y, dim3(nxh), dim3(ty), sizeof(double) * 12 * N1, s, g, b, Ay);
     hipLaunchKernelGGL(k_c2rx_diag, dim3(N1), dim3(256), sizeof(double) * (6 * nxh + 8), s, g, b);
   }
   if (record_diag)
