@@ -700,9 +700,13 @@ YsPlan ys_plan(const Geom &g, size_t tsz, int want_tvx = 0, int want_nb = 0) {
   // 0.333 -> 0.311; 96^4 stays with tile 2, 2.6 ms against 3.0).
   // A tile is passed over when another has over 1/0.9 times as many lanes with
   // cells on a CU: lanes past N0 TVX (to whole waves) and past N2 (last tile)
-  // do nothing, and the workgroups of a CU are bounded by LDS and waves (three
-  // per SIMD for float storage, else two).  (By the share of such lanes alone,
-  // 80 x 96 x 96 x 80 in float took tile 4: 1.76 ms, tile 2 takes 1.09.)
+  // do nothing, and the workgroups of a CU are bounded by LDS and waves, counted
+  // as three per SIMD for float storage, else two.  (By the share of such lanes
+  // alone, 80 x 96 x 96 x 80 in float took tile 4: 1.76 ms, tile 2 takes 1.09.)
+  // Float storage with double arithmetic has the registers for two waves only,
+  // but counted so it fares no better: over 90 ragged grids, rows of 17 to 24
+  // points would take tile 2 instead of 8, 4 % slower (31 of 35 slower, by up to 8
+  // %), the others even (tile 8 to 4 0.99, 4 to 2 0.99 of the time, 0.77 to 1.32).
   // Any extents are taken; the vx-blocked kernel, which ragged grids used to
   // run, is bound by L1 latency: 90 x 77 x 84 x 75 4.23 -> 1.51 ms (double) and
   // 2.95 -> 0.78 (float), 61 x 50 x 45 x 58 0.78 -> 0.33, 20 x 21 x 22 x 23
@@ -764,8 +768,8 @@ void launch_ys_t(const Geom &g, const YsPlan &p, const T *c4, const double *exy,
   const int nslab = g.n[3] + (iv0 >= 0);
   // y segments, when the workgroups would not fill the chip: the fewest
   // rounds of workgroups times steps (three beyond the cells, two steps' time
-  // for the set-up).  Workgroups per CU by LDS and by waves per SIMD (two
-  // with double arithmetic, three with float).  Advection of 16^4 FP64 58 ->
+  // for the set-up).  Workgroups per CU by LDS and by the waves per SIMD that
+  // registers allow (two with double arithmetic, three with float).  Advection of 16^4 FP64 58 ->
   // 23 us, 32^4 float 97 -> 43, 48^4 FP64 355 -> 195; from four rounds on one
   // segment is taken.
   int ylen = g.n[1];
@@ -838,10 +842,9 @@ bool ystream_preferred(const Geom &g, size_t tsz, int tvx, int nb) {
   return p.tvx == tvx && p.nb == nb;
 }
 
-int ystream_tvx(const Geom &g, bool fp32_storage, bool arith32) {
+int ystream_tvx(const Geom &g, bool fp32_storage) {
   if (const char *e = getenv("VLP4D_YSTREAM"))
     if (atoi(e) == 0) return 0;
-  (void)arith32;
   return ys_plan(g, fp32_storage ? sizeof(float) : sizeof(double)).tvx;
 }
 

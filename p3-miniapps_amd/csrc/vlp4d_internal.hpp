@@ -131,7 +131,7 @@ bool ystream_eligible(const Geom &g, size_t tsz, int tvx, int nb);
 // autotuner's incumbent).
 bool ystream_preferred(const Geom &g, size_t tsz, int tvx, int nb);
 // vx tile of the y-streaming kernel for a geometry (0: not used).
-int ystream_tvx(const Geom &g, bool fp32_storage, bool arith32);
+int ystream_tvx(const Geom &g, bool fp32_storage);
 template <typename T>
 void launch_moments(const Geom &g, const T *f, double *rho_part, double *l2_part, hipStream_t s);
 
