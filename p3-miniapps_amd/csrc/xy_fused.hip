@@ -19,6 +19,7 @@
 // field solve.
 #include "spline_scan.hpp"
 
+#include <algorithm>
 #include <cstdlib>
 
 namespace vlp {
@@ -365,18 +366,56 @@ XyPlan xy_plan(const Geom &g, size_t tsz) {
   return p;
 }
 
+// Advection points per lane of nt.
+int xy_points(const Geom &g, int nt) {
+  const int nseg = nt / g.n[0];
+  return nseg ? (g.n[1] + nseg - 1) / nseg : XY_NPT + 1;
+}
+
+// Lanes of a workgroup.  XY_NT with up to 8 points each, else twice as many (or
+// XY_NT with up to 32 points: launch_xy_t); rag planes whose lines take fewer
+// lanes go in workgroups of those, so that more of them share a CU: most lanes
+// of 512 idled through the recursions, and the phases of 25 x 23 x 100 x 100 in
+// float took 157 us, 94 in the separate kernels, now 57 (30 x 30 x 130 x 130 328,
+// 155 and 111; 40 x 40 x 77 x 77 110, 86 and 63).
+int xy_lanes(const Geom &g, const XyPlan &p) {
+  if (p.rag)
+    for (int nt : {128, 256})
+      if (xy_points(g, nt) <= 8 && std::max(g.n[1] * p.Px, (g.n[0] + 4) * p.Py) <= nt) return nt;
+  return xy_points(g, XY_NT) <= 8 ? XY_NT : 2 * XY_NT;
+}
+
 }  // namespace
 
+// Groups of vx planes per vy: the least time of a CU that runs its k workgroups
+// of VG planes (and a plane's time for the start) up to per_cu at once, each
+// plane costing latency once per round and throughput once per workgroup, in
+// equal shares where 512 lanes or more go through a plane and two to one where
+// fewer do.  (Powers of two until the chip was full twice left 130 x 4 = 520
+// workgroups for 512 places, a whole round for the last eight: with 512 lanes, 25
+// x 23 x 130 x 130 in double 344 us, now 238, 90 x 77 x 66 x 66 312 and 222; 96^4
+// 534 and 429.  64 x 64 x 96 x 96 took 236, now 245.  By rounds alone 64 x 64 x
+// 128 x 128 in float was 9 % slower.)
 int xy_fused_groups(const Geom &g, size_t tsz) {
   if (const char *e = getenv("VLP4D_XY_FUSED"))
     if (atoi(e) == 0) return 0;
-  if (!xy_plan(g, tsz).C) return 0;
-  // about two rounds of workgroups over the 256 CUs (one or two per CU)
-  const int per_cu = xy_lds(g, tsz) > 80 * 1024 ? 1 : 2;
-  int G = 1;
-  // (the last group may be shorter)
-  while (G * 2 <= g.n[2] && (long)G * g.n[3] < 256L * per_cu) G *= 2;
-  return G;
+  const XyPlan p = xy_plan(g, tsz);
+  if (!p.C) return 0;
+  const int N2 = g.n[2], nt = xy_lanes(g, p);
+  const long per_cu = std::max(1L, std::min((long)(2 * XY_NT / nt), (long)(160 * 1024 / xy_lds(g, tsz))));
+  int best = 1;
+  long cost = -1;
+  for (int n = 1; n <= N2; n++) {
+    const int VG = (N2 + n - 1) / n;
+    if ((N2 + VG - 1) / VG != n) continue;  // the same groups in fewer workgroups
+    const long k = ((long)n * g.n[3] + 255) / 256;
+    const long c = (VG + 1) * (2 * ((k + per_cu - 1) / per_cu) + (nt >= XY_NT ? 2 : 1) * k);
+    if (cost < 0 || c < cost) {
+      cost = c;
+      best = n;
+    }
+  }
+  return best;
 }
 
 template <typename T, typename A, int C, bool RAG, int NT, int NPT>
@@ -397,8 +436,12 @@ static void launch_xy_n(const Geom &g, const T *f, T *cxy, double dth, int G, do
 template <typename T, typename A, int C, bool RAG>
 static void launch_xy_t(const Geom &g, const T *f, T *cxy, double dth, int G, double *rho_part, int *err,
                         const XyPlan &p, hipStream_t s) {
-  const int nseg = XY_NT / g.n[0], ylen = (g.n[1] + nseg - 1) / nseg;
-  if (ylen <= 8) launch_xy_n<T, A, C, RAG, XY_NT, 8>(g, f, cxy, dth, G, rho_part, err, p, s);
+  if constexpr (RAG) {
+    const int nt = xy_lanes(g, p);
+    if (nt == 128) return launch_xy_n<T, A, C, RAG, 128, 8>(g, f, cxy, dth, G, rho_part, err, p, s);
+    if (nt == 256) return launch_xy_n<T, A, C, RAG, 256, 8>(g, f, cxy, dth, G, rho_part, err, p, s);
+  }
+  if (xy_points(g, XY_NT) <= 8) launch_xy_n<T, A, C, RAG, XY_NT, 8>(g, f, cxy, dth, G, rho_part, err, p, s);
   else if constexpr (RAG && C == 16) launch_xy_n<T, A, C, RAG, XY_NT, XY_NPT>(g, f, cxy, dth, G, rho_part, err, p, s);
   else launch_xy_n<T, A, C, RAG, 2 * XY_NT, XY_NPT / 2>(g, f, cxy, dth, G, rho_part, err, p, s);
 }
