@@ -483,11 +483,15 @@ static int tile_chunk(const LineMap &m, size_t tsz, int &P, int &XT, bool &rag, 
   x_split(m.N, P, logP, C);
   rag = !C || P * 64 > 512;
   if (rag) {
-    // float lines of 68, 72 and 76 points keep the line kernel, whose four
-    // lanes fit them (72^4: 0.110 ms for both passes against 0.121)
+    // float lines that four lanes of the line kernel divide evenly (68 to 124
+    // points) keep it while the pass writes less than 100 MB, which the
+    // last-level cache serves: 24 x 24 x 100 x 100 33 us for both passes against
+    // 45, 44 x 44 x 84 x 84 (72 MB) 58 and 70; but 61 x 50 x 100 x 100 (152 MB) 156
+    // and 137, 90 x 90 x 72 x 72 (204 MB) 198 and 175
     int logQ, D;
-    line_split(m.N, 20, P, logQ, D);
-    if (tsz == sizeof(float) && P == 4 && D > 16) return 0;
+    line_split(m.N, 32, P, logQ, D);
+    const double mb = 1e-6 * tsz * m.X0 * m.X1 * m.A * (m.N + 4);
+    if (tsz == sizeof(float) && P == 4 && D > 16 && mb < 100.) return 0;
     rag_split(m.N, 8, P, C);
   }
   if (!C) return 0;
