@@ -42,6 +42,7 @@ VALU_PEAK_FP32_TFS = 157.3  # FP32 vector peak, reached only with packed FP32 (d
 ADVECT4D_FLOP_PER_CELL = 860
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "advect4d_traffic_sld10_128.txt")
 LAG_TRAFFIC_FILE = os.path.join(ROOT, "profiles", "lagrange_traffic_sld10_128.txt")
+LAG_XY_KERNEL, LAG_V_KERNEL = "k_lag_plane", "k_lag_vv"  # the Lagrange solver's passes, as the traffic file names them
 A100_REF = 2.38e9  # 40*128^4 / 4.51995 s, A100 stdpar MainLoop (docs/vlp4d.md:148,168-171)
 SLD10 = dict(minphy=[0.0, 0.0, -9.0, -9.0], maxphy=[12.56637112, 12.56637112, 9.0, 9.0], idcase=10, dt=0.01)
 
@@ -294,8 +295,8 @@ def lagrange_bench(pkg, n, steps, warmup, with_cpu):
     # (kernel_variants bit 0) or 2 x (k_lag_x + k_lag_y); one k_lag_vv.
     # The dominant family is the one with the larger share of the step.
     n_xy = (steps + 1) / steps if fused else 4
-    kern, launch_s = max([("k_lag_plane" if fused else "k_lag_x/k_lag_y", ph["advec2D"] / n_xy, ph["advec2D"]),
-                          ("k_lag_vv", ph["advec4D"], ph["advec4D"])], key=lambda r: r[2])[:2]
+    kern, launch_s = max([(LAG_XY_KERNEL if fused else "k_lag_x/k_lag_y", ph["advec2D"] / n_xy, ph["advec2D"]),
+                          (LAG_V_KERNEL, ph["advec4D"], ph["advec4D"])], key=lambda r: r[2])[:2]
     launch_bytes = 16 * n ** 4
     achieved = launch_bytes / launch_s / 1e9
     res = {

@@ -236,9 +236,10 @@ __global__ __launch_bounds__(1024) void k_lag_vv(const double *__restrict__ in, 
 // registers.  The LDS row pitch is odd, so neither direction has bank conflicts.
 //
 // Bound: HBM (16 bytes per cell; 0.91 ms per pass at 128^4 at the 4.7 TB/s of a
-// large copy), with one 132 KB plane per CU there: a TWICE pass takes 1.21 ms,
-// and its LDS work (about 0.35 ms) and barriers are not all hidden behind the
-// loads.  128^4 step in a run of steps 4.14 -> 2.97 ms: before, the pair read
+// large copy), with one 132 KB plane per CU there: a TWICE pass takes 1.17 ms.
+// With RHO it moves 5.33 GB, not 4.29, since 60 registers of the density sums of
+// 32 points go through scratch memory; its LDS work (about 0.35 ms) and barriers
+// are not all hidden behind the loads.  128^4 step in a run of steps 4.14 -> 2.97 ms: before, the pair read
 // six stencil values per point and pass from LDS (1.01 ms), the density was a
 // pass of its own (0.41 ms) and neighbouring steps each had their pair.
 struct LagTab {  // stencil of a line: six weights and the wrapped first index of point 0
